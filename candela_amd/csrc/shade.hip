@@ -300,7 +300,9 @@ __device__ __forceinline__ void backward_pixel(const SceneArgs& s, const crt_sha
                                                const float* __restrict__ color, const float* __restrict__ target,
                                                float* __restrict__ g_albedo, float* __restrict__ g_rough,
                                                float* inten_sum, int32_t* my) {
-    crt_shade_record R;
+    // every field is initialized: with some left undefined for the lanes past
+    // the end, the compiler may assume that there are none and drop the bound
+    crt_shade_record R{};
     R.tri0 = -1;
     R.tri1 = -1;
     if (i < npix) R = rec[i];
