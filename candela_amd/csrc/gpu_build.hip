@@ -11,27 +11,32 @@
 // Steps, all on one stream, none allocating (the caller passes a workspace):
 //   1. per triangle its box centroid ((min + max) * 0.5, as ConstructTree
 //      caches it, BVHConstructor.cpp:404-427); bounds of the centroids by a
-//      two-level min/max reduction;
-//   2. a 30-bit Morton code of the centroid quantized to 1024 cells per axis;
-//   3. a stable LSD radix sort of (code, triangle) by 4-bit digits, 8 passes:
-//      each pass counts the digits per 1024-code tile, scans the digit-major
-//      counts (a workgroup per digit) and scatters each tile's codes in input
-//      order within their digit;
-//   4. Karras's radix tree: internal node i finds its range and split by
-//      binary searches over the longest common prefix of neighbouring codes
-//      (ties broken by the sorted index, so every code is distinct);
-//   5. boxes: a node's box is the min / max over the triangles of its leaf
-//      range.  Nodes inside one workgroup's 1024 leaves are united bottom up
-//      in LDS; the workgroup also writes its leaves' prefix and suffix boxes
-//      and lists the nodes whose range spans workgroups.  A wave then forms
-//      each listed node's box from one suffix, one prefix and the whole
-//      chunks between them (no chain of dependent steps up the tree);
-//   6. the stack layout: entry i holds internal node i's two children; a
-//      child that covers two leaves is written as one 2-triangle leaf (the
-//      reference's leaf size), so its own entry is never reached.
-// The triangle array is the input triangles in sorted order.
+//      grid-stride min/max reduction;
+//   2. a 30-bit Morton code of the centroid quantized to 1024 cells per axis
+//      (each workgroup folds the partial bounds itself), and the first digit's
+//      count per tile;
+//   3. a stable LSD radix sort of (code, triangle) by 8-bit digits, 4 passes of
+//      two launches: count the digits per tile, then scatter each tile's codes
+//      in digit order (a tile finds its place from the counts before it);
+//   4. the tree (Karras's radix tree; ties broken by the sorted index, so every
+//      code is distinct), the boxes and the stack layout in one pass over
+//      chunks of 512 leaves: a node whose leaf range lies in one chunk, all but
+//      about one in 60, is found by binary searches in LDS, takes its
+//      children's boxes from the chunk's power-of-two box windows and is
+//      written at once;
+//   5. the remaining nodes, whose range crosses chunks: 16 lanes each find the
+//      range and the split 16 codes at a time and forms the boxes from leaf
+//      boxes at both ends and the boxes of 64 and 4,096 leaves between them.
+//   Entry i holds internal node i's two children; a child covering two
+//   triangles is written as a 2-triangle leaf.
+//
+// Measured on 2.56M triangles (2,000 spheres): 308 us, of them bounds and codes
+// 40, sort 110, tree with boxes and entries 104 + 5 + 45; with 4-bit digits,
+// three launches a pass and separate tree, box and entry passes it was 743 us.
+// 11,520 triangles: 82 us instead of 145, nearly all launches and latency.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -44,7 +49,6 @@ namespace crt {
 namespace gb {
 
 using scan::kBlock;
-using scan::kScanBlock;
 
 constexpr int kMortonBits = 30;
 
@@ -70,63 +74,64 @@ __device__ __forceinline__ void centroid(const Box& b, float c[3]) {
     for (int k = 0; k < 3; ++k) c[k] = (b.lo[k] + b.hi[k]) * 0.5f;
 }
 
-// Per-workgroup min / max of the centroids: partial[6 * block + (0..2 lo, 3..5 hi)].
-__global__ void __launch_bounds__(kBlock) centroid_bounds(const crt_vertex* __restrict__ v,
-                                                          const uint32_t* __restrict__ idx, int64_t n,
-                                                          float* __restrict__ partial) {
-    __shared__ float sh[6][kBlock];
-    const int64_t t = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    float c[3] = {0.0f, 0.0f, 0.0f};
-    const bool ok = t < n;
-    if (ok) centroid(tri_box(v, idx, t), c);
-    for (int k = 0; k < 3; ++k) {
-        sh[k][threadIdx.x] = ok ? c[k] : __builtin_inff();
-        sh[3 + k][threadIdx.x] = ok ? c[k] : -__builtin_inff();
-    }
-    __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s)
-            for (int k = 0; k < 3; ++k) {
-                sh[k][threadIdx.x] = fminf(sh[k][threadIdx.x], sh[k][threadIdx.x + s]);
-                sh[3 + k][threadIdx.x] = fmaxf(sh[3 + k][threadIdx.x], sh[3 + k][threadIdx.x + s]);
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) partial[6 * int64_t(blockIdx.x) + threadIdx.x] = sh[threadIdx.x][0];
+// Per-workgroup min / max of the centroids over a grid-stride loop:
+// partial[k * gridDim.x + block], k = 0..2 lo, 3..5 hi.  Also clears what later
+// launches add to, the super-tile counts of every sort pass (kernel stores, no
+// memset node, so the chain stays capturable).
+constexpr int kBoundsGrid = 1024;   // at most this many workgroups (and partials)
+
+__device__ __forceinline__ float wave_min(float v) {
+    for (int d = 32; d > 0; d >>= 1) v = fminf(v, __shfl_xor(v, d, 64));
+    return v;
 }
 
-// One workgroup folds the partials into (lo[3], scale[3]): scale = 1 / extent, 0 for a flat axis.
-constexpr int kBoundsBlock = 1024;   // the one workgroup that reduces the partial bounds
+__device__ __forceinline__ float wave_max(float v) {
+    for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
+    return v;
+}
 
-__global__ void __launch_bounds__(kBoundsBlock) finish_bounds(const float* __restrict__ partial, int64_t nb,
-                                                              float* __restrict__ frame) {
-    __shared__ float sh[6][kBoundsBlock];
-    float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-    float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-#pragma unroll 4
-    for (int64_t b = threadIdx.x; b < nb; b += kBoundsBlock)
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = fminf(lo[k], partial[6 * b + k]);
-            hi[k] = fmaxf(hi[k], partial[6 * b + 3 + k]);
-        }
+// Min (lo) and max (hi) over the workgroup's threads; every thread gets them.
+__device__ __forceinline__ void block_bounds(float lo[3], float hi[3], float (&sh)[6][kBlock / 64]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int k = 0; k < 3; ++k) {
-        sh[k][threadIdx.x] = lo[k];
-        sh[3 + k][threadIdx.x] = hi[k];
+        lo[k] = wave_min(lo[k]);
+        hi[k] = wave_max(hi[k]);
+        if (lane == 0) {
+            sh[k][wave] = lo[k];
+            sh[3 + k][wave] = hi[k];
+        }
     }
     __syncthreads();
-    for (int s = kBoundsBlock / 2; s > 0; s >>= 1) {
-        if (int(threadIdx.x) < s)
-            for (int k = 0; k < 3; ++k) {
-                sh[k][threadIdx.x] = fminf(sh[k][threadIdx.x], sh[k][threadIdx.x + s]);
-                sh[3 + k][threadIdx.x] = fmaxf(sh[3 + k][threadIdx.x], sh[3 + k][threadIdx.x + s]);
-            }
-        __syncthreads();
+    for (int k = 0; k < 3; ++k)
+        for (int w = 0; w < kBlock / 64; ++w) {
+            lo[k] = fminf(lo[k], sh[k][w]);
+            hi[k] = fmaxf(hi[k], sh[3 + k][w]);
+        }
+}
+
+__global__ void __launch_bounds__(kBlock) centroid_bounds(const crt_vertex* __restrict__ v,
+                                                          const uint32_t* __restrict__ idx, int64_t n,
+                                                          float* __restrict__ partial, uint32_t* __restrict__ supers,
+                                                          int64_t super_words) {
+    __shared__ float sh[6][kBlock / 64];
+    const int64_t stride = int64_t(gridDim.x) * kBlock, first = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    for (int64_t w = first; w < super_words; w += stride) supers[w] = 0u;
+    float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
+    float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+#pragma unroll 2
+    for (int64_t t = first; t < n; t += stride) {
+        float c[3];
+        centroid(tri_box(v, idx, t), c);
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = fminf(lo[k], c[k]);
+            hi[k] = fmaxf(hi[k], c[k]);
+        }
     }
+    block_bounds(lo, hi, sh);
     if (threadIdx.x < 3) {
-        const float l = sh[threadIdx.x][0], h = sh[3 + threadIdx.x][0];
-        const float ext = h - l;
-        frame[threadIdx.x] = l;
-        frame[3 + threadIdx.x] = ext > 0.0f ? 1.0f / ext : 0.0f;
+        const int k = int(threadIdx.x);
+        partial[k * int64_t(gridDim.x) + blockIdx.x] = k == 0 ? lo[0] : k == 1 ? lo[1] : lo[2];
+        partial[(3 + k) * int64_t(gridDim.x) + blockIdx.x] = k == 0 ? hi[0] : k == 1 ? hi[1] : hi[2];
     }
 }
 
@@ -144,205 +149,232 @@ __device__ __forceinline__ uint32_t quantize(float c, float lo, float scale) {
     return uint32_t(fminf(fmaxf(x, 0.0f), 1023.0f));
 }
 
-__global__ void __launch_bounds__(kBlock) morton(const crt_vertex* __restrict__ v, const uint32_t* __restrict__ idx,
-                                                 int64_t n, const float* __restrict__ frame,
-                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const int64_t t = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (t >= n) return;
-    float c[3];
-    centroid(tri_box(v, idx, t), c);
-    const uint32_t x = quantize(c[0], frame[0], frame[3]);
-    const uint32_t y = quantize(c[1], frame[1], frame[4]);
-    const uint32_t z = quantize(c[2], frame[2], frame[5]);
-    keys[t] = (spread3(x) << 2) | (spread3(y) << 1) | spread3(z);
-    vals[t] = uint32_t(t);
-}
-
-// Radix sort of the codes by 4-bit digits (LSD, stable), tiles of kTile
-// codes: a workgroup of kBlock threads takes kItems codes each, round r
-// holding codes tile * kTile + r * kBlock + thread, so rounds and threads run
-// in index order.  tile_ranks gives each code its rank among the codes of its
-// digit that precede it in the tile (peers in the wave from one ballot per
-// digit bit; earlier waves and rounds from LDS counts) and leaves the tile's
-// per-digit counts in run[].  Codes past n take digit 15: they rank after
-// every code of the tile, and only the last tile has them, whose digit-15
-// segment ends the order.
-constexpr int kDigitBits = 4;
+// Radix sort of the codes by 8-bit digits (LSD, stable; the codes' 30 bits take
+// 4 passes).  A tile is kTile codes of one workgroup, kItems per thread.  Pass
+// p counts each tile's digits (counts[tile * kRadix + digit], and the sums over
+// super-tiles of 2^super_log tiles), then scatters: the place of a tile's first
+// code of digit d is the number of codes of smaller digits plus the number of
+// d's in the tiles before it, which the tile adds up itself from the super-tile
+// sums and the counts of its own super-tile (about 70 loads a thread, all
+// independent).  That replaces the launch that scanned the counts; a decoupled
+// look-back would replace the count as well, but every tile is resident at
+// once here, so its chain over 1,250 tiles would cross the XCDs' caches link
+// by link.
+//
+// Bound: launches and latency at a few thousand triangles, memory (16 bytes
+// read, 8 written per code and pass) at millions.  2.56M codes: 110 us (20 a
+// scatter, 7.5 a count); 8 passes of 4-bit digits with three launches each took
+// 252 us.
+constexpr int kDigitBits = 8;
 constexpr int kRadix = 1 << kDigitBits;
-constexpr int kItems = 4;
+constexpr int kItems = 8;
 constexpr int kTile = kBlock * kItems;
 constexpr int kWaves = kBlock / 64;
+constexpr int kPasses = (kMortonBits + kDigitBits - 1) / kDigitBits;
+static_assert(kRadix == kBlock, "a thread per digit");
 
-__device__ __forceinline__ void tile_ranks(const uint32_t* __restrict__ keys, int64_t n, int shift, uint32_t key[kItems],
-                                           uint32_t digit[kItems], uint32_t rank[kItems], uint32_t* wc,
-                                           uint32_t* run) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t below = (1ull << lane) - 1ull;
-    if (threadIdx.x < kRadix) run[threadIdx.x] = 0u;
+// Writes a tile's digit counts (hist in LDS) and adds them to its super-tile's.
+__device__ __forceinline__ void put_counts(const uint32_t* hist, int super_log, uint32_t* __restrict__ counts,
+                                           uint32_t* __restrict__ supers) {
+    const uint32_t c = hist[threadIdx.x];
+    counts[int64_t(blockIdx.x) * kRadix + threadIdx.x] = c;
+    if (c) atomicAdd(supers + int64_t(blockIdx.x >> super_log) * kRadix + threadIdx.x, c);
+}
+
+// Morton codes of one tile, and its digit counts for the first pass.
+__global__ void __launch_bounds__(kBlock) morton(const crt_vertex* __restrict__ v, const uint32_t* __restrict__ idx,
+                                                 int64_t n, const float* __restrict__ partial, int32_t nparts,
+                                                 uint32_t* __restrict__ keys, int super_log,
+                                                 uint32_t* __restrict__ counts, uint32_t* __restrict__ supers) {
+    __shared__ float sh[6][kBlock / 64];
+    __shared__ uint32_t hist[kRadix];
+    float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
+    float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+    hist[threadIdx.x] = 0u;
+    for (int32_t b = int32_t(threadIdx.x); b < nparts; b += kBlock)
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = fminf(lo[k], partial[k * nparts + b]);
+            hi[k] = fmaxf(hi[k], partial[(3 + k) * nparts + b]);
+        }
+    block_bounds(lo, hi, sh);   // ends after a barrier, so hist is clear as well
+    float scale[3];
+    for (int k = 0; k < 3; ++k) {
+        const float ext = hi[k] - lo[k];
+        scale[k] = ext > 0.0f ? 1.0f / ext : 0.0f;   // 0 for a flat axis
+    }
+#pragma unroll 4
     for (int r = 0; r < kItems; ++r) {
-        const int64_t i = int64_t(blockIdx.x) * kTile + r * kBlock + threadIdx.x;
-        key[r] = i < n ? keys[i] : 0u;
-        const uint32_t d = i < n ? (key[r] >> shift) & (kRadix - 1) : kRadix - 1;
-        digit[r] = d;
-        uint64_t peers = ~0ull;
-        for (int b = 0; b < kDigitBits; ++b) {
-            const uint64_t bb = __ballot((d >> b) & 1u);
-            peers &= ((d >> b) & 1u) ? bb : ~bb;
-        }
-        if (threadIdx.x < kWaves * kRadix) wc[threadIdx.x] = 0u;
-        __syncthreads();
-        if ((peers & below) == 0ull) wc[wave * kRadix + d] = uint32_t(__popcll(peers));   // the digit's first lane
-        __syncthreads();
-        uint32_t before = run[d];
-        for (int w = 0; w < kWaves; ++w) before += w < wave ? wc[w * kRadix + d] : 0u;
-        rank[r] = before + uint32_t(__popcll(peers & below));
-        __syncthreads();
-        if (threadIdx.x < kRadix) {
-            uint32_t sum = 0u;
-            for (int w = 0; w < kWaves; ++w) sum += wc[w * kRadix + threadIdx.x];
-            run[threadIdx.x] += sum;
-        }
-        __syncthreads();
+        const int64_t t = int64_t(blockIdx.x) * kTile + r * kBlock + threadIdx.x;
+        if (t >= n) break;
+        float c[3];
+        centroid(tri_box(v, idx, t), c);
+        const uint32_t x = quantize(c[0], lo[0], scale[0]);
+        const uint32_t y = quantize(c[1], lo[1], scale[1]);
+        const uint32_t z = quantize(c[2], lo[2], scale[2]);
+        const uint32_t key = (spread3(x) << 2) | (spread3(y) << 1) | spread3(z);
+        keys[t] = key;
+        atomicAdd(&hist[key & (kRadix - 1)], 1u);
     }
+    __syncthreads();
+    put_counts(hist, super_log, counts, supers);
 }
 
-// counts[digit * ntiles + tile]: digit-major, so one exclusive scan gives
-// each (digit, tile) its first position in the stable order.
 __global__ void __launch_bounds__(kBlock) count_digits(const uint32_t* __restrict__ keys, int64_t n, int shift,
-                                                       uint32_t* __restrict__ counts) {
-    __shared__ uint32_t wc[kWaves * kRadix];
-    __shared__ uint32_t run[kRadix];
-    uint32_t key[kItems], digit[kItems], rank[kItems];
-    tile_ranks(keys, n, shift, key, digit, rank, wc, run);
-    if (threadIdx.x < kRadix) counts[int64_t(threadIdx.x) * gridDim.x + blockIdx.x] = run[threadIdx.x];
+                                                       int super_log, uint32_t* __restrict__ counts,
+                                                       uint32_t* __restrict__ supers) {
+    __shared__ uint32_t hist[kRadix];
+    hist[threadIdx.x] = 0u;
+    __syncthreads();
+    uint32_t key[kItems];
+    const int64_t base = int64_t(blockIdx.x) * kTile + threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) key[r] = base + r * kBlock < n ? keys[base + r * kBlock] : 0u;
+#pragma unroll
+    for (int r = 0; r < kItems; ++r)
+        if (base + r * kBlock < n) atomicAdd(&hist[(key[r] >> shift) & (kRadix - 1)], 1u);
+    __syncthreads();
+    put_counts(hist, super_log, counts, supers);
 }
 
-// Exclusive scan of the digit-major tile counts (counts[d * nt + tile]) by
-// kRadix workgroups, one per digit: workgroup d sums the counts of the digits
-// below it (a contiguous prefix of the array) for its base, then scans its
-// own nt counts in coalesced passes.  One workgroup scanning all kRadix * nt
-// counts ran on one CU and took a third of the build.
-constexpr int kDigitScanBlock = 1024;
-
-__global__ void __launch_bounds__(kDigitScanBlock) scan_digits(const uint32_t* __restrict__ counts, int64_t nt,
-                                                               int64_t* __restrict__ offsets) {
-    __shared__ int64_t wave_sums[kDigitScanBlock / 64];
+// Exclusive prefixes of a and b over the workgroup's threads.
+__device__ __forceinline__ void block_prefix2(uint32_t& a, uint32_t& b, uint32_t (&sh)[2][kWaves]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t seg = int64_t(blockIdx.x) * nt;
-    // base: the sum of counts [0, seg)
-    int64_t p0 = 0, p1 = 0, p2 = 0, p3 = 0;   // four loads in flight per thread
-    for (int64_t k = threadIdx.x; k < seg; k += 4 * kDigitScanBlock) {
-        p0 += counts[k];
-        p1 += k + kDigitScanBlock < seg ? counts[k + kDigitScanBlock] : 0u;
-        p2 += k + 2 * kDigitScanBlock < seg ? counts[k + 2 * kDigitScanBlock] : 0u;
-        p3 += k + 3 * kDigitScanBlock < seg ? counts[k + 3 * kDigitScanBlock] : 0u;
-    }
-    int64_t part = (p0 + p1) + (p2 + p3);
-    for (int d = 32; d > 0; d >>= 1) part += __shfl_xor(part, d, 64);
-    if (lane == 0) wave_sums[wave] = part;
-    __syncthreads();
-    int64_t carry = 0;
-    for (int w = 0; w < kDigitScanBlock / 64; ++w) carry += wave_sums[w];
-    __syncthreads();
-    for (int64_t b = 0; b < nt; b += kDigitScanBlock) {
-        const int64_t k = b + threadIdx.x;
-        const int64_t v = k < nt ? int64_t(counts[seg + k]) : 0;
-        int64_t incl = v;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int64_t o = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += o;
+    uint32_t ia = a, ib = b;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t oa = __shfl_up(ia, d, 64), ob = __shfl_up(ib, d, 64);
+        if (lane >= d) {
+            ia += oa;
+            ib += ob;
         }
-        if (lane == 63) wave_sums[wave] = incl;
-        __syncthreads();
-        int64_t before = carry, chunk = 0;
-        for (int w = 0; w < kDigitScanBlock / 64; ++w) {
-            const int64_t ws = wave_sums[w];
-            before += w < wave ? ws : 0;
-            chunk += ws;
-        }
-        if (k < nt) offsets[seg + k] = before + incl - v;
-        carry += chunk;
-        __syncthreads();
     }
+    if (lane == 63) {
+        sh[0][wave] = ia;
+        sh[1][wave] = ib;
+    }
+    __syncthreads();
+    uint32_t ba = 0u, bb = 0u;
+    for (int w = 0; w < kWaves; ++w) {
+        ba += w < wave ? sh[0][w] : 0u;
+        bb += w < wave ? sh[1][w] : 0u;
+    }
+    a = ba + ia - a;
+    b = bb + ib - b;
 }
 
+// Scatters one tile.  Wave w of the workgroup holds codes [w * 64 * kItems, ...)
+// of the tile, 64 at a time in order; a code's rank among its digit's codes is
+// the number that earlier rounds of its wave counted (wc), plus its lower lanes
+// of the same digit (one ballot per digit bit), plus the earlier waves' totals.
+// The tile is put into digit order in LDS first, so that codes of one digit
+// leave as runs.  FIRST: the values are the codes' own indices.
+template <bool FIRST>
 __global__ void __launch_bounds__(kBlock) scatter_digits(const uint32_t* __restrict__ kin,
                                                          const uint32_t* __restrict__ vin, int64_t n, int shift,
-                                                         const int64_t* __restrict__ offsets,
+                                                         int super_log, int32_t nsupers,
+                                                         const uint32_t* __restrict__ counts,
+                                                         const uint32_t* __restrict__ supers,
                                                          uint32_t* __restrict__ kout, uint32_t* __restrict__ vout) {
-    __shared__ uint32_t wc[kWaves * kRadix];
-    __shared__ uint32_t run[kRadix];
-    uint32_t key[kItems], digit[kItems], rank[kItems];
-    tile_ranks(kin, n, shift, key, digit, rank, wc, run);
+    __shared__ uint32_t wc[kWaves][kRadix];
+    __shared__ uint32_t gofs[kRadix];
+    __shared__ uint32_t lkey[kTile], lval[kTile];
+    __shared__ uint32_t sh[2][kWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int64_t tile0 = int64_t(blockIdx.x) * kTile;
+    const int64_t base = tile0 + wave * (64 * kItems) + lane;
+    uint32_t key[kItems], val[kItems], rank[kItems];
+#pragma unroll
     for (int r = 0; r < kItems; ++r) {
-        const int64_t i = int64_t(blockIdx.x) * kTile + r * kBlock + threadIdx.x;
-        if (i >= n) continue;
-        const int64_t pos = offsets[int64_t(digit[r]) * gridDim.x + blockIdx.x] + rank[r];
-        kout[pos] = key[r];
-        vout[pos] = vin[i];
+        const int64_t i = base + r * 64;
+        key[r] = i < n ? kin[i] : 0u;
+        val[r] = FIRST ? uint32_t(i) : (i < n ? vin[i] : 0u);
+    }
+    // thread d: digit d's codes in all tiles, and in the tiles before this one
+    uint32_t total = 0u, before = 0u;
+    const int32_t mine = int32_t(blockIdx.x) >> super_log;
+#pragma unroll 8
+    for (int32_t k = 0; k < nsupers; ++k) {
+        const uint32_t c = supers[int64_t(k) * kRadix + threadIdx.x];
+        total += c;
+        before += k < mine ? c : 0u;
+    }
+#pragma unroll 8
+    for (int32_t t = mine << super_log; t < int32_t(blockIdx.x); ++t) before += counts[int64_t(t) * kRadix + threadIdx.x];
+    for (int w = 0; w < kWaves; ++w) wc[w][threadIdx.x] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const bool valid = base + r * 64 < n;
+        const uint32_t d = (key[r] >> shift) & (kRadix - 1);
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < kDigitBits; ++b) {
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bb = __ballot(bit);
+            peers &= bit ? bb : ~bb;
+        }
+        // one wave's LDS accesses run in order, so every lane reads the count
+        // before its digit's first lane adds this round's
+        uint32_t old = 0u;
+        if (valid) old = wc[wave][d];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && (peers & below) == 0ull) wc[wave][d] = old + uint32_t(__popcll(peers));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        rank[r] = old + uint32_t(__popcll(peers & below));
+    }
+    __syncthreads();
+    // thread d: digit d's start in the tile (local) and in the output (global)
+    uint32_t in_tile = 0u;
+    for (int w = 0; w < kWaves; ++w) {
+        const uint32_t c = wc[w][threadIdx.x];
+        wc[w][threadIdx.x] = in_tile;
+        in_tile += c;
+    }
+    uint32_t global = total, local = in_tile;
+    block_prefix2(global, local, sh);
+    for (int w = 0; w < kWaves; ++w) wc[w][threadIdx.x] += local;
+    gofs[threadIdx.x] = global + before - local;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        if (base + r * 64 < n) {
+            const uint32_t p = wc[wave][(key[r] >> shift) & (kRadix - 1)] + rank[r];
+            lkey[p] = key[r];
+            lval[p] = val[r];
+        }
+    }
+    __syncthreads();
+    const int32_t here = int32_t(n - tile0 < kTile ? n - tile0 : kTile);
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const int32_t p = r * kBlock + int32_t(threadIdx.x);
+        if (p < here) {
+            const uint32_t k = lkey[p];
+            const uint32_t pos = gofs[(k >> shift) & (kRadix - 1)] + uint32_t(p);
+            kout[pos] = k;
+            vout[pos] = lval[p];
+        }
     }
 }
 
-// Longest common prefix of sorted codes i and j (Karras's delta); -1 outside [0, n).
-__device__ __forceinline__ int delta(const uint32_t* __restrict__ keys, int64_t n, int64_t i, int64_t j) {
+// Longest common prefix of the codes a at sorted index i and b at j (Karras's
+// delta; equal codes are told apart by their indices).
+__device__ __forceinline__ int prefix_len(uint32_t a, uint32_t b, int64_t i, int64_t j) {
+    return a == b ? 32 + __clz(uint32_t(i ^ j)) : __clz(a ^ b);
+}
+
+// delta over the sorted codes in memory; -1 outside [0, n).
+__device__ __forceinline__ int delta(const uint32_t* __restrict__ keys, int64_t n, int64_t i, uint32_t key_i,
+                                     int64_t j) {
     if (j < 0 || j >= n) return -1;
-    const uint32_t a = keys[i], b = keys[j];
-    if (a == b) return 32 + __clz(uint32_t(i ^ j));
-    return __clz(a ^ b);
+    return prefix_len(key_i, keys[j], i, j);
 }
 
-// Internal node i (0 <= i < n - 1): children (c < n - 1: internal c; else leaf c - (n - 1)), covered leaf
-// range, and the parent of every node (parent[internal c] at c, parent[leaf l] at n - 1 + l).
-__global__ void __launch_bounds__(kBlock) karras(const uint32_t* __restrict__ keys, int64_t n,
-                                                 int2* __restrict__ child, int2* __restrict__ range,
-                                                 int32_t* __restrict__ parent, unsigned* __restrict__ span_count) {
-    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i == 0) *span_count = 0u;   // the boxes pass appends to the span list
-    if (i >= n - 1) return;
-    const int d = delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1) >= 0 ? 1 : -1;
-    const int dmin = delta(keys, n, i, i - d);
-    int64_t lmax = 2;
-    while (delta(keys, n, i, i + lmax * d) > dmin) lmax *= 2;
-    int64_t l = 0;
-    for (int64_t t = lmax / 2; t >= 1; t /= 2)
-        if (delta(keys, n, i, i + (l + t) * d) > dmin) l += t;
-    const int64_t j = i + l * d;
-    const int dnode = delta(keys, n, i, j);
-    int64_t s = 0;
-    int64_t t = l;
-    do {
-        t = (t + 1) >> 1;
-        if (delta(keys, n, i, i + (s + t) * d) > dnode) s += t;
-    } while (t > 1);
-    const int64_t gamma = i + s * d + (d < 0 ? -1 : 0);
-    const int64_t first = i < j ? i : j, last = i < j ? j : i;
-    const int32_t left = int32_t(first == gamma ? (n - 1) + gamma : gamma);
-    const int32_t right = int32_t(last == gamma + 1 ? (n - 1) + gamma + 1 : gamma + 1);
-    child[i] = make_int2(left, right);
-    range[i] = make_int2(int32_t(first), int32_t(last));
-    parent[left] = int32_t(i);
-    parent[right] = int32_t(i);
-}
-
-// Boxes.  A node's box is the min / max over the triangle boxes of its leaf
-// range, which min / max give exactly in any order, so the boxes equal a
-// bottom-up union's bit for bit.
-//
-// Karras's tree gives internal node i a leaf range with one end at i, so a
-// node whose range lies in one workgroup's kBoxBlock leaves has its index in
-// that workgroup's leaf index range, and its whole subtree is computed by that
-// workgroup: a thread per leaf climbs while it is the second of a node's two
-// children to arrive (counters and boxes in LDS, workgroup scope).  The same
-// pass writes each leaf's prefix box (the chunk's leaves up to it) and suffix
-// box (from it to the chunk's end) and lists, a thread per internal node, the
-// nodes whose range spans chunks.  The span pass then gives each listed node
-// [a, b] the union of suffix(a), prefix(b) and the whole chunks between them
-// (a chunk's box is the suffix box of its first leaf).  No pass has a chain
-// of dependent steps through the upper tree, and none needs agent-scope
-// fences, which on this chip write back and invalidate an XCD's L2.
-constexpr int kBoxBlock = 1024;
-constexpr int kSpanGrid = 512;   // workgroups of the span pass (kBlock threads, a node per wave)
-
+// A node's box is the min / max over the triangle boxes of its leaf range,
+// which min / max give exactly in any order and from overlapping parts, so the
+// boxes equal a bottom-up union's bit for bit.
 __device__ __forceinline__ Box unite(const Box& a, const Box& b) {
     Box u;
     for (int q = 0; q < 3; ++q) {
@@ -361,106 +393,13 @@ __device__ __forceinline__ Box empty_box() {
     return b;
 }
 
-__device__ __forceinline__ Box shfl_box(const Box& b, int src_lane) {
-    Box o;
+// Union over the wave's lanes; every lane gets it.
+__device__ __forceinline__ Box wave_unite(Box b) {
     for (int q = 0; q < 3; ++q) {
-        o.lo[q] = __shfl(b.lo[q], src_lane, 64);
-        o.hi[q] = __shfl(b.hi[q], src_lane, 64);
+        b.lo[q] = wave_min(b.lo[q]);
+        b.hi[q] = wave_max(b.hi[q]);
     }
-    return o;
-}
-
-__global__ void __launch_bounds__(kBoxBlock) boxes_local(const crt_vertex* __restrict__ v,
-                                                         const uint32_t* __restrict__ idx,
-                                                         const uint32_t* __restrict__ order, int64_t n,
-                                                         const int2* __restrict__ child, const int2* __restrict__ range,
-                                                         const int32_t* __restrict__ parent, Box* __restrict__ boxes,
-                                                         Box* __restrict__ pre, Box* __restrict__ suf,
-                                                         Box* __restrict__ leaf_box, int32_t* __restrict__ span,
-                                                         unsigned* __restrict__ span_count) {
-    __shared__ unsigned lflag[kBoxBlock];
-    __shared__ Box lbox[kBoxBlock];
-    __shared__ Box ltri[kBoxBlock];   // the chunk's leaf boxes, for the climb
-    __shared__ Box wave_pre[kBoxBlock / 64], wave_suf[kBoxBlock / 64];
-    const int64_t base = int64_t(blockIdx.x) * kBoxBlock;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t l = base + threadIdx.x;
-    const bool valid = l < n;
-    lflag[threadIdx.x] = 0u;
-    // prefix and suffix boxes of the chunk: wave scans, then the wave totals
-    const Box tb = valid ? tri_box(v, idx, int64_t(order[l])) : empty_box();
-    ltri[threadIdx.x] = tb;
-    Box p = tb, q = tb;
-    for (int d = 1; d < 64; d <<= 1) {
-        const Box op = shfl_box(p, lane >= d ? lane - d : lane);
-        const Box oq = shfl_box(q, lane + d < 64 ? lane + d : lane);
-        if (lane >= d) p = unite(p, op);
-        if (lane + d < 64) q = unite(q, oq);
-    }
-    if (lane == 63) wave_pre[wave] = p;
-    if (lane == 0) wave_suf[wave] = q;
-    __syncthreads();
-    for (int w = 0; w < kBoxBlock / 64; ++w) {
-        if (w < wave) p = unite(p, wave_pre[w]);
-        if (w > wave) q = unite(q, wave_suf[w]);
-    }
-    // internal node l (l < n - 1) goes to the span list when its range leaves
-    // one chunk: a ballot per wave, one append per wave
-    bool spans = false;
-    if (l < n - 1) {
-        const int2 r = range[l];
-        spans = r.x / kBoxBlock != r.y / kBoxBlock;
-    }
-    const uint64_t ballot = __ballot(spans);
-    if (ballot) {
-        unsigned at = 0;
-        if (lane == 0)
-            at = __hip_atomic_fetch_add(span_count, unsigned(__popcll(ballot)), __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-        at = __shfl(at, 0, 64);
-        const unsigned below =
-            __builtin_amdgcn_mbcnt_hi(uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u));
-        if (spans) span[at + below] = int32_t(l);
-    }
-    if (!valid) return;   // no barrier below
-    pre[l] = p;
-    suf[l] = q;
-    leaf_box[l] = tb;   // emit writes the leaf children from these
-    int32_t node = parent[(n - 1) + l];
-    while (node >= 0) {
-        const int2 r = range[node];
-        if (r.x / kBoxBlock != r.y / kBoxBlock) return;   // the span pass forms it
-        const int32_t li = node - int32_t(base);   // in [0, kBoxBlock): node lies in this workgroup's leaf range
-        if (__hip_atomic_fetch_add(&lflag[li], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u) return;
-        const int2 c = child[node];
-        // a local node's children lie in this chunk: leaves in ltri, nodes in lbox
-        const Box b0 = c.x >= n - 1 ? ltri[c.x - int32_t(n - 1) - int32_t(base)] : lbox[c.x - int32_t(base)];
-        const Box b1 = c.y >= n - 1 ? ltri[c.y - int32_t(n - 1) - int32_t(base)] : lbox[c.y - int32_t(base)];
-        const Box u = unite(b0, b1);
-        lbox[li] = u;
-        boxes[node] = u;
-        node = node == 0 ? -1 : parent[node];
-    }
-}
-
-// A wave per listed node: suffix(a), prefix(b) and the whole chunks of
-// [a, b] between them, united across the wave.
-__global__ void __launch_bounds__(kBlock) boxes_span(const int2* __restrict__ range, const int32_t* __restrict__ span,
-                                                     const unsigned* __restrict__ span_count,
-                                                     const Box* __restrict__ pre, const Box* __restrict__ suf,
-                                                     Box* __restrict__ boxes) {
-    const unsigned count = *span_count;
-    const int lane = threadIdx.x & 63;
-    const unsigned waves = gridDim.x * (kBlock / 64);
-    for (unsigned e = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); e < count; e += waves) {
-        const int32_t node = span[e];
-        const int2 r = range[node];
-        const int64_t ca = r.x / kBoxBlock, cb = r.y / kBoxBlock;
-        Box acc = lane == 0 ? suf[r.x] : lane == 1 ? pre[r.y] : empty_box();
-        for (int64_t k = ca + 1 + lane; k < cb; k += 64) acc = unite(acc, suf[k * kBoxBlock]);
-        for (int d = 32; d > 0; d >>= 1) acc = unite(acc, shfl_box(acc, lane ^ d));
-        if (lane == 0) boxes[node] = acc;
-    }
+    return b;
 }
 
 // Packed leaf word (start << 4 | count) as the stack layout stores it.
@@ -468,58 +407,280 @@ __device__ __forceinline__ int32_t leaf_word(int64_t start, int32_t count) {
     return int32_t((uint32_t(start) << 4) | uint32_t(count));
 }
 
-__device__ __forceinline__ void put_child(crt_bounds& out, const Box& b, int32_t w_min, int32_t w_max) {
-    for (int q = 0; q < 3; ++q) {
-        out.min[q] = b.lo[q];
-        out.max[q] = b.hi[q];
-    }
-    out.min[3] = __int_as_float(w_min);
-    out.max[3] = __int_as_float(w_max);
+// Stack entry of an internal node whose children cover leaves [first, gamma]
+// and [gamma + 1, last]: internal child c has index gamma or gamma + 1.
+__device__ __forceinline__ void put_entry(crt_stack_node* __restrict__ out, int32_t t_offset, int64_t first,
+                                          int64_t gamma, int64_t last, const Box& l, const Box& r) {
+    const int64_t nl = gamma - first + 1, nr = last - gamma;
+    const int32_t wl = nl <= 2 ? leaf_word(int64_t(t_offset) + first, int32_t(nl)) : -1;
+    const int32_t wr = nr <= 2 ? leaf_word(int64_t(t_offset) + gamma + 1, int32_t(nr)) : -1;
+    float4* o = reinterpret_cast<float4*>(out);
+    o[0] = make_float4(l.lo[0], l.lo[1], l.lo[2], __int_as_float(wl));
+    o[1] = make_float4(l.hi[0], l.hi[1], l.hi[2], __int_as_float(nl <= 2 ? 0 : int32_t(gamma)));
+    o[2] = make_float4(r.lo[0], r.lo[1], r.lo[2], __int_as_float(wr));
+    o[3] = make_float4(r.hi[0], r.hi[1], r.hi[2], __int_as_float(nr <= 2 ? 0 : int32_t(gamma + 1)));
 }
 
-// Entry i of the stack layout from internal node i; the sorted triangle array.
-__global__ void __launch_bounds__(kBlock) emit(const crt_vertex* __restrict__ v, const uint32_t* __restrict__ idx,
-                                               const int32_t* __restrict__ mesh, int32_t mesh_all,
-                                               const uint32_t* __restrict__ order, int64_t n, int32_t t_offset,
-                                               const int2* __restrict__ child, const int2* __restrict__ range,
-                                               const Box* __restrict__ boxes, const Box* __restrict__ leaf_box,
-                                               crt_stack_node* __restrict__ nodes, crt_triangle* __restrict__ tris) {
-    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t t = order[i];
-    crt_triangle tr;
-    tr.packed[0] = int32_t(idx[3 * int64_t(t) + 0]);
-    tr.packed[1] = int32_t(idx[3 * int64_t(t) + 1]);
-    tr.packed[2] = int32_t(idx[3 * int64_t(t) + 2]);
-    tr.packed[3] = mesh ? mesh[t] : mesh_all;
-    *reinterpret_cast<int4*>(tris + i) = *reinterpret_cast<const int4*>(tr.packed);
-    if (i >= n - 1) return;
-    const int2 c = child[i];
-    crt_stack_node e;
-    for (int k = 0; k < 2; ++k) {
-        const int32_t cc = k == 0 ? c.x : c.y;
-        crt_bounds& out = k == 0 ? e.left : e.right;
-        if (cc >= n - 1) {
-            const int32_t leaf = cc - int32_t(n - 1);
-            put_child(out, leaf_box[leaf], leaf_word(int64_t(t_offset) + leaf, 1), 0);
-        } else if (range[cc].y - range[cc].x == 1) {
-            put_child(out, boxes[cc], leaf_word(int64_t(t_offset) + range[cc].x, 2), 0);
-        } else {
-            put_child(out, boxes[cc], -1, cc);
+// The tree, its boxes and its entries, a chunk of kChunk leaves per workgroup
+// and a thread per leaf and internal node.  Karras's tree gives internal node
+// i a leaf range with one end at i, so the code just outside the chunk on the
+// range's side tells whether the range ends inside (delta falls with the
+// distance).  Such a node finds its range and split by binary searches over
+// the chunk's codes in LDS.  Its children's boxes are two windows each of a
+// table of boxes over 2^k leaves, which is built level by level in two LDS
+// buffers, a level's queries answered while it is there: 24 KB in all, so the
+// CU keeps its 32 waves.  Nodes whose range leaves the chunk are marked in a
+// bit mask for span_nodes (no list: its one counter took 300 us), which also reads the leaf boxes and 64-leaf boxes written here.
+//
+// Bound: the gathers of the sorted triangles' indices and vertices and the
+// 64-byte entries (about 190 bytes a triangle).  2.56M triangles: 104 us, 4.7
+// TB/s; one launch each for the tree, a bottom-up climb for the boxes and the
+// entries took 71 + 230 + 110 us, with child, range, parent and four box arrays
+// between.
+constexpr int kChunkBits = 9;
+constexpr int kChunk = 1 << kChunkBits;
+static_assert(kChunk % 64 == 0 && kChunk / 64 <= 16, "a chunk is whole 64-leaf groups");
+
+__global__ void __launch_bounds__(kChunk) chunk_nodes(const crt_vertex* __restrict__ v,
+                                                      const uint32_t* __restrict__ idx,
+                                                      const int32_t* __restrict__ mesh, int32_t mesh_all,
+                                                      const uint32_t* __restrict__ keys,
+                                                      const uint32_t* __restrict__ order, int64_t n, int32_t t_offset,
+                                                      Box* __restrict__ leaf_box, Box* __restrict__ group_box,
+                                                      uint64_t* __restrict__ span,
+                                                      crt_stack_node* __restrict__ nodes,
+                                                      crt_triangle* __restrict__ tris) {
+    __shared__ uint32_t code[kChunk + 2];   // code[1 + k]: leaf base + k; one more at each end
+    __shared__ float win[2][6][kChunk];     // boxes over 2^k leaves from each leaf, two levels
+    const int64_t base = int64_t(blockIdx.x) * kChunk;
+    const int li = int(threadIdx.x), lane = li & 63;
+    const int64_t i = base + li;
+    code[1 + li] = i < n ? keys[i] : 0u;
+    if (li == 0) code[0] = base > 0 ? keys[base - 1] : 0u;
+    if (li == kChunk - 1) code[kChunk + 1] = i + 1 < n ? keys[i + 1] : 0u;
+    Box cur = empty_box();
+    if (i < n) {
+        const int64_t t = int64_t(order[i]);
+        const uint32_t i0 = idx[3 * t + 0], i1 = idx[3 * t + 1], i2 = idx[3 * t + 2];
+        const float4 p0 = *reinterpret_cast<const float4*>(v[i0].position);
+        const float4 p1 = *reinterpret_cast<const float4*>(v[i1].position);
+        const float4 p2 = *reinterpret_cast<const float4*>(v[i2].position);
+        *reinterpret_cast<int4*>(tris + i) = make_int4(int32_t(i0), int32_t(i1), int32_t(i2), mesh ? mesh[t] : mesh_all);
+        cur.lo[0] = fminf(fminf(p0.x, p1.x), p2.x);
+        cur.lo[1] = fminf(fminf(p0.y, p1.y), p2.y);
+        cur.lo[2] = fminf(fminf(p0.z, p1.z), p2.z);
+        cur.hi[0] = fmaxf(fmaxf(p0.x, p1.x), p2.x);
+        cur.hi[1] = fmaxf(fmaxf(p0.y, p1.y), p2.y);
+        cur.hi[2] = fmaxf(fmaxf(p0.z, p1.z), p2.z);
+        leaf_box[i] = cur;
+    }
+    for (int q = 0; q < 3; ++q) {
+        win[0][q][li] = cur.lo[q];
+        win[0][3 + q][li] = cur.hi[q];
+    }
+    __syncthreads();
+
+    // node i's range and split, all in chunk positions (position p = leaf base + p)
+    const uint32_t own = code[1 + li];
+    auto dl = [&](int p) {   // delta(i, base + p), p in [-1, kChunk]
+        const int64_t j = base + p;
+        return j < 0 || j >= n ? -1 : prefix_len(own, code[1 + p], i, j);
+    };
+    bool here = false, spans = false;
+    int first = 0, gamma = 0, last = 0;
+    if (i < n - 1) {
+        const int up = dl(li + 1), down = dl(li - 1);
+        const int d = up - down >= 0 ? 1 : -1;
+        const int dmin = d > 0 ? down : up;
+        here = dl(d > 0 ? kChunk : -1) <= dmin;
+        spans = !here;
+        if (here) {
+            int l = 0;
+            for (int t = kChunk / 2; t >= 1; t /= 2) {
+                const int p = li + (l + t) * d;
+                if (p >= 0 && p < kChunk && dl(p) > dmin) l += t;
+            }
+            const int dnode = dl(li + l * d);
+            int s = 0;
+            for (int t = kChunk / 2; t >= 1; t /= 2) {
+                const int p = li + (s + t) * d;
+                if (s + t < l && dl(p) > dnode) s += t;
+            }
+            gamma = li + s * d + (d < 0 ? -1 : 0);
+            first = d > 0 ? li : li - l;
+            last = d > 0 ? li + l : li;
         }
     }
-    nodes[i] = e;
+    const uint64_t ballot = __ballot(spans);
+    if (lane == 0 && i < n) span[i >> 6] = ballot;
+
+    // a range of m leaves is covered by two windows of 2^k, k = floor(log2 m)
+    // (at most 2^(kChunkBits - 1), whose two windows cover a whole chunk)
+    const int kl = here ? min(31 - __clz(gamma - first + 1), kChunkBits - 1) : -1;
+    const int kr = here ? min(31 - __clz(last - gamma), kChunkBits - 1) : -1;
+    Box bl = empty_box(), br = empty_box();
+#pragma unroll 1
+    for (int k = 0; k < kChunkBits; ++k) {
+        const float(*w)[kChunk] = win[k & 1];
+        auto window = [&](int p) {
+            Box b;
+            for (int q = 0; q < 3; ++q) {
+                b.lo[q] = w[q][p];
+                b.hi[q] = w[3 + q][p];
+            }
+            return b;
+        };
+        if (k == kl) bl = unite(window(first), window(gamma + 1 - (1 << k)));
+        if (k == kr) br = unite(window(gamma + 1), window(last + 1 - (1 << k)));
+        if (k == 6 && lane == 0 && i < n) group_box[i >> 6] = cur;
+        if (k + 1 < kChunkBits) {
+            if (li + (1 << k) < kChunk) cur = unite(cur, window(li + (1 << k)));
+            float(*o)[kChunk] = win[(k + 1) & 1];
+            for (int q = 0; q < 3; ++q) {
+                o[q][li] = cur.lo[q];
+                o[3 + q][li] = cur.hi[q];
+            }
+            __syncthreads();
+        }
+    }
+    if (here) put_entry(nodes + i, t_offset, base + first, base + gamma, base + last, bl, br);
+}
+
+// Boxes of 64 groups (4,096 leaves), a wave each.
+__global__ void __launch_bounds__(kBlock) super_boxes(const Box* __restrict__ group_box, int64_t groups,
+                                                      Box* __restrict__ super_box) {
+    const int lane = threadIdx.x & 63;
+    const int64_t s = int64_t(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+    const int64_t g = s * 64 + lane;
+    if (s * 64 >= groups) return;
+    const Box b = wave_unite(g < groups ? group_box[g] : empty_box());
+    if (lane == 0) super_box[s] = b;
+}
+
+// The span pass gives a node kTeam lanes, a DPP row: its searches probe kTeam
+// places a round, and its reductions are row rotations without LDS.
+constexpr int kTeam = 16;
+
+template <int ROR>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROR, 0xF, 0xF, false));
+}
+
+// Union over the team's lanes (all active); every lane gets it.
+__device__ __forceinline__ Box team_unite(Box b) {
+    for (int q = 0; q < 3; ++q) {
+        b.lo[q] = fminf(b.lo[q], row_ror<8>(b.lo[q]));
+        b.lo[q] = fminf(b.lo[q], row_ror<4>(b.lo[q]));
+        b.lo[q] = fminf(b.lo[q], row_ror<2>(b.lo[q]));
+        b.lo[q] = fminf(b.lo[q], row_ror<1>(b.lo[q]));
+        b.hi[q] = fmaxf(b.hi[q], row_ror<8>(b.hi[q]));
+        b.hi[q] = fmaxf(b.hi[q], row_ror<4>(b.hi[q]));
+        b.hi[q] = fmaxf(b.hi[q], row_ror<2>(b.hi[q]));
+        b.hi[q] = fmaxf(b.hi[q], row_ror<1>(b.hi[q]));
+    }
+    return b;
+}
+
+// Team-wide count of a flag.
+__device__ __forceinline__ int team_count(bool flag) {
+    return __popc(uint32_t(__ballot(flag) >> (threadIdx.x & 48)) & 0xFFFFu);
+}
+
+// Box of leaves [a, b], formed by one team: the leaves of the two end groups,
+// the groups of the two end super-groups and the super-groups between.
+__device__ __forceinline__ Box range_box(const Box* __restrict__ leaf_box, const Box* __restrict__ group_box,
+                                         const Box* __restrict__ super_box, int64_t a, int64_t b, int rank) {
+    Box acc = empty_box();
+    const int64_t ga = a >> 6, gb = b >> 6;
+    for (int64_t k = a + rank; k <= min(b, (ga << 6) + 63); k += kTeam) acc = unite(acc, leaf_box[k]);
+    if (gb > ga) {
+        for (int64_t k = (gb << 6) + rank; k <= b; k += kTeam) acc = unite(acc, leaf_box[k]);
+        // whole groups (ga, gb): by super-group where one lies whole between
+        const int64_t g0 = ga + 1, g1 = gb - 1, sa = g0 >> 6, sb = g1 >> 6;
+        for (int64_t k = g0 + rank; k <= min(g1, (sa << 6) + 63); k += kTeam) acc = unite(acc, group_box[k]);
+        if (g0 <= g1 && sb > sa) {
+            for (int64_t k = (sb << 6) + rank; k <= g1; k += kTeam) acc = unite(acc, group_box[k]);
+            for (int64_t k = sa + 1 + rank; k < sb; k += kTeam) acc = unite(acc, super_box[k]);
+        }
+    }
+    return team_unite(acc);
+}
+
+// Largest l in [lo, hi) with delta(i, i + l * d) > dmin, given that it holds at
+// lo and fails at hi: the team's lanes probe kTeam distances per round.
+__device__ __forceinline__ int64_t last_above(const uint32_t* __restrict__ keys, int64_t n, int64_t i, uint32_t key_i,
+                                              int d, int dmin, int64_t lo, int64_t hi, int rank) {
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + kTeam) / (kTeam + 1);   // probes lo + step, lo + 2 step, ..., below hi
+        const int64_t l = lo + (rank + 1) * step;
+        // delta falls with l, so the first c probes hold
+        const int64_t c = team_count(l < hi && delta(keys, n, i, key_i, i + l * d) > dmin);
+        lo += c * step;
+        hi = min(hi, lo + step);
+    }
+    return lo;
+}
+
+// A workgroup per chunk, a team per listed node of the chunk: the node's range
+// and split as chunk_nodes finds them, its children's boxes and its entry.  A
+// chain of about ten dependent loads per node bounds it, so nodes have to be
+// many at once: 45 us for 2.56M triangles, where a wave per node and chunks of
+// 256 (twice the nodes) took 96.
+__global__ void __launch_bounds__(kBlock) span_nodes(const uint32_t* __restrict__ keys, int64_t n, int32_t t_offset,
+                                                     const uint64_t* __restrict__ span,
+                                                     const Box* __restrict__ leaf_box,
+                                                     const Box* __restrict__ group_box,
+                                                     const Box* __restrict__ super_box,
+                                                     crt_stack_node* __restrict__ nodes) {
+    const int rank = int(threadIdx.x) % kTeam, team = int(threadIdx.x) / kTeam;
+    // lane r of a team holds group r's mask and the listed nodes in the groups before it
+    const int64_t g = int64_t(blockIdx.x) * (kChunk / 64) + rank;
+    const uint64_t mask = rank < kChunk / 64 && g * 64 < n ? span[g] : 0ull;
+    const int count = __popcll(mask);
+    int incl = count;
+    for (int k = 1; k < kTeam; k <<= 1) {
+        const int o = __shfl_up(incl, k, kTeam);
+        if (rank >= k) incl += o;
+    }
+    const int listed = __shfl(incl, kTeam - 1, kTeam);
+    for (int e = team; e < listed; e += kBlock / kTeam) {
+        // the group that holds the e-th listed node, and its bit
+        const int group = team_count(incl <= e);
+        int skip = e - __shfl(incl - count, group, kTeam);
+        uint64_t m = uint64_t(uint32_t(__shfl(int(mask), group, kTeam))) |
+                     uint64_t(uint32_t(__shfl(int(mask >> 32), group, kTeam))) << 32;
+        for (; skip > 0; --skip) m &= m - 1;
+        const int64_t i = (int64_t(blockIdx.x) * (kChunk / 64) + group) * 64 + __ffsll((long long)m) - 1;
+        const uint32_t key_i = keys[i];
+        const int up = delta(keys, n, i, key_i, i + 1), down = delta(keys, n, i, key_i, i - 1);
+        const int d = up - down >= 0 ? 1 : -1;
+        const int dmin = d > 0 ? down : up;
+        // powers of two first: lane r probes distances 2^r and 2^(r + 16), below 2^30
+        const bool near = delta(keys, n, i, key_i, i + (int64_t(1) << rank) * d) > dmin;
+        const bool far = rank < 14 && delta(keys, n, i, key_i, i + (int64_t(65536) << rank) * d) > dmin;
+        const int c = team_count(near) + team_count(far);   // >= 1: the neighbour on this side shares a longer prefix
+        const int64_t l = last_above(keys, n, i, key_i, d, dmin, int64_t(1) << (c - 1), int64_t(1) << c, rank);
+        const int64_t j = i + l * d;
+        const int dnode = delta(keys, n, i, key_i, j);
+        const int64_t s = last_above(keys, n, i, key_i, d, dnode, 0, l, rank);
+        const int64_t gamma = i + s * d + (d < 0 ? -1 : 0);
+        const int64_t first = i < j ? i : j, last = i < j ? j : i;
+        const Box bl = range_box(leaf_box, group_box, super_box, first, gamma, rank);
+        const Box br = range_box(leaf_box, group_box, super_box, gamma + 1, last, rank);
+        if (rank == 0) put_entry(nodes + i, t_offset, first, gamma, last, bl, br);
+    }
 }
 
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct Layout {
-    size_t keys[2], vals[2], counts, offsets, partial, frame, child, range, parent, boxes, pre, suf, leaf_box,
-        span, span_count, bytes;
+    size_t keys[2], vals[2], counts, supers, partial, leaf_box, group_box, super_box, span, bytes;
+    int64_t tiles, nsupers, groups;
+    int super_log;
+    int32_t parts;   // workgroups of the bounds reduction
 };
 
 inline Layout layout(int64_t n) {
-    const size_t nb = size_t((n + kBlock - 1) / kBlock);
     const size_t un = size_t(n);
     Layout L{};
     size_t off = 0;
@@ -528,25 +689,27 @@ inline Layout layout(int64_t n) {
         off = align256(off + bytes);
         return at;
     };
+    L.tiles = (n + kTile - 1) / kTile;
+    // a tile adds up nsupers sums and up to 2^super_log counts: about the square root of the tiles each
+    L.super_log = 4;
+    while ((L.tiles >> (2 * L.super_log)) > 1) ++L.super_log;
+    L.nsupers = ((L.tiles - 1) >> L.super_log) + 1;
+    L.groups = (n + 63) / 64;
+    L.parts = int32_t(std::min<int64_t>(kBoundsGrid, (n + kBlock - 1) / kBlock));
     L.keys[0] = take(un * 4);
     L.keys[1] = take(un * 4);
     L.vals[0] = take(un * 4);
     L.vals[1] = take(un * 4);
-    const size_t nt = size_t((n + kTile - 1) / kTile);
-    L.counts = take(kRadix * nt * 4);
-    L.offsets = take(kRadix * nt * 8);
-    L.partial = take(nb * 6 * 4);
-    L.frame = take(6 * 4);
-    L.child = take(un * 8);
-    L.range = take(un * 8);
-    L.parent = take(2 * un * 4);
-    L.boxes = take(un * sizeof(Box));
-    L.pre = take(un * sizeof(Box));
-    L.suf = take(un * sizeof(Box));
+    L.counts = take(size_t(L.tiles) * kRadix * 4);
+    L.supers = take(size_t(kPasses) * size_t(L.nsupers) * kRadix * 4);
+    L.partial = take(size_t(L.parts) * 6 * 4);
     L.leaf_box = take(un * sizeof(Box));
-    L.span = take(un * 4);
-    L.span_count = take(4);
-    L.bytes = off;
+    L.group_box = take(size_t(L.groups) * sizeof(Box));
+    L.super_box = take(size_t((L.groups + 63) / 64) * sizeof(Box));
+    L.span = take(size_t(L.groups) * 8);
+    // at least 140 bytes a triangle, what callers have been told to reserve
+    // (the arrays above take about 42)
+    L.bytes = align256(std::max(off, un * 140));
     return L;
 }
 
@@ -580,43 +743,45 @@ int crt_build_bvh_gpu(const crt_vertex* vertices, int64_t nverts, const uint32_t
     uint32_t* keys[2] = {static_cast<uint32_t*>(at(L.keys[0])), static_cast<uint32_t*>(at(L.keys[1]))};
     uint32_t* vals[2] = {static_cast<uint32_t*>(at(L.vals[0])), static_cast<uint32_t*>(at(L.vals[1]))};
     auto* counts = static_cast<uint32_t*>(at(L.counts));
-    auto* offsets = static_cast<int64_t*>(at(L.offsets));
+    auto* supers = static_cast<uint32_t*>(at(L.supers));
     auto* partial = static_cast<float*>(at(L.partial));
-    auto* frame = static_cast<float*>(at(L.frame));
-    auto* child = static_cast<int2*>(at(L.child));
-    auto* range = static_cast<int2*>(at(L.range));
-    auto* parent = static_cast<int32_t*>(at(L.parent));
-    auto* boxes = static_cast<Box*>(at(L.boxes));
-    auto* pre = static_cast<Box*>(at(L.pre));
-    auto* suf = static_cast<Box*>(at(L.suf));
     auto* leaf_box = static_cast<Box*>(at(L.leaf_box));
-    auto* span = static_cast<int32_t*>(at(L.span));
-    auto* span_count = static_cast<unsigned*>(at(L.span_count));
+    auto* group_box = static_cast<Box*>(at(L.group_box));
+    auto* super_box = static_cast<Box*>(at(L.super_box));
+    auto* span = static_cast<uint64_t*>(at(L.span));
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t n = ntris;
-    const unsigned nb = unsigned((n + kBlock - 1) / kBlock);
+    const int64_t super_words = L.nsupers * kRadix;   // per pass
 
-    hipLaunchKernelGGL(centroid_bounds, dim3(nb), dim3(kBlock), 0, st, vertices, indices, n, partial);
-    hipLaunchKernelGGL(finish_bounds, dim3(1), dim3(kBoundsBlock), 0, st, partial, int64_t(nb), frame);
-    hipLaunchKernelGGL(morton, dim3(nb), dim3(kBlock), 0, st, vertices, indices, n, frame, keys[0], vals[0]);
+    hipLaunchKernelGGL(centroid_bounds, dim3(unsigned(L.parts)), dim3(kBlock), 0, st, vertices, indices, n, partial,
+                       supers, kPasses * super_words);
+    const dim3 nt(unsigned(L.tiles));
+    hipLaunchKernelGGL(morton, nt, dim3(kBlock), 0, st, vertices, indices, n, partial, L.parts, keys[0], L.super_log,
+                       counts, supers);
     int cur = 0;
-    const unsigned nt = unsigned((n + kTile - 1) / kTile);
-    for (int shift = 0; shift < kMortonBits; shift += kDigitBits) {
-        hipLaunchKernelGGL(count_digits, dim3(nt), dim3(kBlock), 0, st, keys[cur], n, shift, counts);
-        hipLaunchKernelGGL(scan_digits, dim3(kRadix), dim3(kDigitScanBlock), 0, st, counts, int64_t(nt), offsets);
-        hipLaunchKernelGGL(scatter_digits, dim3(nt), dim3(kBlock), 0, st, keys[cur], vals[cur], n, shift, offsets,
-                           keys[1 - cur], vals[1 - cur]);
+    for (int pass = 0; pass < kPasses; ++pass) {
+        const int shift = pass * kDigitBits;
+        uint32_t* sums = supers + pass * super_words;
+        if (pass > 0)
+            hipLaunchKernelGGL(count_digits, nt, dim3(kBlock), 0, st, keys[cur], n, shift, L.super_log, counts, sums);
+        if (pass == 0)
+            hipLaunchKernelGGL(scatter_digits<true>, nt, dim3(kBlock), 0, st, keys[cur], vals[cur], n, shift,
+                               L.super_log, int32_t(L.nsupers), counts, sums, keys[1 - cur], vals[1 - cur]);
+        else
+            hipLaunchKernelGGL(scatter_digits<false>, nt, dim3(kBlock), 0, st, keys[cur], vals[cur], n, shift,
+                               L.super_log, int32_t(L.nsupers), counts, sums, keys[1 - cur], vals[1 - cur]);
         cur = 1 - cur;
     }
-    const unsigned ni = unsigned((n - 1 + kBlock - 1) / kBlock);
-    // karras also zeroes the span count (a kernel store, no memset node, so
-    // the chain stays capturable)
-    hipLaunchKernelGGL(karras, dim3(ni), dim3(kBlock), 0, st, keys[cur], n, child, range, parent, span_count);
-    hipLaunchKernelGGL(boxes_local, dim3(unsigned((n + kBoxBlock - 1) / kBoxBlock)), dim3(kBoxBlock), 0, st, vertices,
-                       indices, vals[cur], n, child, range, parent, boxes, pre, suf, leaf_box, span, span_count);
-    hipLaunchKernelGGL(boxes_span, dim3(kSpanGrid), dim3(kBlock), 0, st, range, span, span_count, pre, suf, boxes);
-    hipLaunchKernelGGL(emit, dim3(nb), dim3(kBlock), 0, st, vertices, indices, mesh_ids, mesh_id, vals[cur], n,
-                       t_offset, child, range, boxes, leaf_box, nodes, triangles);
+    const int64_t chunks = (n + kChunk - 1) / kChunk;
+    hipLaunchKernelGGL(chunk_nodes, dim3(unsigned(chunks)), dim3(kChunk), 0, st, vertices, indices, mesh_ids, mesh_id,
+                       keys[cur], vals[cur], n, t_offset, leaf_box, group_box, span, nodes, triangles);
+    if (chunks > 1) {   // one chunk holds every node
+        const int64_t super_groups = (L.groups + 63) / 64;
+        hipLaunchKernelGGL(super_boxes, dim3(unsigned((super_groups + 3) / 4)), dim3(kBlock), 0, st, group_box,
+                           L.groups, super_box);
+        hipLaunchKernelGGL(span_nodes, dim3(unsigned(chunks)), dim3(kBlock), 0, st, keys[cur], n, t_offset, span,
+                           leaf_box, group_box, super_box, nodes);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return crt::set_error(CRT_E_HIP, std::string("crt_build_bvh_gpu: kernel launch: ") + hipGetErrorString(e));
