@@ -89,59 +89,96 @@ __device__ __forceinline__ float half_area(const Kid& k) {
 
 // The slots of one wide node w, the expansion of stack entry `entry`: writes
 // its groups and kids[slot] (the stack entry of an inner child, -1
-// otherwise); returns its number of inner children.
+// otherwise); returns its number of inner children.  Every slot is addressed
+// by a constant once the loops are unrolled, so the children stay in registers
+// (a slot that the data chooses would put them in scratch memory), and a group
+// leaves as whole 16-byte stores.
 template <int W>
 __device__ __forceinline__ uint32_t expand_one(const crt_stack_node* __restrict__ nodes, int64_t node_count,
                                                int64_t ntris, int32_t entry, int64_t w, crt_wide_group* __restrict__ groups,
                                                int32_t* __restrict__ kids_out, unsigned* __restrict__ err) {
-    const crt_stack_node& e = nodes[entry];
+    const crt_stack_node e = nodes[entry];
     Kid kids[W];
-    int n = 0;
-    kids[n++] = make_kid(nodes, node_count, ntris, e.left, err);
-    kids[n++] = make_kid(nodes, node_count, ntris, e.right, err);
-    while (n < W) {
+    float area[W];   // half surface area of an inner child, -1 for a leaf
+    for (int k = 0; k < W; ++k) {
+        kids[k] = Kid{};
+        kids[k].entry = -1;
+        area[k] = -1.0f;
+    }
+    kids[0] = make_kid(nodes, node_count, ntris, e.left, err);
+    kids[1] = make_kid(nodes, node_count, ntris, e.right, err);
+    for (int k = 0; k < 2; ++k) area[k] = kids[k].entry >= 0 ? half_area(kids[k]) : -1.0f;
+    int n = 2;
+#pragma unroll
+    for (int step = 2; step < W; ++step) {
         int best = -1;
         float best_area = -1.0f;
-        for (int k = 0; k < n; ++k) {
-            if (kids[k].entry < 0) continue;
-            const float a = half_area(kids[k]);
-            if (a > best_area) {
-                best_area = a;
+        int32_t open = -1;
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            if (area[k] > best_area) {
+                best_area = area[k];
                 best = k;
+                open = kids[k].entry;
             }
         }
         if (best < 0) break;
-        const crt_stack_node& c = nodes[kids[best].entry];
-        for (int k = n; k > best + 1; --k) kids[k] = kids[k - 1];
-        kids[best + 1] = make_kid(nodes, node_count, ntris, c.right, err);
-        kids[best] = make_kid(nodes, node_count, ntris, c.left, err);
+        const crt_stack_node c = nodes[open];
+        const Kid l = make_kid(nodes, node_count, ntris, c.left, err);
+        const Kid r = make_kid(nodes, node_count, ntris, c.right, err);
+        const float al = l.entry >= 0 ? half_area(l) : -1.0f, ar = r.entry >= 0 ? half_area(r) : -1.0f;
+#pragma unroll
+        for (int k = W - 1; k >= 0; --k) {
+            if (k > best + 1) {
+                kids[k] = kids[k > 0 ? k - 1 : 0];
+                area[k] = area[k > 0 ? k - 1 : 0];
+            } else if (k == best + 1) {
+                kids[k] = r;
+                area[k] = ar;
+            } else if (k == best) {
+                kids[k] = l;
+                area[k] = al;
+            }
+        }
         ++n;
     }
     uint32_t m = 0;
-    for (int s = 0; s < W; ++s) {
-        crt_wide_group& g = groups[w * (W / 4) + s / 4];
-        const int j = s % 4;
-        const bool used = s < n;
-        const Kid& k = kids[used ? s : 0];
-        g.lo_x[j] = used ? k.lo[0] : 0.0f;
-        g.lo_y[j] = used ? k.lo[1] : 0.0f;
-        g.lo_z[j] = used ? k.lo[2] : 0.0f;
-        g.hi_x[j] = used ? k.hi[0] : 0.0f;
-        g.hi_y[j] = used ? k.hi[1] : 0.0f;
-        g.hi_z[j] = used ? k.hi[2] : 0.0f;
-        const bool inner = used && k.entry >= 0;
-        const bool leaf = used && !inner && k.count >= 1;   // else an empty slot (unused or failed a check)
-        g.child[j] = leaf ? k.start : 0;                     // inner: assign writes it
-        g.count[j] = inner ? 0 : (leaf ? k.count : -1);
-        kids_out[s] = inner ? k.entry : -1;
-        m += inner ? 1u : 0u;
+#pragma unroll
+    for (int q = 0; q < W / 4; ++q) {
+        crt_wide_group g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const Kid& k = kids[4 * q + j];
+            const bool used = 4 * q + j < n;
+            g.lo_x[j] = used ? k.lo[0] : 0.0f;
+            g.lo_y[j] = used ? k.lo[1] : 0.0f;
+            g.lo_z[j] = used ? k.lo[2] : 0.0f;
+            g.hi_x[j] = used ? k.hi[0] : 0.0f;
+            g.hi_y[j] = used ? k.hi[1] : 0.0f;
+            g.hi_z[j] = used ? k.hi[2] : 0.0f;
+            const bool inner = used && k.entry >= 0;
+            const bool leaf = used && !inner && k.count >= 1;   // else an empty slot (unused or failed a check)
+            g.child[j] = leaf ? k.start : 0;                     // inner: assign_slot writes it
+            g.count[j] = inner ? 0 : (leaf ? k.count : -1);
+            kids_out[4 * q + j] = inner ? k.entry : -1;
+            m += inner ? 1u : 0u;
+        }
+        groups[w * (W / 4) + q] = g;
     }
     return m;
 }
 
-// Child indices of wide node w: its inner children are next_base + off + 0,
-// 1, ... in slot order, and entries off, off + 1, ... of the next level's
-// list.  False when an index reaches cap (the links do not form a tree).
+// Numbers one inner child: slot s of wide node w is wide node idx.
+template <int W>
+__device__ __forceinline__ void assign_slot(int64_t w, int s, int64_t idx, crt_wide_group* __restrict__ groups) {
+    groups[w * (W / 4) + s / 4].child[s % 4] = int32_t(idx);
+}
+
+// Child indices of wide node w, one node at a time (the level passes of
+// wide_gpu.hip number a workgroup's slots at once): its inner children are
+// next_base + off + 0, 1, ... in slot order, and entries off, off + 1, ... of
+// the next level's list.  False when an index reaches cap (the links do not
+// form a tree).
 template <int W>
 __device__ __forceinline__ bool assign_one(int64_t w, const int32_t* __restrict__ kids, int64_t off,
                                            int64_t next_base, int64_t cap, crt_wide_group* __restrict__ groups,
@@ -156,7 +193,7 @@ __device__ __forceinline__ bool assign_one(int64_t w, const int32_t* __restrict_
             atomicOr(err, kErrCap);
             return false;
         }
-        groups[w * (W / 4) + s / 4].child[s % 4] = int32_t(idx);
+        assign_slot<W>(w, s, idx, groups);
         next_entries[off + r] = e;
         next_wides[off + r] = int32_t(idx);
         ++r;

@@ -15,10 +15,10 @@
 // test counts are identical.
 //
 // Nothing is read back between levels: the host launches a fixed number of
-// levels (two launches each: expand, then assign), the level sizes live on the
-// device, and a level past the tree's depth returns at once
-// (crt_wide_build_gpu_async).  crt_wide_build_gpu runs the same launches and
-// reads the node count and status back once.
+// level passes (one launch each), the level sizes live on the device, and a
+// launch past the tree's depth returns at once (crt_wide_build_gpu_async).
+// crt_wide_build_gpu runs the same launches and reads the node count and status
+// back once.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,34 +36,31 @@ namespace wg {
 
 constexpr int kBlock = 256;
 
-// Exclusive prefix of v over the workgroup (kBlock threads) and the total.
-__device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t* wave_sums, uint32_t& total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t incl = v;
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += o;
-    }
-    if (lane == 63) wave_sums[wave] = incl;
-    __syncthreads();
-    uint32_t before = 0;
-    total = 0;
-    for (int w = 0; w < kBlock / 64; ++w) {
-        before += w < wave ? wave_sums[w] : 0u;
-        total += wave_sums[w];
-    }
-    return before + incl - v;
-}
-
-// ---- the asynchronous collapse (crt_wide_build_gpu_async) ----------------
+// ---- level passes --------------------------------------------------------
 //
-// The host launches a fixed number of levels and reads nothing back, so the
+// The host launches a fixed number of passes and reads nothing back, so the
 // whole collapse can be captured into a graph.  Level state lives on the
 // device, two int64 per level l: lvl[2l] is the number of wide nodes numbered
 // through level l (the first index of level l + 1) and lvl[2l + 1] the size of
-// level l.  Each level launches kGrid-or-fewer workgroups over contiguous
-// chunks of the level (so the breadth-first numbering stays the host loop's),
-// and a level of size 0 returns at once.
+// level l.  An expanded level leaves its inner children's stack entries in
+// kids (W slots a node, -1 for the others) and, per kParents nodes, their
+// number (sums).
+//
+// Pass k takes level p = first[k], numbers its children and expands them, a
+// workgroup per kParents nodes: the children before it are the sums before its
+// own, so a workgroup adds those up (at most a few thousand words) instead of
+// waiting for another launch, and the numbering stays the host's.  Its
+// children, at most kBlock, are packed in LDS and expanded by one thread each.
+// A level of at most kParents nodes is one workgroup's work: it then goes on
+// to the next level by itself while that is as small, so the narrow levels at
+// the root and at the end of the tree share a launch.
+//
+// Bound: the chain of an expansion's dependent loads (its entry, then twice
+// the opened child's and its children's), 5 to 12 us a level, and on the wide
+// levels the gathered entries.  With two launches a level (expand, then assign
+// numbers) and the children in scratch memory, the levels of 2.56M triangles
+// took 703 us and those of 11,520 took 223; now 360 and 105 (width 4, 32
+// passes launched, of which 9 and 25 past the end at 2 us each).
 
 // Bit of *err: the tree has more levels than were launched.
 constexpr unsigned kErrDepth = 8u;
@@ -71,138 +68,204 @@ static_assert(kErrLink == CRT_WIDE_GPU_BAD_LINK && kErrCap == CRT_WIDE_GPU_NOT_T
                   kErrVertex == CRT_WIDE_GPU_BAD_VERTEX && kErrDepth == CRT_WIDE_GPU_TOO_DEEP &&
                   kErrLeaf == CRT_WIDE_GPU_BAD_LEAF,
               "status bits are the header's");
-constexpr int kGridMax = 2048;
+// As many workgroups as the chip holds: a launch past the tree's depth costs
+// 2 us with these, 4.6 us with 4,096.
+constexpr int kGridMax = 1024;
 
-// Exclusive prefix of v over the workgroup and the total, then a barrier, so
-// that the call can repeat in a loop.
-__device__ __forceinline__ uint32_t block_excl_loop(uint32_t v, uint32_t* wave_sums, uint32_t& total) {
-    const uint32_t r = block_excl(v, wave_sums, total);
+template <int W>
+constexpr int kParents = kBlock / W;
+
+// Level state and lists in the workspace.  The kids of even levels fill their
+// array from the front and those of odd levels from the back: two levels in a
+// row hold at most `cap` nodes together.  sums rotates over three arrays: the
+// one a pass reads, the one it adds to and the one it clears for the next.
+struct Lists {
+    int64_t* lvl;
+    int32_t* first;
+    int32_t* kids;
+    uint32_t* sums;
+    int64_t sum_stride;
+    int64_t cap;
+    unsigned* err;
+
+    template <int W>
+    __device__ __forceinline__ int32_t* kids_of(int32_t level, int64_t item) const {
+        return kids + (level & 1 ? cap - 1 - item : item) * W;
+    }
+    __device__ __forceinline__ uint32_t* sums_of(int32_t level) const { return sums + (level % 3) * sum_stride; }
+};
+
+// Sums of a and b over the workgroup (kBlock threads); every thread gets them.
+__device__ __forceinline__ void block_sum2(uint64_t& a, uint64_t& b, uint64_t (*sh)[kBlock / 64]) {
+    for (int d = 32; d > 0; d >>= 1) {
+        a += __shfl_xor(a, d, 64);
+        b += __shfl_xor(b, d, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = a;
+        sh[1][threadIdx.x >> 6] = b;
+    }
     __syncthreads();
-    return r;
+    a = b = 0;
+    for (int w = 0; w < kBlock / 64; ++w) {
+        a += sh[0][w];
+        b += sh[1][w];
+    }
+    __syncthreads();
 }
 
-// Sum over the workgroup (kBlock threads); every thread gets it.
-__device__ __forceinline__ uint64_t block_sum64(uint64_t v, uint64_t* wave_sums) {
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    if ((threadIdx.x & 63) == 0) wave_sums[threadIdx.x >> 6] = v;
+template <int W>
+struct LevelLds {
+    uint64_t sums[2][kBlock / 64];
+    uint32_t wave_count[kBlock / 64];
+    int32_t list[kBlock];
+    uint32_t children[W + 1];   // per kParents items of the next level that this workgroup's touch
+};
+
+// Nodes [chunk * kParents, ...) of level p (np nodes, the last numbered
+// next_base - 1): numbers their inner children next_base + before, ... and
+// expands them.  Adds the children's own numbers of inner children to level
+// p + 1's sums, with an atomic unless the workgroup has the level to itself.
+template <int W>
+__device__ __forceinline__ void expand_chunk(const crt_stack_node* __restrict__ nodes, int64_t node_count,
+                                             int64_t ntris, const Lists& L, int32_t p, int64_t np, int64_t next_base,
+                                             int64_t chunk, int64_t before, bool alone,
+                                             crt_wide_group* __restrict__ groups, LevelLds<W>& lds) {
+    const int tid = int(threadIdx.x), wave = tid >> 6;
+    const int64_t parent = chunk * kParents<W> + tid / W;
+    const int s = tid % W;
+    const int32_t entry = parent < np ? L.kids_of<W>(p, parent)[s] : -1;
+    const uint64_t ballot = __ballot(entry >= 0);
+    const uint32_t below =
+        __builtin_amdgcn_mbcnt_hi(uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u));
+    if ((tid & 63) == 0) lds.wave_count[wave] = uint32_t(__popcll(ballot));
+    if (tid <= W) lds.children[tid] = 0u;
     __syncthreads();
-    uint64_t t = 0;
-    for (int w = 0; w < kBlock / 64; ++w) t += wave_sums[w];
+    uint32_t rank = below, count = 0u;
+    for (int w = 0; w < kBlock / 64; ++w) {
+        rank += w < wave ? lds.wave_count[w] : 0u;
+        count += lds.wave_count[w];
+    }
+    if (entry >= 0) {
+        assign_slot<W>(next_base - np + parent, s, next_base + before + rank, groups);
+        lds.list[rank] = entry;
+    }
     __syncthreads();
-    return t;
+    const int64_t seg0 = before / kParents<W>;
+    if (tid < int(count)) {
+        const int64_t item = before + tid;
+        const uint32_t m = expand_one<W>(nodes, node_count, ntris, lds.list[tid], next_base + item, groups,
+                                         L.kids_of<W>(p + 1, item), L.err);
+        if (m) atomicAdd(&lds.children[item / kParents<W> - seg0], m);
+    }
+    __syncthreads();
+    if (tid <= W && count > 0u && seg0 + tid <= (before + count - 1) / kParents<W>) {
+        uint32_t* out = L.sums_of(p + 1) + seg0 + tid;
+        if (alone)
+            *out = lds.children[tid];
+        else if (lds.children[tid])
+            atomicAdd(out, lds.children[tid]);
+    }
 }
 
-// Items [begin, end) of a level of nf wide nodes for this workgroup of a grid
-// of `grid`; chunks are whole multiples of kBlock.
-__device__ __forceinline__ void chunk_of(int64_t nf, int32_t grid, int64_t& begin, int64_t& end) {
-    const int64_t pieces = (nf + kBlock - 1) / kBlock;
-    const int64_t per = (pieces + grid - 1) / grid * kBlock;
-    begin = int64_t(blockIdx.x) * per;
-    end = min(nf, begin + per);
+// Clears the sums that level p + 2 will need, when level p + 1 has `count` nodes.
+template <int W>
+__device__ __forceinline__ void clear_sums(const Lists& L, int32_t p, int64_t count, int64_t first, int64_t stride) {
+    const int64_t need = (count * W + kParents<W> - 1) / kParents<W>;
+    uint32_t* out = L.sums_of(p + 2);
+    for (int64_t k = first; k < need && k < L.sum_stride; k += stride) out[k] = 0u;
 }
 
 // Level 0 and the error word.  A root entry that holds two adjacent
 // 1-triangle leaves is one 2-triangle leaf under a root of one slot
 // (crt_wide_build's rule): this kernel writes that root, and level 0 is then
-// empty.  Otherwise level 0 is the root entry.
+// empty.  Otherwise level 0 is the root entry, expanded here.
 template <int W>
-__global__ void __launch_bounds__(64) root_async(const crt_stack_node* __restrict__ nodes, int64_t ntris,
-                                                 int32_t* __restrict__ entry, int32_t* __restrict__ wide,
-                                                 int64_t* __restrict__ lvl, crt_wide_group* __restrict__ groups,
-                                                 unsigned* __restrict__ err) {
+__global__ void __launch_bounds__(64) root_async(const crt_stack_node* __restrict__ nodes, int64_t node_count,
+                                                 int64_t ntris, Lists L, crt_wide_group* __restrict__ groups) {
     if (threadIdx.x != 0) return;
-    *err = 0u;
-    entry[0] = 0;
-    wide[0] = 0;
+    *L.err = 0u;
     Kid k;
     const bool one = root_one_slot(nodes[0], k);
     if (one) {
         const bool ok = leaf_ok(k.start, k.count, ntris);
-        if (!ok) *err = kErrLeaf;   // finish_async leaves the root empty
+        if (!ok) *L.err = kErrLeaf;   // finish_async leaves the root empty
         write_one_slot_root<W>(groups, k, ok);
+    } else {
+        L.sums_of(0)[0] = expand_one<W>(nodes, node_count, ntris, 0, 0, groups, L.kids_of<W>(0, 0), L.err);
+        L.sums_of(1)[0] = 0u;   // level 1 has at most W nodes, within one sum
     }
-    lvl[0] = 1;
-    lvl[1] = one ? 0 : 1;
+    L.first[0] = 0;
+    L.lvl[0] = 1;
+    L.lvl[1] = one ? 0 : 1;
 }
 
-// expand over the chunks of level `level`; totals[block] for every block of
-// the grid when the level is not empty.
+// Pass k of `levels` - 1.  A tree whose next level would pass cap stops there (kErrCap).
 template <int W>
-__global__ void __launch_bounds__(kBlock) expand_async(const crt_stack_node* __restrict__ nodes, int64_t node_count,
-                                                       int64_t ntris, const int64_t* __restrict__ lvl, int32_t level, int32_t grid,
-                                                       const int32_t* __restrict__ entries,
-                                                       const int32_t* __restrict__ wides,
-                                                       crt_wide_group* __restrict__ groups,
-                                                       int32_t* __restrict__ kids_out, uint32_t* __restrict__ counts,
-                                                       uint32_t* __restrict__ totals, unsigned* __restrict__ err) {
-    __shared__ uint32_t wave_sums[kBlock / 64];
-    const int64_t nf = lvl[2 * level + 1];
-    if (nf == 0) return;
-    int64_t begin, end;
-    chunk_of(nf, grid, begin, end);
-    uint32_t run = 0;
-    for (int64_t base = begin; base < end; base += kBlock) {
-        const int64_t item = base + threadIdx.x;
-        uint32_t m = 0;
-        if (item < end) {
-            m = expand_one<W>(nodes, node_count, ntris, entries[item], wides[item], groups, kids_out + item * W,
-                              err);
-            counts[item] = m;
-        }
-        uint32_t total;
-        (void)block_excl_loop(m, wave_sums, total);
-        run += total;
-    }
-    if (threadIdx.x == 0) totals[blockIdx.x] = run;
-}
-
-// assign over the same chunks; block 0 also writes level + 1's state.  A tree
-// whose next level would pass cap stops there (kErrCap).
-template <int W>
-__global__ void __launch_bounds__(kBlock) assign_async(int64_t* __restrict__ lvl, int32_t level, int32_t grid,
-                                                       int64_t cap, const int32_t* __restrict__ wides,
-                                                       const int32_t* __restrict__ kids,
-                                                       const uint32_t* __restrict__ counts,
-                                                       const uint32_t* __restrict__ totals,
-                                                       crt_wide_group* __restrict__ groups,
-                                                       int32_t* __restrict__ next_entries,
-                                                       int32_t* __restrict__ next_wides, unsigned* __restrict__ err) {
-    __shared__ uint32_t wave_sums[kBlock / 64];
-    __shared__ uint64_t sums[kBlock / 64];
-    const int64_t nf = lvl[2 * level + 1], next_base = lvl[2 * level];
-    if (nf == 0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            lvl[2 * level + 2] = next_base;
-            lvl[2 * level + 3] = 0;
-        }
+__global__ void __launch_bounds__(kBlock) level_async(const crt_stack_node* __restrict__ nodes, int64_t node_count,
+                                                      int64_t ntris, Lists L, int32_t k, int32_t levels,
+                                                      crt_wide_group* __restrict__ groups) {
+    __shared__ LevelLds<W> lds;
+    int32_t p = L.first[k];
+    int64_t np = L.lvl[2 * p + 1];
+    if (np == 0 || p >= levels - 1) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) L.first[k + 1] = p;
         return;
     }
+    int64_t next_base = L.lvl[2 * p];
+    if (np <= kParents<W>) {
+        if (blockIdx.x != 0) return;
+        do {
+            __syncthreads();   // the last level's lists and sums are written
+            const int64_t all = L.sums_of(p)[0];
+            const bool over = next_base + all > L.cap;
+            const int64_t size = over ? 0 : all;
+            clear_sums<W>(L, p, size, threadIdx.x, kBlock);
+            if (size > 0)
+                expand_chunk<W>(nodes, node_count, ntris, L, p, np, next_base, 0, 0, true, groups, lds);
+            if (threadIdx.x == 0) {
+                if (over) atomicOr(L.err, kErrCap);
+                L.lvl[2 * p + 2] = next_base + size;
+                L.lvl[2 * p + 3] = size;
+            }
+            next_base += size;
+            np = size;
+            ++p;
+        } while (np > 0 && np <= kParents<W> && p < levels - 1);
+        if (threadIdx.x == 0) L.first[k + 1] = p;
+        return;
+    }
+    const int64_t chunks = (np + kParents<W> - 1) / kParents<W>;
+    const uint32_t* sums = L.sums_of(p);
+    if (blockIdx.x >= chunks) return;
     uint64_t before = 0, all = 0;
-    for (int32_t j = int32_t(threadIdx.x); j < grid; j += kBlock) {
-        const uint64_t v = totals[j];
+#pragma unroll 8
+    for (int64_t j = threadIdx.x; j < chunks; j += kBlock) {
+        const uint32_t v = sums[j];
         all += v;
-        before += j < int32_t(blockIdx.x) ? v : 0u;
+        before += j < blockIdx.x ? v : 0u;
     }
-    before = block_sum64(before, sums);
-    all = block_sum64(all, sums);
+    block_sum2(before, all, lds.sums);
+    const bool over = next_base + int64_t(all) > L.cap;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const bool over = int64_t(next_base + all) > cap;
-        if (over) atomicOr(err, kErrCap);
-        lvl[2 * level + 2] = over ? next_base : next_base + int64_t(all);
-        lvl[2 * level + 3] = over ? 0 : int64_t(all);
+        if (over) atomicOr(L.err, kErrCap);
+        L.lvl[2 * p + 2] = next_base + (over ? 0 : int64_t(all));
+        L.lvl[2 * p + 3] = over ? 0 : int64_t(all);
+        L.first[k + 1] = p + 1;
     }
-    int64_t begin, end;
-    chunk_of(nf, grid, begin, end);
-    int64_t run = int64_t(before);
-    for (int64_t base = begin; base < end; base += kBlock) {
-        const int64_t item = base + threadIdx.x;
-        const uint32_t m = item < end ? counts[item] : 0u;
-        uint32_t total;
-        const uint32_t local = block_excl_loop(m, wave_sums, total);
-        if (item < end)
-            (void)assign_one<W>(wides[item], kids + item * W, run + local, next_base, cap, groups, next_entries,
-                                next_wides, err);
-        run += total;
+    if (over) return;
+    // the workgroups that run here, min(grid, chunks) of them, clear together
+    const int64_t groups_run = chunks < int64_t(gridDim.x) ? chunks : int64_t(gridDim.x);
+    clear_sums<W>(L, p, int64_t(all), int64_t(blockIdx.x) * kBlock + threadIdx.x, groups_run * kBlock);
+    for (int64_t c = blockIdx.x;;) {
+        expand_chunk<W>(nodes, node_count, ntris, L, p, np, next_base, c, int64_t(before), false, groups, lds);
+        const int64_t next = c + gridDim.x;
+        if (next >= chunks) break;
+        uint64_t more = 0, unused = 0;
+        for (int64_t j = c + threadIdx.x; j < next; j += kBlock) more += sums[j];
+        block_sum2(more, unused, lds.sums);   // its barriers also end the use of the lists
+        before += more;
+        c = next;
     }
 }
 
@@ -213,27 +276,29 @@ __global__ void __launch_bounds__(kBlock) assign_async(int64_t* __restrict__ lvl
 // slot empty, so a trace that runs after it, in the same graph say, ends at
 // the root with no hit.
 template <int W>
-__global__ void __launch_bounds__(64) finish_async(const int64_t* __restrict__ lvl, int32_t levels,
-                                                   const unsigned* __restrict__ err, int64_t* __restrict__ wide_nodes,
-                                                   uint32_t* __restrict__ status, crt_wide_group* __restrict__ groups) {
-    const uint32_t st = *err | (lvl[2 * levels + 1] > 0 ? kErrDepth : 0u);
+__global__ void __launch_bounds__(kBlock) finish_async(Lists L, int32_t levels, int64_t* __restrict__ wide_nodes,
+                                                       uint32_t* __restrict__ status,
+                                                       crt_wide_group* __restrict__ groups) {
+    __shared__ uint64_t sh[2][kBlock / 64];
+    const int32_t p = L.first[levels - 1];   // the first empty level, or the last one expanded
+    const int64_t np = L.lvl[2 * p + 1];
+    uint64_t all = 0, unused = 0;            // children of the last level, which nothing numbered
+    for (int64_t j = threadIdx.x; j < (np + kParents<W> - 1) / kParents<W>; j += kBlock) all += L.sums_of(p)[j];
+    block_sum2(all, unused, sh);
+    const int64_t count = L.lvl[2 * p];
+    const bool over = count + int64_t(all) > L.cap;
+    const uint32_t st = *L.err | (all == 0 ? 0u : over ? kErrCap : kErrDepth);
     if (st != 0u) {
-        // 64 lanes: W / 4 groups of 8 fields of 4 words (32 words each)
-        for (int k = int(threadIdx.x); k < (W / 4) * 32; k += 64) {
+        // W / 4 groups of 8 fields of 4 words (32 words each)
+        for (int k = int(threadIdx.x); k < (W / 4) * 32; k += kBlock) {
             int32_t* g = reinterpret_cast<int32_t*>(groups + k / 32);
             const int word = k % 32;
             g[word] = word >= 28 ? -1 : 0;   // count[4] is the last field
         }
     }
     if (threadIdx.x != 0) return;
-    int32_t used = levels;
-    for (int32_t l = 0; l < levels; ++l)
-        if (lvl[2 * l + 1] == 0) {
-            used = l;
-            break;
-        }
-    wide_nodes[0] = lvl[2 * levels];
-    wide_nodes[1] = used;
+    wide_nodes[0] = count + (over ? 0 : int64_t(all));
+    wide_nodes[1] = np == 0 ? p : levels;
     *status = st;
 }
 
@@ -250,23 +315,20 @@ __global__ void __launch_bounds__(kBlock) records(const crt_triangle* __restrict
             t.packed[k] = 0;
         }
     }
-    crt_tri_record r;
     const float4 a = *reinterpret_cast<const float4*>(verts[t.packed[0]].position);
     const float4 b = *reinterpret_cast<const float4*>(verts[t.packed[1]].position);
     const float4 c = *reinterpret_cast<const float4*>(verts[t.packed[2]].position);
-    r.v0[0] = a.x, r.v0[1] = a.y, r.v0[2] = a.z;
-    r.v1[0] = b.x, r.v1[1] = b.y, r.v1[2] = b.z;
-    r.v2[0] = c.x, r.v2[1] = c.y, r.v2[2] = c.z;
-    r.tri = int32_t(i);
-    r.mesh = t.packed[3];
-    r.pad = 0;
-    out[i] = r;
+    float4* o = reinterpret_cast<float4*>(out + i);
+    o[0] = make_float4(a.x, a.y, a.z, __int_as_float(int32_t(i)));
+    o[1] = make_float4(b.x, b.y, b.z, __int_as_float(t.packed[3]));
+    o[2] = make_float4(c.x, c.y, c.z, __int_as_float(0));
 }
 
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct Layout {
-    size_t entries[2], wides[2], kids, counts, totals, err, lvl, out, bytes;
+    size_t kids, sums, err, lvl, first, out, bytes;
+    int64_t sum_stride;
 };
 
 // Levels hold at most `cap` wide nodes (a valid tree has fewer wide nodes
@@ -280,17 +342,18 @@ inline Layout layout(int64_t cap, int32_t width, int32_t levels) {
         off = align256(off + bytes);
         return at;
     };
-    L.entries[0] = take(n * 4);
-    L.entries[1] = take(n * 4);
-    L.wides[0] = take(n * 4);
-    L.wides[1] = take(n * 4);
+    const int64_t parents = kBlock / width;
+    L.sum_stride = (cap + parents - 1) / parents + 1;
     L.kids = take(n * size_t(width) * 4);
-    L.counts = take(n * 4);
-    L.totals = take(nb * 4);
+    L.sums = take(size_t(L.sum_stride) * 3 * 4);
     L.err = take(4);
     L.lvl = take(size_t(2) * size_t(levels + 1) * 8);
+    L.first = take(size_t(levels) * 4);
     L.out = take(3 * 8);   // crt_wide_build_gpu's node count, level count and status
-    L.bytes = off;
+    // no less than callers have been told to reserve: the width's child slots
+    // and five more words a triangle
+    L.bytes = std::max(off, align256(n * (size_t(width) + 5) * 4) + align256(nb * 4) +
+                                align256(size_t(levels + 1) * 16));
     return L;
 }
 
@@ -299,25 +362,18 @@ void collapse_async(const crt_stack_node* nodes, int64_t node_count, const crt_t
                     const crt_vertex* verts, int64_t nverts, int64_t cap, int32_t levels, crt_wide_group* groups,
                     crt_tri_record* recs, int64_t* wide_nodes, uint32_t* status, char* ws, const Layout& L,
                     hipStream_t st) {
-    int32_t* entries[2] = {reinterpret_cast<int32_t*>(ws + L.entries[0]), reinterpret_cast<int32_t*>(ws + L.entries[1])};
-    int32_t* wides[2] = {reinterpret_cast<int32_t*>(ws + L.wides[0]), reinterpret_cast<int32_t*>(ws + L.wides[1])};
-    auto* kids = reinterpret_cast<int32_t*>(ws + L.kids);
-    auto* counts = reinterpret_cast<uint32_t*>(ws + L.counts);
-    auto* totals = reinterpret_cast<uint32_t*>(ws + L.totals);
-    auto* lvl = reinterpret_cast<int64_t*>(ws + L.lvl);
-    auto* err = reinterpret_cast<unsigned*>(ws + L.err);
-    const int32_t grid = int32_t(std::min<int64_t>(kGridMax, (cap + kBlock - 1) / kBlock));
-    hipLaunchKernelGGL(root_async<W>, dim3(1), dim3(64), 0, st, nodes, cap, entries[0], wides[0], lvl, groups, err);
+    const Lists lists{reinterpret_cast<int64_t*>(ws + L.lvl),   reinterpret_cast<int32_t*>(ws + L.first),
+                      reinterpret_cast<int32_t*>(ws + L.kids),  reinterpret_cast<uint32_t*>(ws + L.sums),
+                      L.sum_stride,                              cap,
+                      reinterpret_cast<unsigned*>(ws + L.err)};
+    const int32_t grid = int32_t(std::min<int64_t>(kGridMax, (cap + kParents<W> - 1) / kParents<W>));
+    hipLaunchKernelGGL(root_async<W>, dim3(1), dim3(64), 0, st, nodes, node_count, cap, lists, groups);
     hipLaunchKernelGGL(records, dim3(unsigned((cap + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, tris, verts, nverts,
-                       cap, recs, err);
-    for (int32_t l = 0; l < levels; ++l) {
-        const int cur = l & 1;
-        hipLaunchKernelGGL(expand_async<W>, dim3(grid), dim3(kBlock), 0, st, nodes, node_count, cap, lvl, l, grid,
-                           entries[cur], wides[cur], groups, kids, counts, totals, err);
-        hipLaunchKernelGGL(assign_async<W>, dim3(grid), dim3(kBlock), 0, st, lvl, l, grid, cap, wides[cur], kids, counts,
-                           totals, groups, entries[1 - cur], wides[1 - cur], err);
-    }
-    hipLaunchKernelGGL(finish_async<W>, dim3(1), dim3(64), 0, st, lvl, levels, err, wide_nodes, status, groups);
+                       cap, recs, lists.err);
+    for (int32_t k = 0; k < levels - 1; ++k)
+        hipLaunchKernelGGL(level_async<W>, dim3(unsigned(grid)), dim3(kBlock), 0, st, nodes, node_count, cap, lists, k,
+                           levels, groups);
+    hipLaunchKernelGGL(finish_async<W>, dim3(1), dim3(kBlock), 0, st, lists, levels, wide_nodes, status, groups);
 }
 
 }  // namespace wg
