@@ -2,6 +2,7 @@
 // and the RayIntersector<T> context (Source/Core/BVH/Intersector.h:60-351).
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -321,6 +322,14 @@ struct crt_context {
     int64_t nodes_buffered = 0;               // m_NodeCountBuffered
     int64_t entities_buffered = 0;            // m_EntityPushed
     bool data_buffered = false;
+    // Derived from the buffered data for crt_intersect and crt_intersect_primary:
+    // one record per triangle, and the child pairs of a stackless tree.  Null
+    // where the data allow none; those calls then walk the buffered data.
+    void* d_records = nullptr;
+    void* d_pairs = nullptr;
+    std::vector<std::pair<int32_t, int32_t>> appended;   // (first node, nodes) of the host copies' objects
+    std::vector<std::pair<int32_t, int32_t>> paired;     // the same of d_pairs
+    bool pairs_fit = false;                   // every buffered entity walks an object of d_pairs
     // Wide layout derived from the buffered data and entities.
     void* d_wide_groups = nullptr;
     void* d_wide_records = nullptr;
@@ -338,7 +347,22 @@ struct crt_context {
         if (d_verts) (void)hipFree(d_verts);
         if (d_entities) (void)hipFree(d_entities);
         d_nodes = d_tris = d_verts = d_entities = nullptr;
+        free_derived();
         free_wide();
+    }
+    void free_derived() {
+        if (d_records) (void)hipFree(d_records);
+        if (d_pairs) (void)hipFree(d_pairs);
+        d_records = d_pairs = nullptr;
+        paired.clear();
+        pairs_fit = false;
+    }
+    // An entity may name an object of data that is no longer buffered.
+    void match_entities() {
+        pairs_fit = d_pairs != nullptr;
+        for (const crt_entity& e : entities)
+            pairs_fit = pairs_fit && std::binary_search(paired.begin(), paired.end(),   // in order of the nodes
+                                                        std::make_pair(e.node_offset, e.node_count));
     }
     void free_wide() {
         if (d_wide_groups) (void)hipFree(d_wide_groups);
@@ -428,6 +452,7 @@ int append_object(crt_context* ctx, int32_t object_id, const void* nodes, int64_
     od.triangle_offset = int64_t(ctx->triangles.size());
     od.vertices_offset = int64_t(ctx->vertices.size());
     od.node_count = node_count;
+    ctx->appended.emplace_back(int32_t(od.node_offset), int32_t(node_count));
     if (ctx->format == CRT_FORMAT_STACKLESS) {
         const auto* n = static_cast<const crt_stackless_node*>(nodes);
         ctx->stackless.insert(ctx->stackless.end(), n, n + node_count);
@@ -448,6 +473,52 @@ int append_object(crt_context* ctx, int32_t object_id, const void* nodes, int64_
     ctx->objects[object_id] = od;
     ctx->data_buffered = false;
     return CRT_OK;
+}
+
+// The records and pairs of the data just buffered.  They only speed a walk up,
+// so data that allow none (or too little memory) leave them out.
+void derive_unguarded(crt_context* ctx) {
+    const int64_t ntris = int64_t(ctx->triangles.size());
+    const uint32_t nverts = uint32_t(ctx->vertices.size());
+    if (ntris == 0) return;
+    for (const crt_triangle& t : ctx->triangles)
+        if (uint32_t(t.packed[0]) >= nverts || uint32_t(t.packed[1]) >= nverts || uint32_t(t.packed[2]) >= nverts)
+            return;
+    void* records = nullptr;
+    bool ok = hipMalloc(&records, size_t(ntris) * sizeof(crt_tri_record)) == hipSuccess;
+    if (ok) {
+        ctx->d_records = records;
+        ok = crt::launch_gather_records(static_cast<const crt_triangle*>(ctx->d_tris),
+                                        static_cast<const crt_vertex*>(ctx->d_verts), ntris,
+                                        static_cast<crt_tri_record*>(records), nullptr) == hipSuccess &&
+             hipStreamSynchronize(nullptr) == hipSuccess;
+    }
+    if (ok && ctx->format == CRT_FORMAT_STACKLESS) {
+        std::vector<crt_stack_node> pairs((ctx->stackless.size() + 1) / 2 + 1);
+        for (const auto& o : ctx->appended)
+            if (crt::build_pairs(ctx->stackless.data(), o.first, o.second, ntris, pairs.data()))
+                ctx->paired.push_back(o);
+        void* d = nullptr;
+        const size_t bytes = pairs.size() * sizeof(crt_stack_node);
+        ok = hipMalloc(&d, bytes) == hipSuccess;
+        if (ok) {
+            ctx->d_pairs = d;
+            ok = hipMemcpy(d, pairs.data(), bytes, hipMemcpyHostToDevice) == hipSuccess;
+        }
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        ctx->free_derived();
+    }
+}
+
+void derive(crt_context* ctx) {
+    ctx->free_derived();
+    try {
+        derive_unguarded(ctx);
+    } catch (const std::bad_alloc&) {
+        ctx->free_derived();
+    }
 }
 
 }  // namespace
@@ -731,6 +802,7 @@ int crt_buffer_entities(crt_context* ctx) {
     ctx->entities_buffered = int64_t(ctx->pending.size());
     ctx->entities = ctx->pending;
     ctx->pending.clear();
+    ctx->match_entities();
     ctx->free_wide();
     return CRT_OK;
 }
@@ -743,8 +815,11 @@ int crt_buffer_data(crt_context* ctx, int clear_cpu_data) {
     if (rc) return rc;
     ctx->nodes_buffered = ctx->node_count();
     ctx->data_buffered = true;
+    derive(ctx);
+    ctx->match_entities();
     ctx->free_wide();
     if (clear_cpu_data) {
+        ctx->appended.clear();
         ctx->stackless.clear();
         ctx->stack.clear();
         ctx->vertices.clear();
@@ -844,11 +919,24 @@ int crt_context_wide_scene(const crt_context* ctx, crt_scene_view* out) {
     return CRT_OK;
 }
 
+static crt::PairScene pair_scene(const crt_context* ctx) {
+    return crt::PairScene{int32_t(ctx->entities_buffered), static_cast<const crt_entity*>(ctx->d_entities),
+                          static_cast<const float4*>(ctx->d_nodes), static_cast<const float4*>(ctx->d_pairs),
+                          static_cast<const float4*>(ctx->d_records)};
+}
+
 int crt_intersect(crt_context* ctx, int query, uint32_t flags, const crt_ray* rays, crt_hit* hits, int64_t nrays,
                   void* stream) {
     crt_scene_view s;
     int rc = crt_context_scene(ctx, &s);
     if (rc) return rc;
+    if (ctx->pairs_fit && (query == CRT_QUERY_CLOSEST || query == CRT_QUERY_ANY) && nrays > 0 &&
+        nrays < (int64_t(1) << 31) && rays && hits) {
+        CRT_HIP(crt::launch_pair_grid(pair_scene(ctx), query, rays, hits, nrays, flags, crt::kMaxIterations,
+                                      static_cast<hipStream_t>(stream)),
+                "crt_intersect: kernel launch");
+        return CRT_OK;
+    }
     return crt::trace(&s, query, flags, rays, hits, nrays, nullptr, stream);
 }
 
@@ -863,6 +951,12 @@ int crt_intersect_primary(crt_context* ctx, crt_ray* rays, crt_hit* hits, int wi
     std::memcpy(cam.inv_view, inv_view, sizeof(cam.inv_view));
     std::memcpy(cam.inv_proj, inv_proj, sizeof(cam.inv_proj));
     cam.tmax = 1000000.0f;  // IntersectScene's TMax (TraverseBVHStackless.glsl:309)
+    if (ctx->pairs_fit && int64_t(width) * height < (int64_t(1) << 31)) {
+        CRT_HIP(crt::launch_pair_primary(pair_scene(ctx), cam, rays, hits, width, height, flags, crt::kMaxIterations,
+                                         static_cast<hipStream_t>(stream)),
+                "crt_intersect_primary: kernel launch");
+        return CRT_OK;
+    }
     const crt::SceneArgs a = crt::scene_args(s);
     CRT_HIP(crt::launch_primary(a, cam, rays, hits, width, height, flags, crt::kMaxIterations, 256,
                                 static_cast<hipStream_t>(stream)),

@@ -26,6 +26,7 @@
 #include "crt_internal.h"
 #include "trace_launch.h"
 #include "device_math.h"
+#include "primary_ray.h"
 #include "thread_walk.h"
 
 #pragma clang fp contract(off)
@@ -57,25 +58,8 @@ __global__ void __launch_bounds__(1024) primary_kernel(SceneArgs s, Camera cam, 
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= int64_t(width) * height) return;
     const int32_t x = int32_t(i % width), y = int32_t(i / width);
-    const float u = float(x) / float(width), v = float(y) / float(height);
-    const float cx = u * 2.0f - 1.0f, cy = v * 2.0f - 1.0f;
-    const float* ip = cam.inv_proj;
-    const float ex = ip[0] * cx + ip[4] * cy + ip[8] * -1.0f + ip[12] * 1.0f;
-    const float ey = ip[1] * cx + ip[5] * cy + ip[9] * -1.0f + ip[13] * 1.0f;
-    const f3 d = xform(cam.inv_view, mk(ex, ey, -1.0f), 0.0f);
-    const float il = 1.0f / sqrtf(dot(d, d));
-    crt_ray r;
-    r.org[0] = cam.inv_view[12];
-    r.org[1] = cam.inv_view[13];
-    r.org[2] = cam.inv_view[14];
-    r.tmax = cam.tmax;
-    r.dir[0] = d.x * il;
-    r.dir[1] = d.y * il;
-    r.dir[2] = d.z * il;
-    r.id = uint32_t(i);
-    float4* rp = reinterpret_cast<float4*>(rays + i);
-    rp[0] = make_float4(r.org[0], r.org[1], r.org[2], r.tmax);
-    rp[1] = make_float4(r.dir[0], r.dir[1], r.dir[2], __uint_as_float(r.id));
+    const crt_ray r = primary_ray(cam, width, height, x, y, uint32_t(i));
+    store_ray(rays + i, r);
     trace_one<FORMAT, false, LDS_DEPTH>(s, r, flags, max_iter, hits + i, nullptr, lds_stack + threadIdx.x,
                                         int32_t(blockDim.x));
 }

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime_api.h>
+#include <hip/hip_vector_types.h>
 
 #include <cstdint>
 
@@ -33,6 +34,34 @@ struct Camera {
     float inv_proj[16];
     float tmax;
 };
+
+// A context's stackless scene with the derived arrays of pair_layout.cpp: the
+// child pairs of every inner node (an object's first pair is that of its root,
+// at pair_base of its first node) and one record per triangle.
+struct PairScene {
+    int32_t entity_count;
+    const crt_entity* entities;
+    const float4* nodes;     // crt_stackless_node[]
+    const float4* pairs;     // crt_stack_node[]; min.w holds the child (pair_walk.h), max.w nothing
+    const float4* records;   // crt_tri_record[] by triangle index
+};
+
+// Objects are full binary trees one behind the other, so (start + 1) / 2
+// leaves every object room for its (nodes - 1) / 2 pairs.
+__host__ __device__ constexpr int32_t pair_base(int32_t start) { return (start + 1) >> 1; }
+constexpr int32_t kPairStack = 64;   // levels below the root that a pair walk can hold
+
+// The child pairs of one object's nodes (pair_layout.cpp) into `pairs` from
+// pair_base(start) on; false when the nodes are no pre-order tree of at most
+// kPairStack levels below the root with leaves inside [0, ntris).
+bool build_pairs(const crt_stackless_node* nodes, int64_t start, int64_t count, int64_t ntris, crt_stack_node* pairs);
+
+hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* verts, int64_t n, crt_tri_record* out,
+                                 hipStream_t stream);
+hipError_t launch_pair_grid(const PairScene& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
+                            uint32_t flags, int32_t max_iter, hipStream_t stream);
+hipError_t launch_pair_primary(const PairScene& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,
+                               int height, uint32_t flags, int32_t max_iter, hipStream_t stream);
 
 constexpr int32_t kMaxIterations = 1024;  // TraverseBVHStackless.glsl:184
 
