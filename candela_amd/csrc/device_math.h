@@ -103,5 +103,11 @@ __device__ __forceinline__ uint32_t pack_status(uint32_t visits, uint32_t flags)
     return (visits > CRT_STATUS_VISITS_MASK ? CRT_STATUS_VISITS_MASK : visits) | flags;
 }
 
+// Four loaded registers that are used from here on: without it the compiler
+// moves the loads of a value that only one side of a later branch needs behind
+// the branch, where they cost a second round trip.
+__device__ __forceinline__ void pin(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+__device__ __forceinline__ void pin(int4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+
 }  // namespace dm
 }  // namespace crt

@@ -89,11 +89,6 @@ struct PairStack {
     }
 };
 
-// Four loaded registers that are used from here on: without it the compiler
-// moves the loads of a value that only one side of a later branch needs behind
-// the branch, where they cost a second round trip.
-__device__ __forceinline__ void pin(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
-
 // Entry distance of a box, infinity when the ray passes it by (see the top).
 __device__ __forceinline__ float entry(float4 bmin, float4 bmax, f3 ro, f3 inv) {
     const float t0x = (bmin.x - ro.x) * inv.x, t0y = (bmin.y - ro.y) * inv.y, t0z = (bmin.z - ro.z) * inv.z;

@@ -31,8 +31,8 @@
 #include "candela_rt.h"
 #include "crt_internal.h"
 #include "device_math.h"
-#include "thread_walk.h"
 #include "trace_launch.h"
+#include "walker.h"
 
 namespace crt {
 namespace shade {
@@ -40,6 +40,19 @@ namespace shade {
 using namespace ::crt::dm;
 
 constexpr int kMaxLights = 16;
+
+// A workgroup of kWaves waves works on tiles of 64 pixels, one per lane, and
+// deals a tile's rays (one bounce, a shadow ray from p and one from q to every
+// light) to its waves one kind of ray at a time: a wave traces the same ray of
+// all 64 pixels, which neighbours share most of.  The launch fills the device
+// once, and workgroup b takes the tiles b, b + grid, ...
+// Bound: VALU issue (80% of the forward pass; the boxes' tree stays in the
+// caches).  One forward and backward pass over 1024 x 1024 pixels with 8 lights:
+// 1,661 us with a wave per tile, each with its 17 rays in turn (waves of 135 to
+// 560 us in two rounds, the chip half empty); 1,160 us as here, 1,295 when a
+// lane's leaf is tested as soon as it is reached; 805 us with gradients met in
+// LDS and one loop condition per node.  3 waves a tile take 6% more, 4 take 9%.
+constexpr int kWaves = 2, kBlock = 64 * kWaves;
 constexpr float kPi = 3.14159265359f;      // CookTorranceBRDF.glsl:7
 constexpr float kOffset = 1e-4f;           // surface offset of secondary rays
 constexpr float kTwoPi = 2.0f * 3.14159265359f;  // Sampling.glsl:3
@@ -57,6 +70,8 @@ __device__ __forceinline__ f3 add(f3 a, f3 b) { return mk(a.x + b.x, a.y + b.y, 
 __device__ __forceinline__ f3 scale(f3 a, float s) { return mk(a.x * s, a.y * s, a.z * s); }
 __device__ __forceinline__ f3 normalize(f3 a) { return scale(a, 1.0f / sqrtf(dot(a, a))); }
 
+__device__ __forceinline__ f3 load3(const float* p, int32_t i) { return mk(p[3 * i], p[3 * i + 1], p[3 * i + 2]); }
+
 __device__ __forceinline__ uint32_t pcg(uint32_t v) {
     const uint32_t state = v * 747796405u + 2891336453u;
     const uint32_t word = ((state >> ((state >> 28u) + 4u)) ^ state) * 277803737u;
@@ -72,24 +87,61 @@ __device__ __forceinline__ f3 face_normal(const SceneArgs& s, int32_t tri, f3 di
     return n;
 }
 
+constexpr int kStackLds = 16;   // stack layout: entries a lane keeps in LDS
+
 template <int FORMAT>
-__device__ __forceinline__ bool visible(const SceneArgs& s, f3 x, f3 n, f3 light, int32_t* lds, int32_t stride) {
+constexpr int stack_ints() {
+    return FORMAT == CRT_FORMAT_STACK ? kStackLds * kBlock : 1;
+}
+
+// The scene loop for one ray per lane (IntersectScene / its occlusion form,
+// TraverseBVHStackless.glsl:280-366, :558-579): the hit triangle or -1, its
+// distance in tmax.
+template <int FORMAT, bool ANY>
+__device__ __forceinline__ int32_t trace(const SceneArgs& s, f3 org, f3 dir, float& tmax, int32_t* lds) {
+    constexpr int kSpill = FORMAT == CRT_FORMAT_STACK ? sdev::spill_entries<kStackLds>() : 1;
+    int32_t spill[kSpill];
+    walker::Walker<FORMAT, kStackLds> w;
+    w.init(lds, kBlock, spill);
+    w.tmax = tmax;
+    int32_t hit = -1;
+    for (int32_t i = 0; i < s.entity_count; ++i) {
+        const crt_entity& e = s.entities[i];
+        w.ro = xform(e.inverse, org, 1.0f);
+        w.rd = xform(e.inverse, dir, 0.0f);
+        w.inv = mk(1.0f / w.rd.x, 1.0f / w.rd.y, 1.0f / w.rd.z);
+        w.begin(e.node_offset, e.node_count, s.total_nodes);
+        while (w.leaves(s)) {
+            int32_t leaf = w.leaf;
+            while (true) {
+                const int32_t first = leaf >> 4, end = first + (leaf & 0xF);
+                for (int32_t k = first; k < end; ++k) {
+                    const int4 tr = *reinterpret_cast<const int4*>(s.tris[k].packed);
+                    const float t = tri_t(w.ro, w.rd, vertex_pos(s.verts, tr.x), vertex_pos(s.verts, tr.y),
+                                          vertex_pos(s.verts, tr.z));
+                    if (t > 0.0f && t < w.tmax) {
+                        w.tmax = t;
+                        hit = k;
+                        if (ANY) break;
+                    }
+                }
+                if ((ANY && hit >= 0) || leaf == w.leaf2 || w.leaf2 < 0) break;
+                leaf = w.leaf2;
+            }
+            if (ANY && hit >= 0) break;
+        }
+        if (ANY && hit >= 0) break;
+    }
+    tmax = w.tmax;
+    return hit;
+}
+
+template <int FORMAT>
+__device__ __forceinline__ bool visible(const SceneArgs& s, f3 x, f3 n, f3 light, int32_t* lds) {
     const f3 o = add(x, scale(n, kOffset));
     const f3 d = sub(light, o);
-    const float dist = sqrtf(dot(d, d));
-    crt_ray r;
-    r.org[0] = o.x;
-    r.org[1] = o.y;
-    r.org[2] = o.z;
-    r.tmax = dist;
-    const f3 dn = scale(d, 1.0f / dist);
-    r.dir[0] = dn.x;
-    r.dir[1] = dn.y;
-    r.dir[2] = dn.z;
-    r.id = 0;
-    uint32_t tests = 0;
-    const crt_hit h = dev::scene_trace<FORMAT, true, 16>(s, r, 0u, kMaxIterations, tests, lds, stride);
-    return !(h.t > 0.0f);
+    float dist = sqrtf(dot(d, d));
+    return trace<FORMAT, true>(s, o, scale(d, 1.0f / dist), dist, lds) < 0;
 }
 
 // Cook-Torrance terms of one light at x: f_c = A * (kd * albedo_c + spec),
@@ -151,109 +203,161 @@ __device__ __forceinline__ float lambert(f3 x, f3 n, f3 light, float intensity) 
     return radiance * fminf(fmaxf(dot(n, Li), 0.0f), 1.0f);
 }
 
-__device__ __forceinline__ f3 load3(const float* p, int32_t i) { return mk(p[3 * i], p[3 * i + 1], p[3 * i + 2]); }
+
+// What the waves of a workgroup share of one tile.  Two of them take turns, so
+// that one wave can finish a tile while the others trace the next.
+struct Tile {
+    unsigned long long vis_p[kMaxLights], vis_q[kMaxLights];   // per light, a bit per pixel
+    int32_t next[2];                                           // rays claimed, per phase
+    float q[3][64], nq[3][64];
+    int32_t tri1[64];
+};
+
+// The next ray of a phase for the calling wave.
+__device__ __forceinline__ int32_t claim(int32_t* counter) {
+    int32_t k = 0;
+    if (__lane_id() == 0) k = atomicAdd(counter, 1);
+    return __builtin_amdgcn_readfirstlane(k);
+}
+
+__device__ __forceinline__ int32_t wave_id() { return __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x >> 6)); }
 
 template <int FORMAT>
-__global__ void __launch_bounds__(128) forward_kernel(SceneArgs s, const crt_ray* __restrict__ rays,
-                                                      const crt_hit* __restrict__ hits, int64_t npix, Params P,
-                                                      uint32_t seed, float* __restrict__ color,
-                                                      crt_shade_record* __restrict__ rec) {
-    __shared__ int32_t lds[16 * 128];
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= npix) return;
-    int32_t* my = lds + threadIdx.x;
-    const crt_ray r = rays[i];
-    const crt_hit h = hits[i];
-    crt_shade_record out;
-    out.pad0 = out.pad1 = 0.0f;
-    out.vis = 0;
-    out.tri1 = -1;
-    const f3 eye = mk(r.org[0], r.org[1], r.org[2]);
-    const f3 dir = mk(r.dir[0], r.dir[1], r.dir[2]);
-    out.eye[0] = eye.x;
-    out.eye[1] = eye.y;
-    out.eye[2] = eye.z;
-    if (!(h.t > 0.0f) || h.tri < 0) {
-        out.tri0 = -1;
-        for (int k = 0; k < 3; ++k) out.p[k] = out.n[k] = out.q[k] = out.nq[k] = 0.0f;
+__global__ void __launch_bounds__(kBlock) forward_kernel(SceneArgs s, const crt_ray* __restrict__ rays,
+                                                         const crt_hit* __restrict__ hits, int64_t npix, Params P,
+                                                         uint32_t seed, float* __restrict__ color,
+                                                         crt_shade_record* __restrict__ rec) {
+    __shared__ int32_t stack[stack_ints<FORMAT>()];
+    __shared__ Tile tiles[2];
+    int32_t* my = stack + (FORMAT == CRT_FORMAT_STACK ? threadIdx.x : 0);
+    if (threadIdx.x < 4) tiles[threadIdx.x >> 1].next[threadIdx.x & 1] = 0;
+    __syncthreads();
+    const uint32_t lane = __lane_id();
+    const int64_t ntiles = (npix + 63) / 64;
+    int32_t turn = 0;
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, ++turn) {
+        Tile& T = tiles[turn & 1];
+        const int64_t i = tile * 64 + lane;
+        int32_t t0 = -1;
+        f3 eye = mk(0.0f, 0.0f, 0.0f), p = eye, n = eye;
+        if (i < npix) {
+            const crt_ray r = rays[i];
+            const crt_hit h = hits[i];
+            eye = mk(r.org[0], r.org[1], r.org[2]);
+            if (h.t > 0.0f && h.tri >= 0) {
+                const f3 dir = mk(r.dir[0], r.dir[1], r.dir[2]);
+                t0 = h.tri;
+                p = add(eye, scale(dir, h.t));
+                n = face_normal(s, t0, dir);
+            }
+        }
+        const bool any = __any(t0 >= 0);
+        // the bounce, then p to every light
+        for (int32_t k = any ? claim(&T.next[0]) : P.nl + 1; k <= P.nl; k = claim(&T.next[0])) {
+            if (k == 0) {
+                f3 q = mk(0.0f, 0.0f, 0.0f), nq = q;
+                int32_t t1 = -1;
+                if (t0 >= 0) {
+                    // cosine-weighted bounce (Sampling.glsl:1-12) from per-pixel PCG uniforms
+                    const uint32_t h1 = pcg(uint32_t(i) ^ (seed * 0x9E3779B9u));
+                    const uint32_t h2 = pcg(h1);
+                    const float u1 = float(h1 >> 8) * (1.0f / 16777216.0f);
+                    const float u2 = float(h2 >> 8) * (1.0f / 16777216.0f);
+                    f3 uu = cross(n, mk(0.0f, 1.0f, 1.0f));
+                    if (dot(uu, uu) < 1e-12f) uu = cross(n, mk(1.0f, 0.0f, 0.0f));
+                    uu = normalize(uu);
+                    const f3 vv = cross(uu, n);
+                    const float ra = sqrtf(u2);
+                    const float rx = ra * cosf(kTwoPi * u1), ry = ra * sinf(kTwoPi * u1), rz = sqrtf(1.0f - u2);
+                    const f3 bd = normalize(add(add(scale(uu, rx), scale(vv, ry)), scale(n, rz)));
+                    const f3 bo = add(p, scale(n, kOffset));
+                    float t = 1000000.0f;
+                    t1 = trace<FORMAT, false>(s, bo, bd, t, my);
+                    if (t1 >= 0) {
+                        q = add(bo, scale(bd, t));
+                        nq = face_normal(s, t1, bd);
+                    }
+                }
+                T.tri1[lane] = t1;
+                T.q[0][lane] = q.x;
+                T.q[1][lane] = q.y;
+                T.q[2][lane] = q.z;
+                T.nq[0][lane] = nq.x;
+                T.nq[1][lane] = nq.y;
+                T.nq[2][lane] = nq.z;
+            } else {
+                const bool seen = t0 >= 0 && visible<FORMAT>(s, p, n, load3(P.lpos, k - 1), my);
+                const unsigned long long m = __ballot(seen);
+                if (lane == 0) T.vis_p[k - 1] = m;
+            }
+        }
+        __syncthreads();
+        int32_t t1 = -1;
+        f3 q = mk(0.0f, 0.0f, 0.0f), nq = q;
+        if (t0 >= 0) {
+            t1 = T.tri1[lane];
+            q = mk(T.q[0][lane], T.q[1][lane], T.q[2][lane]);
+            nq = mk(T.nq[0][lane], T.nq[1][lane], T.nq[2][lane]);
+        }
+        // q to every light
+        for (int32_t l = any ? claim(&T.next[1]) : P.nl; l < P.nl; l = claim(&T.next[1])) {
+            const bool seen = t1 >= 0 && visible<FORMAT>(s, q, nq, load3(P.lpos, l), my);
+            const unsigned long long m = __ballot(seen);
+            if (lane == 0) T.vis_q[l] = m;
+        }
+        __syncthreads();
+        // one wave, another each time, writes the tile's records and colors; the others go on
+        if (wave_id() != turn % kWaves) continue;
+        if (lane < 2) T.next[lane] = 0;
+        if (i >= npix) continue;
+        crt_shade_record out;
+        uint32_t vis = 0;
+        f3 c = mk(0.0f, 0.0f, 0.0f);
+        if (t0 >= 0) {
+            const f3 alb0 = load3(P.albedo, t0);
+            const float r0 = P.rough[t0];
+            const f3 alb1 = t1 >= 0 ? load3(P.albedo, t1) : mk(0.0f, 0.0f, 0.0f);
+            float B1 = 0.0f;
+            for (int32_t l = 0; l < P.nl; ++l) {
+                const f3 L = load3(P.lpos, l);
+                const float I = P.inten[l];
+                if (T.vis_p[l] >> lane & 1ull) {
+                    vis |= 1u << l;
+                    const CT t = cook_torrance(p, n, eye, L, I, r0);
+                    c = add(c, mk(t.A * (t.kd * alb0.x + t.spec), t.A * (t.kd * alb0.y + t.spec),
+                                  t.A * (t.kd * alb0.z + t.spec)));
+                }
+                if (T.vis_q[l] >> lane & 1ull) {
+                    vis |= 1u << (16 + l);
+                    B1 += lambert(q, nq, L, I);
+                }
+            }
+            c = add(c, mk(alb0.x * alb1.x * B1, alb0.y * alb1.y * B1, alb0.z * alb1.z * B1));
+        }
+        color[3 * i] = c.x;
+        color[3 * i + 1] = c.y;
+        color[3 * i + 2] = c.z;
+        out.pad0 = out.pad1 = 0.0f;
+        out.tri0 = t0;
+        out.tri1 = t1;
+        out.vis = vis;
+        out.eye[0] = eye.x;
+        out.eye[1] = eye.y;
+        out.eye[2] = eye.z;
+        out.p[0] = p.x;
+        out.p[1] = p.y;
+        out.p[2] = p.z;
+        out.n[0] = n.x;
+        out.n[1] = n.y;
+        out.n[2] = n.z;
+        out.q[0] = q.x;
+        out.q[1] = q.y;
+        out.q[2] = q.z;
+        out.nq[0] = nq.x;
+        out.nq[1] = nq.y;
+        out.nq[2] = nq.z;
         rec[i] = out;
-        color[3 * i] = color[3 * i + 1] = color[3 * i + 2] = 0.0f;
-        return;
     }
-    const int32_t t0 = h.tri;
-    const f3 p = add(eye, scale(dir, h.t));
-    const f3 n = face_normal(s, t0, dir);
-    // cosine-weighted bounce (Sampling.glsl:1-12) from per-pixel PCG uniforms
-    const uint32_t h1 = pcg(uint32_t(i) ^ (seed * 0x9E3779B9u));
-    const uint32_t h2 = pcg(h1);
-    const float u1 = float(h1 >> 8) * (1.0f / 16777216.0f);
-    const float u2 = float(h2 >> 8) * (1.0f / 16777216.0f);
-    f3 uu = cross(n, mk(0.0f, 1.0f, 1.0f));
-    if (dot(uu, uu) < 1e-12f) uu = cross(n, mk(1.0f, 0.0f, 0.0f));
-    uu = normalize(uu);
-    const f3 vv = cross(uu, n);
-    const float ra = sqrtf(u2);
-    const float rx = ra * cosf(kTwoPi * u1), ry = ra * sinf(kTwoPi * u1), rz = sqrtf(1.0f - u2);
-    const f3 bd = normalize(add(add(scale(uu, rx), scale(vv, ry)), scale(n, rz)));
-    const f3 bo = add(p, scale(n, kOffset));
-    crt_ray br;
-    br.org[0] = bo.x;
-    br.org[1] = bo.y;
-    br.org[2] = bo.z;
-    br.tmax = 1000000.0f;
-    br.dir[0] = bd.x;
-    br.dir[1] = bd.y;
-    br.dir[2] = bd.z;
-    br.id = 0;
-    uint32_t tests = 0;
-    const crt_hit bh = dev::scene_trace<FORMAT, false, 16>(s, br, 0u, kMaxIterations, tests, my, 128);
-    int32_t t1 = -1;
-    f3 q = mk(0.0f, 0.0f, 0.0f), nq = q;
-    if (bh.t > 0.0f && bh.tri >= 0) {
-        t1 = bh.tri;
-        q = add(bo, scale(bd, bh.t));
-        nq = face_normal(s, t1, bd);
-    }
-    const f3 alb0 = load3(P.albedo, t0);
-    const float r0 = P.rough[t0];
-    const f3 alb1 = t1 >= 0 ? load3(P.albedo, t1) : mk(0.0f, 0.0f, 0.0f);
-    f3 c = mk(0.0f, 0.0f, 0.0f);
-    float B1 = 0.0f;
-    uint32_t vis = 0;
-    for (int32_t l = 0; l < P.nl; ++l) {
-        const f3 L = load3(P.lpos, l);
-        const float I = P.inten[l];
-        if (visible<FORMAT>(s, p, n, L, my, 128)) {
-            vis |= 1u << l;
-            const CT t = cook_torrance(p, n, eye, L, I, r0);
-            c = add(c, mk(t.A * (t.kd * alb0.x + t.spec), t.A * (t.kd * alb0.y + t.spec),
-                          t.A * (t.kd * alb0.z + t.spec)));
-        }
-        if (t1 >= 0 && visible<FORMAT>(s, q, nq, L, my, 128)) {
-            vis |= 1u << (16 + l);
-            B1 += lambert(q, nq, L, I);
-        }
-    }
-    c = add(c, mk(alb0.x * alb1.x * B1, alb0.y * alb1.y * B1, alb0.z * alb1.z * B1));
-    color[3 * i] = c.x;
-    color[3 * i + 1] = c.y;
-    color[3 * i + 2] = c.z;
-    out.tri0 = t0;
-    out.tri1 = t1;
-    out.vis = vis;
-    out.p[0] = p.x;
-    out.p[1] = p.y;
-    out.p[2] = p.z;
-    out.n[0] = n.x;
-    out.n[1] = n.y;
-    out.n[2] = n.z;
-    out.q[0] = q.x;
-    out.q[1] = q.y;
-    out.q[2] = q.z;
-    out.nq[0] = nq.x;
-    out.nq[1] = nq.y;
-    out.nq[2] = nq.z;
-    rec[i] = out;
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -262,10 +366,39 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// Adds v[0..NV) into base[idx * NV + k] for every lane with idx >= 0; lanes
-// that share an index are summed in-wave first.  Called by all lanes of a wave.
-template <int NV>
-__device__ __forceinline__ void wave_scatter_add(float* __restrict__ base, int32_t idx, const float (&v)[NV]) {
+// Gradients that several pixels of a wave add to one triangle meet in the
+// workgroup's LDS first: a few triangles cover most of an image, and their
+// global atomics queue up behind each other.  One entry per set; an entry that
+// another triangle needs, and every entry at the end, goes to memory.
+struct Gradients {
+    static constexpr int kSets = 128;
+    float v[kSets][4];   // albedo, roughness
+    int32_t tri[kSets];
+
+    __device__ __forceinline__ void clear() {
+        for (int k = threadIdx.x; k < kSets; k += kBlock) tri[k] = -1;
+    }
+    __device__ __forceinline__ void flush(int k, float* __restrict__ g_albedo, float* __restrict__ g_rough) const {
+        if (tri[k] < 0) return;
+        for (int c = 0; c < 3; ++c) atomicAdd(g_albedo + 3 * int64_t(tri[k]) + c, v[k][c]);
+        if (v[k][3] != 0.0f) atomicAdd(g_rough + tri[k], v[k][3]);
+    }
+    // One lane adds for triangle t.
+    __device__ __forceinline__ void add(int32_t t, const float (&g)[4], float* __restrict__ g_albedo,
+                                        float* __restrict__ g_rough) {
+        const int k = t % kSets;
+        const bool mine = tri[k] == t;
+        if (!mine) flush(k, g_albedo, g_rough);
+        tri[k] = t;
+        for (int c = 0; c < 4; ++c) v[k][c] = mine ? v[k][c] + g[c] : g[c];
+    }
+};
+
+// Adds v to the gradients of triangle idx (none below 0) for every lane; lanes
+// that share a triangle are summed in-wave first.  Called by all lanes of a
+// wave, by one wave of the workgroup at a time.
+__device__ __forceinline__ void wave_scatter_add(Gradients& G, int32_t idx, const float (&v)[4],
+                                                 float* __restrict__ g_albedo, float* __restrict__ g_rough) {
     unsigned long long pending = __ballot(idx >= 0);
     const unsigned lane = __lane_id();
     while (pending) {
@@ -276,36 +409,28 @@ __device__ __forceinline__ void wave_scatter_add(float* __restrict__ base, int32
         if (m == (1ull << leader)) {
             // the leader alone holds this index: its own values, no reduction
             if (lane == unsigned(leader)) {
-#pragma unroll
-                for (int k = 0; k < NV; ++k) atomicAdd(base + int64_t(lidx) * NV + k, v[k]);
+                for (int c = 0; c < 3; ++c) atomicAdd(g_albedo + 3 * int64_t(lidx) + c, v[c]);
+                if (v[3] != 0.0f) atomicAdd(g_rough + lidx, v[3]);
             }
         } else {
+            float sum[4];
 #pragma unroll
-            for (int k = 0; k < NV; ++k) {
-                const float sum = wave_sum(mine ? v[k] : 0.0f);
-                if (lane == unsigned(leader)) atomicAdd(base + int64_t(lidx) * NV + k, sum);
-            }
+            for (int k = 0; k < 4; ++k) sum[k] = wave_sum(mine ? v[k] : 0.0f);
+            if (lane == unsigned(leader)) G.add(lidx, sum, g_albedo, g_rough);
         }
         pending &= ~m;
     }
 }
 
-// The adjoint of one pixel (a tile of 128 pixels per workgroup: every lane
-// of a wave calls it, with i >= npix for lanes past the end): albedo and
-// roughness gradients are added to the triangles' entries, and each light's
-// intensity gradient, summed over the wave, into the workgroup's LDS sum.
-template <int FORMAT>
-__device__ __forceinline__ void backward_pixel(const SceneArgs& s, const crt_shade_record* __restrict__ rec,
-                                               int64_t i, int64_t npix, const Params& P,
-                                               const float* __restrict__ color, const float* __restrict__ target,
-                                               float* __restrict__ g_albedo, float* __restrict__ g_rough,
-                                               float* inten_sum, int32_t* my) {
-    // every field is initialized: with some left undefined for the lanes past
-    // the end, the compiler may assume that there are none and drop the bound
-    crt_shade_record R{};
-    R.tri0 = -1;
-    R.tri1 = -1;
-    if (i < npix) R = rec[i];
+// The adjoint of a tile's pixels, one per lane of the wave (a lane without one
+// has tri0 < 0), with the visibility its workgroup traced: albedo and
+// roughness gradients are added to the triangles' entries, each light's
+// intensity gradient, summed over the wave, to the workgroup's LDS sum.
+__device__ __forceinline__ void adjoint(const Params& P, const crt_shade_record& R, int64_t i, const Tile& T,
+                                        const float* __restrict__ color, const float* __restrict__ target,
+                                        float* __restrict__ g_albedo, float* __restrict__ g_rough, Gradients& G,
+                                        float* inten_sum) {
+    const uint32_t lane = __lane_id();
     const bool valid = R.tri0 >= 0;
     const int32_t t0 = R.tri0;
     const int32_t t1 = valid ? R.tri1 : -1;
@@ -322,57 +447,97 @@ __device__ __forceinline__ void backward_pixel(const SceneArgs& s, const crt_sha
         if (t1 >= 0) alb1 = load3(P.albedo, t1);
     }
     float SAkd0 = 0.0f, Sd0 = 0.0f, B1 = 0.0f;
-    // the light loop is wave-uniform so each light's intensity gradient is
-    // reduced in-wave and added to the workgroup's sum with one LDS atomic
     for (int32_t l = 0; l < P.nl; ++l) {
         float dI = 0.0f;
-        if (valid) {
-            const f3 L = load3(P.lpos, l);
-            const float I = P.inten[l];
-            if (visible<FORMAT>(s, p, n, L, my, 128)) {
-                const CT t = cook_torrance(p, n, eye, L, I, r0);
-                SAkd0 += t.A * t.kd;
-                Sd0 += t.A * t.dspec;
-                dI += (g.x * t.A * (t.kd * alb0.x + t.spec) + g.y * t.A * (t.kd * alb0.y + t.spec) +
-                       g.z * t.A * (t.kd * alb0.z + t.spec)) / I;
-            }
-            if (t1 >= 0 && visible<FORMAT>(s, q, nq, L, my, 128)) {
-                const float b = lambert(q, nq, L, I);
-                B1 += b;
-                dI += (g.x * alb0.x * alb1.x + g.y * alb0.y * alb1.y + g.z * alb0.z * alb1.z) * b / I;
-            }
+        const f3 L = load3(P.lpos, l);
+        const float I = P.inten[l];
+        if (T.vis_p[l] >> lane & 1ull) {
+            const CT t = cook_torrance(p, n, eye, L, I, r0);
+            SAkd0 += t.A * t.kd;
+            Sd0 += t.A * t.dspec;
+            dI += (g.x * t.A * (t.kd * alb0.x + t.spec) + g.y * t.A * (t.kd * alb0.y + t.spec) +
+                   g.z * t.A * (t.kd * alb0.z + t.spec)) / I;
+        }
+        if (T.vis_q[l] >> lane & 1ull) {
+            const float b = lambert(q, nq, L, I);
+            B1 += b;
+            dI += (g.x * alb0.x * alb1.x + g.y * alb0.y * alb1.y + g.z * alb0.z * alb1.z) * b / I;
         }
         const float sum = wave_sum(dI);
-        if (__lane_id() == 0) atomicAdd(inten_sum + l, sum);
+        if (lane == 0) atomicAdd(inten_sum + l, sum);
     }
-    const float a0[3] = {g.x * (SAkd0 + alb1.x * B1), g.y * (SAkd0 + alb1.y * B1), g.z * (SAkd0 + alb1.z * B1)};
-    const float r0g[1] = {(g.x + g.y + g.z) * Sd0};
-    const float a1[3] = {g.x * alb0.x * B1, g.y * alb0.y * B1, g.z * alb0.z * B1};
-    wave_scatter_add<3>(g_albedo, valid ? t0 : -1, a0);
-    wave_scatter_add<1>(g_rough, valid ? t0 : -1, r0g);
-    wave_scatter_add<3>(g_albedo, t1, a1);
+    const float a0[4] = {g.x * (SAkd0 + alb1.x * B1), g.y * (SAkd0 + alb1.y * B1), g.z * (SAkd0 + alb1.z * B1),
+                         (g.x + g.y + g.z) * Sd0};
+    const float a1[4] = {g.x * alb0.x * B1, g.y * alb0.y * B1, g.z * alb0.z * B1, 0.0f};
+    wave_scatter_add(G, valid ? t0 : -1, a0, g_albedo, g_rough);
+    wave_scatter_add(G, t1, a1, g_albedo, g_rough);
 }
 
-// Workgroups of 128 lanes take tiles of 128 pixels in a grid-stride loop
-// (the launch caps the grid at a few workgroups per CU), so the intensity
-// gradients, which every pixel adds to, leave each workgroup as one global
-// atomic per light instead of one per wave: the few addresses they share are
-// otherwise the kernel's bottleneck.
+// The intensity gradients, which every pixel adds to, leave each workgroup as
+// one global atomic per light instead of one per wave: the few addresses they
+// share are otherwise the kernel's bottleneck.
 template <int FORMAT>
-__global__ void __launch_bounds__(128) backward_kernel(SceneArgs s, const crt_shade_record* __restrict__ rec,
-                                                       int64_t npix, Params P, const float* __restrict__ color,
-                                                       const float* __restrict__ target, float* __restrict__ g_albedo,
-                                                       float* __restrict__ g_rough, float* __restrict__ g_inten) {
-    __shared__ int32_t lds[16 * 128];
+__global__ void __launch_bounds__(kBlock) backward_kernel(SceneArgs s, const crt_shade_record* __restrict__ rec,
+                                                          int64_t npix, Params P, const float* __restrict__ color,
+                                                          const float* __restrict__ target,
+                                                          float* __restrict__ g_albedo, float* __restrict__ g_rough,
+                                                          float* __restrict__ g_inten) {
+    __shared__ int32_t stack[stack_ints<FORMAT>()];
+    __shared__ Tile tiles[2];
+    __shared__ Gradients G;
     __shared__ float inten_sum[kMaxLights];
+    int32_t* my = stack + (FORMAT == CRT_FORMAT_STACK ? threadIdx.x : 0);
     if (threadIdx.x < unsigned(kMaxLights)) inten_sum[threadIdx.x] = 0.0f;
+    if (threadIdx.x < 2) tiles[threadIdx.x].next[0] = 0;
+    G.clear();
     __syncthreads();
-    int32_t* my = lds + threadIdx.x;
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    for (int64_t base = int64_t(blockIdx.x) * blockDim.x; base < npix; base += stride)
-        backward_pixel<FORMAT>(s, rec, base + threadIdx.x, npix, P, color, target, g_albedo, g_rough, inten_sum, my);
+    const uint32_t lane = __lane_id();
+    const int64_t ntiles = (npix + 63) / 64;
+    int32_t turn = 0;
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, ++turn) {
+        Tile& T = tiles[turn & 1];
+        const int64_t i = tile * 64 + lane;
+        // every field is initialized: with some left undefined for the lanes past
+        // the end, the compiler may assume that there are none and drop the bound
+        crt_shade_record R{};
+        R.tri0 = R.tri1 = -1;
+        if (i < npix) R = rec[i];
+        const bool valid = R.tri0 >= 0;
+        const bool again = valid && R.tri1 >= 0;
+        const bool any = __any(valid);
+        for (int32_t k = any ? claim(&T.next[0]) : 2 * P.nl; k < 2 * P.nl; k = claim(&T.next[0])) {
+            const bool first = k < P.nl;
+            const int32_t l = first ? k : k - P.nl;
+            const float* x = first ? R.p : R.q;
+            const float* xn = first ? R.n : R.nq;
+            const bool seen = (first ? valid : again) &&
+                              visible<FORMAT>(s, mk(x[0], x[1], x[2]), mk(xn[0], xn[1], xn[2]), load3(P.lpos, l), my);
+            const unsigned long long m = __ballot(seen);
+            if (lane == 0) (first ? T.vis_p : T.vis_q)[l] = m;
+        }
+        __syncthreads();
+        // one wave, another each time, takes the tile's gradients; the others go on
+        if (wave_id() != turn % kWaves) continue;
+        if (lane == 0) T.next[0] = 0;
+        if (any) adjoint(P, R, i, T, color, target, g_albedo, g_rough, G, inten_sum);
+    }
     __syncthreads();
+    for (int k = threadIdx.x; k < Gradients::kSets; k += kBlock) G.flush(k, g_albedo, g_rough);
     if (threadIdx.x < unsigned(P.nl)) atomicAdd(g_inten + threadIdx.x, inten_sum[threadIdx.x]);
+}
+
+// Workgroups that fill the device once, or one per tile where there are fewer.
+template <typename F>
+unsigned tile_grid(F kernel, int64_t npix) {
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), kBlock, 0) !=
+            hipSuccess || per_cu <= 0)
+        per_cu = 4;
+    const int64_t tiles = (npix + 63) / 64;
+    return unsigned(tiles < int64_t(cus) * per_cu ? tiles : int64_t(cus) * per_cu);
 }
 
 }  // namespace shade
@@ -408,14 +573,10 @@ int crt_shade_forward(const crt_scene_view* scene, const crt_ray* primary_rays, 
     if (npix < 0 || (npix > 0 && (!primary_rays || !primary_hits || !color || !records)))
         return crt::set_error(CRT_E_INVALID, "crt_shade_forward: bad buffers");
     if (npix == 0) return CRT_OK;
-    const unsigned grid = unsigned((npix + 127) / 128);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (a.format == CRT_FORMAT_STACKLESS)
-        hipLaunchKernelGGL(crt::shade::forward_kernel<CRT_FORMAT_STACKLESS>, dim3(grid), dim3(128), 0, st, a,
-                           primary_rays, primary_hits, npix, p, seed, color, records);
-    else
-        hipLaunchKernelGGL(crt::shade::forward_kernel<CRT_FORMAT_STACK>, dim3(grid), dim3(128), 0, st, a,
-                           primary_rays, primary_hits, npix, p, seed, color, records);
+    const auto fn = a.format == CRT_FORMAT_STACKLESS ? crt::shade::forward_kernel<CRT_FORMAT_STACKLESS>
+                                                     : crt::shade::forward_kernel<CRT_FORMAT_STACK>;
+    hipLaunchKernelGGL(fn, dim3(crt::shade::tile_grid(fn, npix)), dim3(crt::shade::kBlock), 0,
+                       static_cast<hipStream_t>(stream), a, primary_rays, primary_hits, npix, p, seed, color, records);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return crt::set_error(CRT_E_HIP, std::string("crt_shade_forward: ") + hipGetErrorString(e));
     return CRT_OK;
@@ -432,21 +593,11 @@ int crt_shade_backward(const crt_scene_view* scene, const crt_shade_record* reco
                                   !grad_intensity)))
         return crt::set_error(CRT_E_INVALID, "crt_shade_backward: bad buffers");
     if (npix == 0) return CRT_OK;
-    // at most 16 workgroups of 128 lanes per CU (more than fit at once), so
-    // each workgroup walks several tiles
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    const int64_t tiles = (npix + 127) / 128;
-    const unsigned grid = unsigned(tiles < int64_t(cus) * 16 ? tiles : int64_t(cus) * 16);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (a.format == CRT_FORMAT_STACKLESS)
-        hipLaunchKernelGGL(crt::shade::backward_kernel<CRT_FORMAT_STACKLESS>, dim3(grid), dim3(128), 0, st, a,
-                           records, npix, p, color, target, grad_albedo, grad_roughness, grad_intensity);
-    else
-        hipLaunchKernelGGL(crt::shade::backward_kernel<CRT_FORMAT_STACK>, dim3(grid), dim3(128), 0, st, a, records,
-                           npix, p, color, target, grad_albedo, grad_roughness, grad_intensity);
+    const auto fn = a.format == CRT_FORMAT_STACKLESS ? crt::shade::backward_kernel<CRT_FORMAT_STACKLESS>
+                                                     : crt::shade::backward_kernel<CRT_FORMAT_STACK>;
+    hipLaunchKernelGGL(fn, dim3(crt::shade::tile_grid(fn, npix)), dim3(crt::shade::kBlock), 0,
+                       static_cast<hipStream_t>(stream), a, records, npix, p, color, target, grad_albedo,
+                       grad_roughness, grad_intensity);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return crt::set_error(CRT_E_HIP, std::string("crt_shade_backward: ") + hipGetErrorString(e));
     return CRT_OK;
