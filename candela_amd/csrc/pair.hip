@@ -16,25 +16,23 @@ namespace pair {
 
 template <bool ANY, int D, int I, int LB>
 __global__ void __launch_bounds__(256) pair_grid(PairScene s, const crt_ray* rays, crt_hit* __restrict__ hits,
-                                                 int64_t n, uint32_t flags, int32_t max_iter, int32_t blocks) {
+                                                 int64_t n, uint32_t flags, int32_t max_iter, int32_t log2,
+                                                 int32_t blocks) {
     __shared__ typename PairStack<D>::Entry lds[D * 256];
-    const int32_t per = (blocks + 7) / 8;  // the grid is padded to a multiple of 8
-    const int32_t logical = int32_t(blockIdx.x % 8u) * per + int32_t(blockIdx.x / 8u);
-    if (logical >= blocks) return;
-    const int64_t i = int64_t(logical) * 256 + threadIdx.x;
+    const int64_t i = grid_ray(n, log2, blocks);
     typename PairStack<D>::Entry spill[spill_entries<D>()];
     PairStack<D> st{lds + threadIdx.x, 256, spill};
     PairWave<ANY, D, I, LB> w;
-    w.run(s, rays, hits, i < n ? i : -1, flags, max_iter, st);
+    w.run(s, rays, hits, i, flags, max_iter, st);
 }
 
 template <int D, int I, int LB>
 __global__ void __launch_bounds__(256) pair_primary(PairScene s, Camera cam, crt_ray* rays, crt_hit* __restrict__ hits,
-                                                    int32_t width, int32_t height, uint32_t flags, int32_t max_iter) {
+                                                    ImageTiles image, uint32_t flags, int32_t max_iter) {
     __shared__ typename PairStack<D>::Entry lds[D * 256];
-    const Pixel p = image_pixel(width, height);
+    const Pixel p = image_pixel(image);
     // a lane reads back only the ray that it wrote itself
-    if (p.i >= 0) store_ray(rays + p.i, primary_ray(cam, width, height, p.x, p.y, uint32_t(p.i)));
+    if (p.i >= 0) store_ray(rays + p.i, primary_ray(cam, image.width, image.height, p.x, p.y, uint32_t(p.i)));
     typename PairStack<D>::Entry spill[spill_entries<D>()];
     PairStack<D> st{lds + threadIdx.x, 256, spill};
     PairWave<false, D, I, LB> w;
@@ -72,22 +70,23 @@ hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* ver
 hipError_t launch_pair_grid(const PairScene& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                             uint32_t flags, int32_t max_iter, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    const int32_t blocks = int32_t((n + 255) / 256);
+    const int32_t log2 = rays_per_wave_log2(n);
+    const int32_t blocks = int32_t((n + (4 << log2) - 1) >> (log2 + 2));
     const unsigned padded = unsigned((blocks + 7) / 8 * 8);
     if (query == CRT_QUERY_ANY)
         hipLaunchKernelGGL((pair::pair_grid<true, CRT_PAIR_SHAPE>), dim3(padded), dim3(256), 0, stream, s, rays, hits,
-                           n, flags, max_iter, blocks);
+                           n, flags, max_iter, log2, blocks);
     else
         hipLaunchKernelGGL((pair::pair_grid<false, CRT_PAIR_SHAPE>), dim3(padded), dim3(256), 0, stream, s, rays, hits,
-                           n, flags, max_iter, blocks);
+                           n, flags, max_iter, log2, blocks);
     return hipGetLastError();
 }
 
 hipError_t launch_pair_primary(const PairScene& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,
                                int height, uint32_t flags, int32_t max_iter, hipStream_t stream) {
+    const dm::ImageTiles image = dm::image_tiles(width, height);
     hipLaunchKernelGGL((pair::pair_primary<CRT_PAIR_SHAPE>),
-                       dim3(unsigned(dm::image_grid(dm::image_blocks(width, height)))), dim3(256), 0, stream, s, cam,
-                       rays, hits, width, height, flags, max_iter);
+                       dim3(dm::image_grid(image)), dim3(256), 0, stream, s, cam, rays, hits, image, flags, max_iter);
     return hipGetLastError();
 }
 

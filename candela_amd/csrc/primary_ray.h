@@ -42,51 +42,65 @@ __device__ __forceinline__ void store_ray(crt_ray* out, const crt_ray& r) {
     p[1] = make_float4(r.dir[0], r.dir[1], r.dir[2], __uint_as_float(r.id));
 }
 
-// Pixel of a workgroup's lane: waves take 8 x 8 pixels (a workgroup 16 x 16),
-// whose rays share more of their walk than 64 pixels of one row do.  Images
-// narrower or lower than a tile are taken in row order.  Runs of kTileRun
-// workgroups go to one XCD (consecutive tiles share nodes in its L2), runs in
-// turn so that cheap and costly bands of the image are spread over all eight.
+// Pixel of a workgroup's lane: waves take blocks of pixels, 8 x 8 when full
+// (rays_per_wave_log2), and a workgroup 2 x 2 of them; they share more of their
+// walk than pixels of one row do.  Images narrower or lower than 8 pixels are
+// taken in row order.  Runs of kTileRun workgroups go to one XCD (consecutive
+// tiles share nodes in its L2), runs in turn so that cheap and costly bands of
+// the image are spread over all eight.
 constexpr int32_t kTileRun = 32;
+
+struct ImageTiles {
+    int32_t width, height;
+    int32_t log2;       // pixels of a wave
+    int32_t tiles_x;    // workgroups across; 0: row order
+    int64_t blocks;
+};
+
+inline ImageTiles image_tiles(int32_t width, int32_t height) {
+    ImageTiles t;
+    t.width = width;
+    t.height = height;
+    t.log2 = rays_per_wave_log2(int64_t(width) * height);
+    const int32_t w = 2 << ((t.log2 + 1) / 2), h = 2 << (t.log2 / 2);
+    t.tiles_x = width >= 8 && height >= 8 ? (width + w - 1) / w : 0;
+    t.blocks = t.tiles_x ? int64_t(t.tiles_x) * ((height + h - 1) / h)
+                         : ((int64_t(width) * height + (4 << t.log2) - 1) >> (t.log2 + 2));
+    return t;
+}
+
+// Workgroups to launch: whole rounds of runs.
+inline unsigned image_grid(const ImageTiles& t) {
+    const int64_t round = 8 * kTileRun;
+    return unsigned(t.blocks <= round ? t.blocks : (t.blocks + round - 1) / round * round);
+}
 
 struct Pixel {
     int32_t x, y;
     int64_t i;   // -1: none
 };
 
-__host__ __device__ inline bool image_tiled(int32_t width, int32_t height) { return width >= 8 && height >= 8; }
-
-inline int64_t image_blocks(int32_t width, int32_t height) {
-    return image_tiled(width, height) ? int64_t((width + 15) / 16) * ((height + 15) / 16)
-                                      : (int64_t(width) * height + 255) / 256;
-}
-
-// Grid of image_blocks(...) workgroups, padded to whole rounds of runs.
-inline int64_t image_grid(int64_t blocks) {
-    const int64_t round = 8 * kTileRun;
-    return blocks <= round ? blocks : (blocks + round - 1) / round * round;
-}
-
-__device__ __forceinline__ Pixel image_pixel(int32_t width, int32_t height) {
+__device__ __forceinline__ Pixel image_pixel(const ImageTiles& t) {
     int64_t b = blockIdx.x;
     if (gridDim.x > 8 * kTileRun) {
         const uint32_t k = blockIdx.x / 8u;
         b = (int64_t(k / kTileRun) * 8 + blockIdx.x % 8u) * kTileRun + k % kTileRun;
     }
-    Pixel p;
-    if (image_tiled(width, height)) {
-        const int32_t tiles = (width + 15) / 16;
-        const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63u;
-        const int64_t ty = b / tiles;
-        p.x = int32_t(b - ty * tiles) * 16 + int32_t((w & 1u) * 8 + (l & 7u));
-        const int64_t y = ty * 16 + int64_t((w >> 1) * 8 + (l >> 3));
-        p.y = int32_t(y);
-        p.i = p.x < width && y < height ? y * width + p.x : -1;
+    const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63u;
+    Pixel p{0, 0, -1};
+    if (l >> t.log2 || b >= t.blocks) return p;
+    if (t.tiles_x) {
+        const int32_t lx = (t.log2 + 1) / 2, ly = t.log2 / 2;
+        const int64_t ty = b / t.tiles_x;
+        p.x = (int32_t(b - ty * t.tiles_x) << (lx + 1)) + int32_t(((w & 1u) << lx) + (l & ((1u << lx) - 1u)));
+        p.y = (int32_t(ty) << (ly + 1)) + int32_t(((w >> 1) << ly) + (l >> lx));
+        if (p.x < t.width && p.y < t.height) p.i = int64_t(p.y) * t.width + p.x;
     } else {
-        p.i = b * 256 + threadIdx.x;
-        if (p.i >= int64_t(width) * height) p.i = -1;
-        p.y = int32_t(p.i / width);
-        p.x = int32_t(p.i - int64_t(p.y) * width);
+        const int64_t i = ((b * 4 + w) << t.log2) + l;
+        if (i >= int64_t(t.width) * t.height) return p;
+        p.i = i;
+        p.y = int32_t(i / t.width);
+        p.x = int32_t(i - int64_t(p.y) * t.width);
     }
     return p;
 }

@@ -925,15 +925,25 @@ static crt::PairScene pair_scene(const crt_context* ctx) {
                           static_cast<const float4*>(ctx->d_records)};
 }
 
+// The context's scene with its triangle records.
+static crt::SceneArgs record_scene(const crt_context* ctx, const crt_scene_view& s) {
+    crt::SceneArgs a = crt::scene_args(s);
+    a.tri_records = static_cast<const crt_tri_record*>(ctx->d_records);
+    return a;
+}
+
 int crt_intersect(crt_context* ctx, int query, uint32_t flags, const crt_ray* rays, crt_hit* hits, int64_t nrays,
                   void* stream) {
     crt_scene_view s;
     int rc = crt_context_scene(ctx, &s);
     if (rc) return rc;
-    if (ctx->pairs_fit && (query == CRT_QUERY_CLOSEST || query == CRT_QUERY_ANY) && nrays > 0 &&
+    const bool stack = ctx->format == CRT_FORMAT_STACK && ctx->d_records;
+    if ((ctx->pairs_fit || stack) && (query == CRT_QUERY_CLOSEST || query == CRT_QUERY_ANY) && nrays > 0 &&
         nrays < (int64_t(1) << 31) && rays && hits) {
-        CRT_HIP(crt::launch_pair_grid(pair_scene(ctx), query, rays, hits, nrays, flags, crt::kMaxIterations,
-                                      static_cast<hipStream_t>(stream)),
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        CRT_HIP(stack ? crt::launch_stack_records(record_scene(ctx, s), query, rays, hits, nrays, flags,
+                                                  crt::kMaxIterations, st)
+                      : crt::launch_pair_grid(pair_scene(ctx), query, rays, hits, nrays, flags, crt::kMaxIterations, st),
                 "crt_intersect: kernel launch");
         return CRT_OK;
     }
@@ -954,6 +964,12 @@ int crt_intersect_primary(crt_context* ctx, crt_ray* rays, crt_hit* hits, int wi
     if (ctx->pairs_fit && int64_t(width) * height < (int64_t(1) << 31)) {
         CRT_HIP(crt::launch_pair_primary(pair_scene(ctx), cam, rays, hits, width, height, flags, crt::kMaxIterations,
                                          static_cast<hipStream_t>(stream)),
+                "crt_intersect_primary: kernel launch");
+        return CRT_OK;
+    }
+    if (ctx->format == CRT_FORMAT_STACK && ctx->d_records && int64_t(width) * height < (int64_t(1) << 31)) {
+        CRT_HIP(crt::launch_stack_primary(record_scene(ctx, s), cam, rays, hits, width, height, flags,
+                                          crt::kMaxIterations, static_cast<hipStream_t>(stream)),
                 "crt_intersect_primary: kernel launch");
         return CRT_OK;
     }

@@ -15,6 +15,7 @@
 
 #include "candela_rt.h"
 #include "crt_internal.h"
+#include "primary_ray.h"
 #include "stack_walk.h"
 #include "trace_launch.h"
 
@@ -81,6 +82,34 @@ stack_persistent_occ(SceneArgs s, const crt_ray* __restrict__ rays, crt_hit* __r
                      unsigned long long* __restrict__ counters) {
     __shared__ int32_t lds[D * 256];
     persistent_body<ANY, D, I, LB, R>(s, rays, hits, n, flags, max_iter, tri_tests, counters, lds);
+}
+
+// The walk over a context's triangle records: a ray batch, or an image's
+// primary rays.
+template <bool ANY, int D, int I, int LB, int OCC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
+stack_records(SceneArgs s, const crt_ray* rays, crt_hit* __restrict__ hits, int64_t n, uint32_t flags, int32_t max_iter,
+              int32_t log2, int32_t blocks) {
+    __shared__ int32_t lds[D * 256];
+    const int64_t i = grid_ray(n, log2, blocks);
+    int32_t spill[spill_entries<D>()];
+    NodeStack<D> st{lds + threadIdx.x, 256, spill};
+    StackWave<ANY, D, I, LB, true> w;
+    w.run(s, rays, hits, i, flags, max_iter, nullptr, st);
+}
+
+template <int D, int I, int LB, int OCC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
+stack_primary(SceneArgs s, Camera cam, crt_ray* rays, crt_hit* __restrict__ hits, ImageTiles image, uint32_t flags,
+              int32_t max_iter) {
+    __shared__ int32_t lds[D * 256];
+    const Pixel p = image_pixel(image);
+    // a lane reads back only the ray that it wrote itself
+    if (p.i >= 0) store_ray(rays + p.i, primary_ray(cam, image.width, image.height, p.x, p.y, uint32_t(p.i)));
+    int32_t spill[spill_entries<D>()];
+    NodeStack<D> st{lds + threadIdx.x, 256, spill};
+    StackWave<false, D, I, LB, true> w;
+    w.run(s, rays, hits, p.i, flags, max_iter, nullptr, st);
 }
 
 template <bool ANY, int D, int I, int LB, int OCC>
@@ -198,6 +227,34 @@ hipError_t launch_stack_persistent(const SceneArgs& s, int query, const crt_ray*
     void* args[] = {&sa, &r, &h, &nn, &fl, &mi, &tt, &c};
     e = hipLaunchKernel(fn, dim3(unsigned(grid)), dim3(256), args, 0, stream);
     if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+
+// LDS stack entries, node steps per round, parked lanes that end the node
+// phase, waves per SIMD asked for (the registers allow 6).  552,960 occlusion
+// rays over 640,000 triangles: 159 us; (16, 4, 16) 164, (16, 8, 16) 165, (16, 2,
+// 16) 172, 7 waves (with spills) 176, the thread-per-ray walk 240.
+#define CRT_STACK_REC 16, 4, 32, 1
+
+hipError_t launch_stack_records(const SceneArgs& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
+                                uint32_t flags, int32_t max_iter, hipStream_t stream) {
+    if (n <= 0) return hipSuccess;
+    const int32_t log2 = rays_per_wave_log2(n);
+    const int32_t blocks = int32_t((n + (4 << log2) - 1) >> (log2 + 2));
+    const unsigned padded = unsigned((blocks + 7) / 8 * 8);
+    if (query == CRT_QUERY_ANY)
+        hipLaunchKernelGGL((sdev::stack_records<true, CRT_STACK_REC>), dim3(padded), dim3(256), 0, stream, s, rays,
+                           hits, n, flags, max_iter, log2, blocks);
+    else
+        hipLaunchKernelGGL((sdev::stack_records<false, CRT_STACK_REC>), dim3(padded), dim3(256), 0, stream, s, rays,
+                           hits, n, flags, max_iter, log2, blocks);
+    return hipGetLastError();
+}
+
+hipError_t launch_stack_primary(const SceneArgs& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,
+                                int height, uint32_t flags, int32_t max_iter, hipStream_t stream) {
+    const dm::ImageTiles image = dm::image_tiles(width, height);
+    hipLaunchKernelGGL((sdev::stack_primary<CRT_STACK_REC>), dim3(dm::image_grid(image)), dim3(256), 0, stream, s, cam, rays, hits, image, flags, max_iter);
     return hipGetLastError();
 }
 

@@ -26,6 +26,11 @@
 //
 // The stack keeps its first LDS_DEPTH entries in LDS (entry-major, lane i of
 // a wave on bank i) and the rest in a per-lane scratch array.
+//
+// Bound: the chain of node fetches, then VALU issue.  All of an entry is loaded
+// before any of it is used (pin), and both triangles of a pair of tests: the
+// compiler otherwise moves a child's box, or the second triangle, behind the
+// branch that needs it, a round trip more per step.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -58,13 +63,18 @@ struct NodeStack {
     int32_t* spill;
 
     __device__ __forceinline__ LdsInt* col() const { return (LdsInt*)lds; }   // see LdsInt
+    // Entries beyond the LDS part are rare: one uniform test skips the scratch code.
     __device__ __forceinline__ void put(int32_t sp, int32_t v) {
-        if (sp < LDS_DEPTH)
+        if (!__any(sp >= LDS_DEPTH)) {
             col()[sp * stride] = v;
-        else
+        } else if (sp < LDS_DEPTH) {
+            col()[sp * stride] = v;
+        } else {
             spill[sp - LDS_DEPTH] = v;
+        }
     }
     __device__ __forceinline__ int32_t get(int32_t sp) const {
+        if (!__any(sp >= LDS_DEPTH)) return col()[sp * stride];
         return sp < LDS_DEPTH ? col()[sp * stride] : spill[sp - LDS_DEPTH];
     }
 };
@@ -73,7 +83,8 @@ enum StepResult : int32_t { kNext = 0, kLeaves = 1, kEnd = 2 };
 
 __device__ __forceinline__ bool leaf_nonempty(int32_t packed) { return packed != -1 && (packed & 0xF) > 0; }
 
-template <bool ANY, int LDS_DEPTH, int INNER, int LEAF_BATCH>
+// REC: triangles come from s.tri_records (one per triangle, by its index).
+template <bool ANY, int LDS_DEPTH, int INNER, int LEAF_BATCH, bool REC = false>
 struct StackWave {
     f3 ro, rd, inv;        // ray in the current entity's space
     float tmax;            // walk TMax: closest shrinks with every hit; any-hit starts each walk at ray_tmax
@@ -92,7 +103,7 @@ struct StackWave {
 
     // Next entity that takes part (IgnoreTransparent skips alpha < 0.99);
     // false when the entity loop is over.
-    __device__ __forceinline__ bool begin_walk(const SceneArgs& s, const crt_ray* __restrict__ rays, uint32_t flags) {
+    __device__ __forceinline__ bool begin_walk(const SceneArgs& s, const crt_ray* rays, uint32_t flags) {
         int32_t e = ent + 1;
         while (e < s.entity_count && (flags & CRT_FLAG_IGNORE_TRANSPARENT) &&
                __int_as_float(s.entities[e].data[1]) < 0.99f)
@@ -116,7 +127,7 @@ struct StackWave {
         return true;
     }
 
-    __device__ __forceinline__ void finish(const SceneArgs& s, const crt_ray* __restrict__ rays,
+    __device__ __forceinline__ void finish(const SceneArgs& s, const crt_ray* rays,
                                            crt_hit* __restrict__ hits, uint32_t* __restrict__ tri_tests,
                                            uint32_t flags) {
         float4 tuvw = make_float4(-1.0f, -1.0f, -1.0f, -1.0f);
@@ -132,8 +143,8 @@ struct StackWave {
                 const float4 a = rp[0], b = rp[1];
                 const f3 lro = xform(e.inverse, mk(a.x, a.y, a.z), 1.0f);
                 const f3 lrd = xform(e.inverse, mk(b.x, b.y, b.z), 0.0f);
-                const int4 tr = *reinterpret_cast<const int4*>(s.tris[tri].packed);
-                const f3 va = vertex_pos(s.verts, tr.x), vb = vertex_pos(s.verts, tr.y), vc = vertex_pos(s.verts, tr.z);
+                f3 va, vb, vc;
+                (void)corners(s, tri, va, vb, vc);
                 const f3 p = mk(lro.x + lrd.x * closest, lro.y + lrd.y * closest, lro.z + lrd.z * closest);
                 const f3 uvw = barycentrics(p, va, vb, vc);
                 tuvw = make_float4(closest, uvw.x, uvw.y, uvw.z);
@@ -147,7 +158,7 @@ struct StackWave {
     }
 
     // Lane takes ray i.
-    __device__ __forceinline__ void begin_ray(const SceneArgs& s, const crt_ray* __restrict__ rays,
+    __device__ __forceinline__ void begin_ray(const SceneArgs& s, const crt_ray* rays,
                                               crt_hit* __restrict__ hits, int64_t i, uint32_t flags,
                                               uint32_t* __restrict__ tri_tests) {
         active = true;
@@ -179,11 +190,16 @@ struct StackWave {
         }
         it++;
         const float4* np = reinterpret_cast<const float4*>(s.nodes) + 4 * int64_t(cur);
-        const float4 lmin = np[0], lmax = np[1], rmin = np[2], rmax = np[3];
+        float4 lmin = np[0], lmax = np[1], rmin = np[2], rmax = np[3];
+        pin(lmin);
+        pin(lmax);
+        pin(rmin);
+        pin(rmax);
         const int32_t lp = __float_as_int(lmin.w), rp = __float_as_int(rmin.w);
         const bool lleaf = lp != -1, rleaf = rp != -1;
-        const float lt = lleaf ? -1.0f : bounds_stack(lmin, lmax, ro, inv, tmax);
-        const float rt = rleaf ? -1.0f : bounds_stack(rmin, rmax, ro, inv, tmax);
+        const float lb = bounds_stack(lmin, lmax, ro, inv, tmax), rb = bounds_stack(rmin, rmax, ro, inv, tmax);
+        const float lt = lleaf ? -1.0f : lb;
+        const float rt = rleaf ? -1.0f : rb;
         leaf0 = lp;
         leaf1 = rp;
         uint32_t end = 0;
@@ -221,21 +237,53 @@ struct StackWave {
         return kNext;
     }
 
-    __device__ __forceinline__ bool test(int32_t idx, int4 tr, f3 a, f3 b, f3 c) {
-        const float t = tri_t(ro, rd, a, b, c);
-        tests++;
-        if (t > 0.0f && t < tmax) {
-            tmax = t;
-            mesh = tr.w;
-            tri = idx;
-            hit_ent = ent;
-            if (ANY) return true;
+    // Triangle i: its corners, and its mesh in the return value.
+    __device__ __forceinline__ static int32_t corners(const SceneArgs& s, int32_t i, f3& a, f3& b, f3& c) {
+        if constexpr (REC) {
+            const float4* p = reinterpret_cast<const float4*>(s.tri_records) + 3 * int64_t(i);
+            float4 va = p[0], vb = p[1], vc = p[2];
+            pin(va);
+            pin(vb);
+            pin(vc);
+            a = mk(va.x, va.y, va.z);
+            b = mk(vb.x, vb.y, vb.z);
+            c = mk(vc.x, vc.y, vc.z);
+            return __float_as_int(vb.w);
+        } else {
+            int4 tr = *reinterpret_cast<const int4*>(s.tris[i].packed);
+            pin(tr);
+            a = vertex_pos(s.verts, tr.x);
+            b = vertex_pos(s.verts, tr.y);
+            c = vertex_pos(s.verts, tr.z);
+            return tr.w;
         }
-        return false;
+    }
+
+    // Tests two triangles of a leaf (the same twice changes nothing); true when an any-hit walk ends.
+    __device__ __forceinline__ bool test(const SceneArgs& s, int32_t first, int32_t second) {
+        f3 a0, b0, c0, a1, b1, c1;
+        const int32_t m0 = corners(s, first, a0, b0, c0), m1 = corners(s, second, a1, b1, c1);
+        const float t0 = tri_t(ro, rd, a0, b0, c0), t1 = tri_t(ro, rd, a1, b1, c1);
+        const bool h0 = t0 > 0.0f && t0 < tmax;
+        tests += ANY && h0 ? 1 : second - first + 1;
+        if (h0) {
+            tmax = t0;
+            mesh = m0;
+            tri = first;
+            hit_ent = ent;
+        }
+        const bool h1 = t1 > 0.0f && t1 < tmax && !(ANY && h0);
+        if (h1) {
+            tmax = t1;
+            mesh = m1;
+            tri = second;
+            hit_ent = ent;
+        }
+        return ANY && (h0 || h1);
     }
 
     // One round of the wave: node phase, leaf phase, walk ends.
-    __device__ __forceinline__ void round(const SceneArgs& s, const crt_ray* __restrict__ rays,
+    __device__ __forceinline__ void round(const SceneArgs& s, const crt_ray* rays,
                                           crt_hit* __restrict__ hits, uint32_t flags, int32_t max_iter,
                                           uint32_t* __restrict__ tri_tests, NodeStack<LDS_DEPTH>& st) {
         // --- node phase ----------------------------------------------------------
@@ -262,12 +310,7 @@ struct StackWave {
                 const int32_t first = (leaf >> 4) + off, left = len - off;
                 // the second triangle, or the first again when one is left
                 const int32_t second = first + (left > 1 ? 1 : 0);
-                const int4 t0 = *reinterpret_cast<const int4*>(s.tris[first].packed);
-                const int4 t1 = *reinterpret_cast<const int4*>(s.tris[second].packed);
-                const f3 a0 = vertex_pos(s.verts, t0.x), b0 = vertex_pos(s.verts, t0.y), c0 = vertex_pos(s.verts, t0.z);
-                const f3 a1 = vertex_pos(s.verts, t1.x), b1 = vertex_pos(s.verts, t1.y), c1 = vertex_pos(s.verts, t1.z);
-                bool done = test(first, t0, a0, b0, c0);
-                if (!done && left > 1) done = test(second, t1, a1, b1, c1);
+                const bool done = test(s, first, second);
                 off += left > 1 ? 2 : 1;
                 if (done) {   // an any-hit walk ends at its first accepted triangle
                     leafing = false;
@@ -305,7 +348,7 @@ struct StackWave {
     }
 
     // Ray i per lane (i < 0: idle) until every lane is done.
-    __device__ __forceinline__ void run(const SceneArgs& s, const crt_ray* __restrict__ rays,
+    __device__ __forceinline__ void run(const SceneArgs& s, const crt_ray* rays,
                                         crt_hit* __restrict__ hits, int64_t i, uint32_t flags, int32_t max_iter,
                                         uint32_t* __restrict__ tri_tests, NodeStack<LDS_DEPTH> st) {
         active = false;
@@ -318,7 +361,7 @@ struct StackWave {
     // Rays [0, n) claimed from the sharded queue (queue.h): between rounds,
     // once at least `refill` lanes are idle, one claim takes a ray for each
     // idle lane.  Ends when the queue is dry and every lane is done.
-    __device__ __forceinline__ void run_refill(const SceneArgs& s, const crt_ray* __restrict__ rays,
+    __device__ __forceinline__ void run_refill(const SceneArgs& s, const crt_ray* rays,
                                                crt_hit* __restrict__ hits, int64_t n, uint32_t flags,
                                                int32_t max_iter, uint32_t* __restrict__ tri_tests,
                                                NodeStack<LDS_DEPTH> st, unsigned long long* __restrict__ counters,

@@ -1,8 +1,7 @@
 // Kernel arguments and launchers shared by the host runtime and trace.hip.
 #pragma once
 
-#include <hip/hip_runtime_api.h>
-#include <hip/hip_vector_types.h>
+#include <hip/hip_runtime.h>
 
 #include <cstdint>
 
@@ -114,6 +113,29 @@ hipError_t launch_stack_grid(const SceneArgs& s, int query, const crt_ray* rays,
 hipError_t launch_stack_persistent(const SceneArgs& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                                    uint32_t flags, int32_t max_iter, unsigned long long* counters,
                                    uint32_t* tri_tests, int variant, int grid, hipStream_t stream);
+
+// log2 of the rays a wave takes.
+inline int32_t rays_per_wave_log2(int64_t) { return 6; }
+
+// Ray of a grid launch's lane (workgroups of four waves, dealt to the XCDs so
+// that consecutive ones share an L2; the grid is padded to a multiple of 8), or
+// -1.  `blocks` = ceil(n / (4 << log2)).
+#ifdef __HIPCC__
+__device__ __forceinline__ int64_t grid_ray(int64_t n, int32_t log2, int32_t blocks) {
+    const int32_t per = (blocks + 7) / 8;
+    const int32_t logical = int32_t(blockIdx.x % 8u) * per + int32_t(blockIdx.x / 8u);
+    const uint32_t lane = threadIdx.x & 63u;
+    if (logical >= blocks || lane >> log2) return -1;
+    const int64_t i = ((int64_t(logical) * 4 + (threadIdx.x >> 6)) << log2) + lane;
+    return i < n ? i : -1;
+}
+#endif
+
+// The stack walk over a context's triangle records (s.tri_records, by triangle index).
+hipError_t launch_stack_records(const SceneArgs& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
+                                uint32_t flags, int32_t max_iter, hipStream_t stream);
+hipError_t launch_stack_primary(const SceneArgs& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,
+                                int height, uint32_t flags, int32_t max_iter, hipStream_t stream);
 
 // Speculative wave walk of the wide layouts (spec.hip; variant 0..5): grid
 // launch, and device-filling waves that refill from a queue block.
