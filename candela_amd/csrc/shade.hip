@@ -52,7 +52,9 @@ constexpr int kMaxLights = 16;
 // 560 us in two rounds, the chip half empty); 1,160 us as here, 1,295 when a
 // lane's leaf is tested as soon as it is reached; 805 us with gradients met in
 // LDS and one loop condition per node.  3 waves a tile take 6% more, 4 take 9%.
-constexpr int kWaves = 2, kBlock = 64 * kWaves;
+// An image of so few tiles that all fit the device at once with kWide waves each
+// takes those: 64 x 64 pixels 204 -> 151 us, 192 x 192 224 -> 171.
+constexpr int kWaves = 2, kWide = 8;
 constexpr float kPi = 3.14159265359f;      // CookTorranceBRDF.glsl:7
 constexpr float kOffset = 1e-4f;           // surface offset of secondary rays
 constexpr float kTwoPi = 2.0f * 3.14159265359f;  // Sampling.glsl:3
@@ -89,20 +91,20 @@ __device__ __forceinline__ f3 face_normal(const SceneArgs& s, int32_t tri, f3 di
 
 constexpr int kStackLds = 16;   // stack layout: entries a lane keeps in LDS
 
-template <int FORMAT>
+template <int FORMAT, int BLOCK>
 constexpr int stack_ints() {
-    return FORMAT == CRT_FORMAT_STACK ? kStackLds * kBlock : 1;
+    return FORMAT == CRT_FORMAT_STACK ? kStackLds * BLOCK : 1;
 }
 
 // The scene loop for one ray per lane (IntersectScene / its occlusion form,
 // TraverseBVHStackless.glsl:280-366, :558-579): the hit triangle or -1, its
 // distance in tmax.
-template <int FORMAT, bool ANY>
+template <int FORMAT, bool ANY, int BLOCK>
 __device__ __forceinline__ int32_t trace(const SceneArgs& s, f3 org, f3 dir, float& tmax, int32_t* lds) {
     constexpr int kSpill = FORMAT == CRT_FORMAT_STACK ? sdev::spill_entries<kStackLds>() : 1;
     int32_t spill[kSpill];
     walker::Walker<FORMAT, kStackLds> w;
-    w.init(lds, kBlock, spill);
+    w.init(lds, BLOCK, spill);
     w.tmax = tmax;
     int32_t hit = -1;
     for (int32_t i = 0; i < s.entity_count; ++i) {
@@ -136,12 +138,12 @@ __device__ __forceinline__ int32_t trace(const SceneArgs& s, f3 org, f3 dir, flo
     return hit;
 }
 
-template <int FORMAT>
+template <int FORMAT, int BLOCK>
 __device__ __forceinline__ bool visible(const SceneArgs& s, f3 x, f3 n, f3 light, int32_t* lds) {
     const f3 o = add(x, scale(n, kOffset));
     const f3 d = sub(light, o);
     float dist = sqrtf(dot(d, d));
-    return trace<FORMAT, true>(s, o, scale(d, 1.0f / dist), dist, lds) < 0;
+    return trace<FORMAT, true, BLOCK>(s, o, scale(d, 1.0f / dist), dist, lds) < 0;
 }
 
 // Cook-Torrance terms of one light at x: f_c = A * (kd * albedo_c + spec),
@@ -222,12 +224,13 @@ __device__ __forceinline__ int32_t claim(int32_t* counter) {
 
 __device__ __forceinline__ int32_t wave_id() { return __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x >> 6)); }
 
-template <int FORMAT>
-__global__ void __launch_bounds__(kBlock) forward_kernel(SceneArgs s, const crt_ray* __restrict__ rays,
-                                                         const crt_hit* __restrict__ hits, int64_t npix, Params P,
-                                                         uint32_t seed, float* __restrict__ color,
-                                                         crt_shade_record* __restrict__ rec) {
-    __shared__ int32_t stack[stack_ints<FORMAT>()];
+template <int FORMAT, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) forward_kernel(SceneArgs s, const crt_ray* __restrict__ rays,
+                                                             const crt_hit* __restrict__ hits, int64_t npix, Params P,
+                                                             uint32_t seed, float* __restrict__ color,
+                                                             crt_shade_record* __restrict__ rec) {
+    constexpr int BLOCK = 64 * WAVES;
+    __shared__ int32_t stack[stack_ints<FORMAT, BLOCK>()];
     __shared__ Tile tiles[2];
     int32_t* my = stack + (FORMAT == CRT_FORMAT_STACK ? threadIdx.x : 0);
     if (threadIdx.x < 4) tiles[threadIdx.x >> 1].next[threadIdx.x & 1] = 0;
@@ -272,7 +275,7 @@ __global__ void __launch_bounds__(kBlock) forward_kernel(SceneArgs s, const crt_
                     const f3 bd = normalize(add(add(scale(uu, rx), scale(vv, ry)), scale(n, rz)));
                     const f3 bo = add(p, scale(n, kOffset));
                     float t = 1000000.0f;
-                    t1 = trace<FORMAT, false>(s, bo, bd, t, my);
+                    t1 = trace<FORMAT, false, BLOCK>(s, bo, bd, t, my);
                     if (t1 >= 0) {
                         q = add(bo, scale(bd, t));
                         nq = face_normal(s, t1, bd);
@@ -286,7 +289,7 @@ __global__ void __launch_bounds__(kBlock) forward_kernel(SceneArgs s, const crt_
                 T.nq[1][lane] = nq.y;
                 T.nq[2][lane] = nq.z;
             } else {
-                const bool seen = t0 >= 0 && visible<FORMAT>(s, p, n, load3(P.lpos, k - 1), my);
+                const bool seen = t0 >= 0 && visible<FORMAT, BLOCK>(s, p, n, load3(P.lpos, k - 1), my);
                 const unsigned long long m = __ballot(seen);
                 if (lane == 0) T.vis_p[k - 1] = m;
             }
@@ -301,13 +304,13 @@ __global__ void __launch_bounds__(kBlock) forward_kernel(SceneArgs s, const crt_
         }
         // q to every light
         for (int32_t l = any ? claim(&T.next[1]) : P.nl; l < P.nl; l = claim(&T.next[1])) {
-            const bool seen = t1 >= 0 && visible<FORMAT>(s, q, nq, load3(P.lpos, l), my);
+            const bool seen = t1 >= 0 && visible<FORMAT, BLOCK>(s, q, nq, load3(P.lpos, l), my);
             const unsigned long long m = __ballot(seen);
             if (lane == 0) T.vis_q[l] = m;
         }
         __syncthreads();
         // one wave, another each time, writes the tile's records and colors; the others go on
-        if (wave_id() != turn % kWaves) continue;
+        if (wave_id() != turn % WAVES) continue;
         if (lane < 2) T.next[lane] = 0;
         if (i >= npix) continue;
         crt_shade_record out;
@@ -375,13 +378,18 @@ struct Gradients {
     float v[kSets][4];   // albedo, roughness
     int32_t tri[kSets];
 
-    __device__ __forceinline__ void clear() {
-        for (int k = threadIdx.x; k < kSets; k += kBlock) tri[k] = -1;
-    }
     __device__ __forceinline__ void flush(int k, float* __restrict__ g_albedo, float* __restrict__ g_rough) const {
         if (tri[k] < 0) return;
         for (int c = 0; c < 3; ++c) atomicAdd(g_albedo + 3 * int64_t(tri[k]) + c, v[k][c]);
         if (v[k][3] != 0.0f) atomicAdd(g_rough + tri[k], v[k][3]);
+    }
+    // Takes over entry k of another table.
+    __device__ __forceinline__ void merge(int k, const Gradients& o, float* __restrict__ g_albedo,
+                                          float* __restrict__ g_rough) {
+        if (o.tri[k] < 0) return;
+        if (tri[k] >= 0 && tri[k] != o.tri[k]) return o.flush(k, g_albedo, g_rough);
+        for (int c = 0; c < 4; ++c) v[k][c] = tri[k] < 0 ? o.v[k][c] : v[k][c] + o.v[k][c];
+        tri[k] = o.tri[k];
     }
     // One lane adds for triangle t.
     __device__ __forceinline__ void add(int32_t t, const float (&g)[4], float* __restrict__ g_albedo,
@@ -396,7 +404,7 @@ struct Gradients {
 
 // Adds v to the gradients of triangle idx (none below 0) for every lane; lanes
 // that share a triangle are summed in-wave first.  Called by all lanes of a
-// wave, by one wave of the workgroup at a time.
+// wave, by one wave at a time for the same table.
 __device__ __forceinline__ void wave_scatter_add(Gradients& G, int32_t idx, const float (&v)[4],
                                                  float* __restrict__ g_albedo, float* __restrict__ g_rough) {
     unsigned long long pending = __ballot(idx >= 0);
@@ -473,29 +481,46 @@ __device__ __forceinline__ void adjoint(const Params& P, const crt_shade_record&
     wave_scatter_add(G, t1, a1, g_albedo, g_rough);
 }
 
-// The intensity gradients, which every pixel adds to, leave each workgroup as
-// one global atomic per light instead of one per wave: the few addresses they
-// share are otherwise the kernel's bottleneck.
-template <int FORMAT>
-__global__ void __launch_bounds__(kBlock) backward_kernel(SceneArgs s, const crt_shade_record* __restrict__ rec,
-                                                          int64_t npix, Params P, const float* __restrict__ color,
-                                                          const float* __restrict__ target,
-                                                          float* __restrict__ g_albedo, float* __restrict__ g_rough,
-                                                          float* __restrict__ g_inten) {
-    __shared__ int32_t stack[stack_ints<FORMAT>()];
-    __shared__ Tile tiles[2];
-    __shared__ Gradients G;
+// Waits until every wave of a tile's group has come here `round` times; the
+// waves of a workgroup run at the same time, so each of them does.
+template <int WAVES>
+__device__ __forceinline__ void group_barrier(int32_t* arrived, int32_t round) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if (__lane_id() == 0) __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (__hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < round * WAVES)
+        __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// GROUPS tiles per workgroup, WAVES waves on each.  The sums that every pixel
+// adds to (a light's intensity, the triangles that cover the image) leave a
+// workgroup as one atomic each: one after the other at the same address, they
+// are the kernel's bottleneck when every wave sends its own, and each rounds
+// the growing sum once more, so few large workgroups are also more exact.
+template <int FORMAT, int WAVES, int GROUPS>
+__global__ void __launch_bounds__(64 * WAVES * GROUPS)
+backward_kernel(SceneArgs s, const crt_shade_record* __restrict__ rec, int64_t npix, Params P,
+                const float* __restrict__ color, const float* __restrict__ target, float* __restrict__ g_albedo,
+                float* __restrict__ g_rough, float* __restrict__ g_inten) {
+    constexpr int BLOCK = 64 * WAVES * GROUPS;
+    __shared__ int32_t stack[stack_ints<FORMAT, BLOCK>()];
+    __shared__ Tile tiles[GROUPS][2];
+    __shared__ Gradients G[GROUPS];
     __shared__ float inten_sum[kMaxLights];
+    __shared__ int32_t arrived[GROUPS];
     int32_t* my = stack + (FORMAT == CRT_FORMAT_STACK ? threadIdx.x : 0);
     if (threadIdx.x < unsigned(kMaxLights)) inten_sum[threadIdx.x] = 0.0f;
-    if (threadIdx.x < 2) tiles[threadIdx.x].next[0] = 0;
-    G.clear();
+    if (threadIdx.x < 2 * GROUPS) tiles[threadIdx.x >> 1][threadIdx.x & 1].next[0] = 0;
+    if (threadIdx.x < GROUPS) arrived[threadIdx.x] = 0;
+    for (int k = threadIdx.x; k < GROUPS * Gradients::kSets; k += BLOCK)
+        G[k / Gradients::kSets].tri[k % Gradients::kSets] = -1;
     __syncthreads();
     const uint32_t lane = __lane_id();
+    const int32_t group = wave_id() / WAVES, wave = wave_id() % WAVES;
     const int64_t ntiles = (npix + 63) / 64;
     int32_t turn = 0;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, ++turn) {
-        Tile& T = tiles[turn & 1];
+    for (int64_t tile = int64_t(group) * gridDim.x + blockIdx.x; tile < ntiles; tile += int64_t(gridDim.x) * GROUPS, ++turn) {
+        Tile& T = tiles[group][turn & 1];
         const int64_t i = tile * 64 + lane;
         // every field is initialized: with some left undefined for the lanes past
         // the end, the compiler may assume that there are none and drop the bound
@@ -511,33 +536,71 @@ __global__ void __launch_bounds__(kBlock) backward_kernel(SceneArgs s, const crt
             const float* x = first ? R.p : R.q;
             const float* xn = first ? R.n : R.nq;
             const bool seen = (first ? valid : again) &&
-                              visible<FORMAT>(s, mk(x[0], x[1], x[2]), mk(xn[0], xn[1], xn[2]), load3(P.lpos, l), my);
+                              visible<FORMAT, BLOCK>(s, mk(x[0], x[1], x[2]), mk(xn[0], xn[1], xn[2]), load3(P.lpos, l), my);
             const unsigned long long m = __ballot(seen);
             if (lane == 0) (first ? T.vis_p : T.vis_q)[l] = m;
         }
-        __syncthreads();
+        if constexpr (GROUPS == 1)
+            __syncthreads();
+        else
+            group_barrier<WAVES>(&arrived[group], turn + 1);
         // one wave, another each time, takes the tile's gradients; the others go on
-        if (wave_id() != turn % kWaves) continue;
+        if (wave != turn % WAVES) continue;
         if (lane == 0) T.next[0] = 0;
-        if (any) adjoint(P, R, i, T, color, target, g_albedo, g_rough, G, inten_sum);
+        if (any) adjoint(P, R, i, T, color, target, g_albedo, g_rough, G[group], inten_sum);
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < Gradients::kSets; k += kBlock) G.flush(k, g_albedo, g_rough);
+    for (int k = threadIdx.x; k < Gradients::kSets; k += BLOCK) {
+        for (int g = 1; g < GROUPS; ++g) G[0].merge(k, G[g], g_albedo, g_rough);
+        G[0].flush(k, g_albedo, g_rough);
+    }
     if (threadIdx.x < unsigned(P.nl)) atomicAdd(g_inten + threadIdx.x, inten_sum[threadIdx.x]);
 }
 
-// Workgroups that fill the device once, or one per tile where there are fewer.
+// Workgroups of `block` threads that fill the device once.
 template <typename F>
-unsigned tile_grid(F kernel, int64_t npix) {
+int64_t resident(F kernel, int block) {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), kBlock, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), block, 0) !=
             hipSuccess || per_cu <= 0)
-        per_cu = 4;
+        per_cu = 1;
+    return int64_t(cus) * per_cu;
+}
+
+template <int FORMAT>
+void launch_forward(const SceneArgs& s, const crt_ray* rays, const crt_hit* hits, int64_t npix, const Params& P,
+                    uint32_t seed, float* color, crt_shade_record* rec, hipStream_t st) {
     const int64_t tiles = (npix + 63) / 64;
-    return unsigned(tiles < int64_t(cus) * per_cu ? tiles : int64_t(cus) * per_cu);
+    const auto wide = forward_kernel<FORMAT, kWide>;
+    const auto fn = forward_kernel<FORMAT, kWaves>;
+    if (tiles <= resident(wide, 64 * kWide)) {
+        hipLaunchKernelGGL(wide, dim3(unsigned(tiles)), dim3(64 * kWide), 0, st, s, rays, hits, npix, P, seed, color, rec);
+        return;
+    }
+    const int64_t grid = resident(fn, 64 * kWaves);
+    hipLaunchKernelGGL(fn, dim3(unsigned(tiles < grid ? tiles : grid)), dim3(64 * kWaves), 0, st, s, rays, hits, npix, P,
+                       seed, color, rec);
+}
+
+template <int FORMAT>
+void launch_backward(const SceneArgs& s, const crt_shade_record* rec, int64_t npix, const Params& P,
+                     const float* color, const float* target, float* g_albedo, float* g_rough, float* g_inten,
+                     hipStream_t st) {
+    constexpr int kGroups = kWide / kWaves;
+    const int64_t tiles = (npix + 63) / 64;
+    const auto wide = backward_kernel<FORMAT, kWide, 1>;
+    const auto fn = backward_kernel<FORMAT, kWaves, kGroups>;
+    if (tiles <= resident(wide, 64 * kWide)) {
+        hipLaunchKernelGGL(wide, dim3(unsigned(tiles)), dim3(64 * kWide), 0, st, s, rec, npix, P, color, target,
+                           g_albedo, g_rough, g_inten);
+        return;
+    }
+    const int64_t grid = resident(fn, 64 * kWide), need = (tiles + kGroups - 1) / kGroups;
+    hipLaunchKernelGGL(fn, dim3(unsigned(need < grid ? need : grid)), dim3(64 * kWide), 0, st, s, rec, npix, P, color,
+                       target, g_albedo, g_rough, g_inten);
 }
 
 }  // namespace shade
@@ -573,10 +636,11 @@ int crt_shade_forward(const crt_scene_view* scene, const crt_ray* primary_rays, 
     if (npix < 0 || (npix > 0 && (!primary_rays || !primary_hits || !color || !records)))
         return crt::set_error(CRT_E_INVALID, "crt_shade_forward: bad buffers");
     if (npix == 0) return CRT_OK;
-    const auto fn = a.format == CRT_FORMAT_STACKLESS ? crt::shade::forward_kernel<CRT_FORMAT_STACKLESS>
-                                                     : crt::shade::forward_kernel<CRT_FORMAT_STACK>;
-    hipLaunchKernelGGL(fn, dim3(crt::shade::tile_grid(fn, npix)), dim3(crt::shade::kBlock), 0,
-                       static_cast<hipStream_t>(stream), a, primary_rays, primary_hits, npix, p, seed, color, records);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (a.format == CRT_FORMAT_STACKLESS)
+        crt::shade::launch_forward<CRT_FORMAT_STACKLESS>(a, primary_rays, primary_hits, npix, p, seed, color, records, st);
+    else
+        crt::shade::launch_forward<CRT_FORMAT_STACK>(a, primary_rays, primary_hits, npix, p, seed, color, records, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return crt::set_error(CRT_E_HIP, std::string("crt_shade_forward: ") + hipGetErrorString(e));
     return CRT_OK;
@@ -593,11 +657,13 @@ int crt_shade_backward(const crt_scene_view* scene, const crt_shade_record* reco
                                   !grad_intensity)))
         return crt::set_error(CRT_E_INVALID, "crt_shade_backward: bad buffers");
     if (npix == 0) return CRT_OK;
-    const auto fn = a.format == CRT_FORMAT_STACKLESS ? crt::shade::backward_kernel<CRT_FORMAT_STACKLESS>
-                                                     : crt::shade::backward_kernel<CRT_FORMAT_STACK>;
-    hipLaunchKernelGGL(fn, dim3(crt::shade::tile_grid(fn, npix)), dim3(crt::shade::kBlock), 0,
-                       static_cast<hipStream_t>(stream), a, records, npix, p, color, target, grad_albedo,
-                       grad_roughness, grad_intensity);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (a.format == CRT_FORMAT_STACKLESS)
+        crt::shade::launch_backward<CRT_FORMAT_STACKLESS>(a, records, npix, p, color, target, grad_albedo,
+                                                          grad_roughness, grad_intensity, st);
+    else
+        crt::shade::launch_backward<CRT_FORMAT_STACK>(a, records, npix, p, color, target, grad_albedo, grad_roughness,
+                                                      grad_intensity, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return crt::set_error(CRT_E_HIP, std::string("crt_shade_backward: ") + hipGetErrorString(e));
     return CRT_OK;
