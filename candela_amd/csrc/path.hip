@@ -450,23 +450,23 @@ struct PathSpecWave {
         }
     }
 
+    template <typename Queue>
     __device__ __forceinline__ void run(const SceneArgs& s, const Params& P, int64_t npaths, float tmax,
                                         int32_t max_iter, Stack<LDS_DEPTH> st, spec::WaveLds<Q>& L,
-                                        unsigned long long* __restrict__ counters, int32_t refill,
-                                        crt_path_sample* __restrict__ out) {
+                                        Queue q, int32_t refill, crt_path_sample* __restrict__ out) {
         w.active = false;
         w.walk_done = false;
         w.nq = 0;
-        ShardQueue q;
-        q.init(counters, npaths);
+        const int32_t takers = __popcll(q.lanes);
+        refill = takers < refill ? takers : refill;
         while (true) {
             if (q.more) {
-                const unsigned long long idle = __ballot(!w.active);
+                const unsigned long long idle = __ballot(!w.active) & q.lanes;
                 const int32_t cnt = __popcll(idle);
                 if (cnt >= refill) {
                     int32_t got = 0;
                     const int64_t first = q.claim(cnt, got);
-                    if (!w.active) {
+                    if (!w.active && (q.lanes >> __lane_id() & 1ull)) {
                         const int32_t rank = spec::lanes_below(idle);
                         if (rank < got) start_path(s, P, q.at(first + rank), tmax, out);
                     }
@@ -492,10 +492,12 @@ struct SpecPathLds {
     spec::WaveLds<spec_queue_slots<W, Q>()> waves[4];
 };
 
-template <int W, int LDS_DEPTH, int INNER, int Q, int REFILL, int OCC>
+// DIRECT: the paths all fit the launch (queue.h: DirectQueue).
+template <int W, int LDS_DEPTH, int INNER, int Q, int REFILL, int OCC, bool DIRECT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1, 8)))
 spec_path_kernel(SceneArgs s, Params P, int64_t npaths, float tmax, int32_t max_iter,
-                 unsigned long long* __restrict__ counters, crt_path_sample* __restrict__ out) {
+                 unsigned long long* __restrict__ counters, crt_path_sample* __restrict__ out, int32_t log2,
+                 int32_t blocks) {
     __shared__ SpecPathLds<W, LDS_DEPTH, Q> lds;
     int32_t spill_node[wide::kSpill];
     float spill_t[wide::kSpill];
@@ -505,7 +507,16 @@ spec_path_kernel(SceneArgs s, Params P, int64_t npaths, float tmax, int32_t max_
     st.spill_node = spill_node;
     st.spill_t = spill_t;
     PathSpecWave<W, LDS_DEPTH, INNER, spec_queue_slots<W, Q>()> pw;
-    pw.run(s, P, npaths, tmax, max_iter, st, lds.waves[threadIdx.x >> 6], counters, REFILL, out);
+    spec::WaveLds<spec_queue_slots<W, Q>()>& wave = lds.waves[threadIdx.x >> 6];
+    if constexpr (DIRECT) {
+        DirectQueue q;
+        q.init(npaths, log2, blocks);
+        pw.run(s, P, npaths, tmax, max_iter, st, wave, q, REFILL, out);
+    } else {
+        ShardQueue q;
+        q.init(counters, npaths);
+        pw.run(s, P, npaths, tmax, max_iter, st, wave, q, REFILL, out);
+    }
 }
 
 template <int W, int D, int I, int LB, int R, int OCC>
@@ -535,12 +546,13 @@ const void* path_kernel_ptr() {
     X(8, 8, 4, 8, 16, 5)         \
     X(9, 8, 8, 8, 8, 5)
 
-template <int W>
+// DIRECT is for the speculative presets; the others have no such form.
+template <int W, bool DIRECT>
 const void* path_fn(int variant) {
 #define CRT_PATH_FN(V, D, I, LB, R, OCC) \
     case V: return path_kernel_ptr<W, D, I, LB, R, OCC>();
 #define CRT_SPEC_PATH_FN(V, D, I, Q, R, OCC) \
-    case V: return reinterpret_cast<const void*>(&spec_path_kernel<W, D, I, Q, R, OCC>);
+    case V: return reinterpret_cast<const void*>(&spec_path_kernel<W, D, I, Q, R, OCC, DIRECT>);
     switch (variant) {
         CRT_PATH_PRESETS(CRT_PATH_FN)
         CRT_SPEC_PATH_PRESETS(CRT_SPEC_PATH_FN)
@@ -590,30 +602,42 @@ extern "C" int crt_trace_paths(const crt_scene_view* scene, const crt_path_param
     int rc = crt::queue_acquire(config, stream, "crt_trace_paths", lease);
     if (rc) return rc;
     unsigned long long* counters = lease.ptr;
-    const void* fn = scene->format == CRT_FORMAT_WIDE8 ? crt::path::path_fn<8>(variant) : crt::path::path_fn<4>(variant);
+    const void* fn = scene->format == CRT_FORMAT_WIDE8 ? crt::path::path_fn<8, false>(variant)
+                                                           : crt::path::path_fn<4, false>(variant);
     int grid = config && config->grid > 0 ? config->grid : 0;
-    if (grid == 0) {
+    const bool own_grid = grid == 0;
+    if (own_grid) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess) dev = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0) != hipSuccess || per_cu <= 0) per_cu = 4;
         grid = cus * per_cu;
     }
-    const int64_t need = (npaths + 255) / 256;
-    if (need < grid) grid = int(need);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(crt::reset_queue, dim3(1), dim3(64), 0, st, counters);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        (void)crt::queue_release(lease, stream);
-        return crt::set_error(CRT_E_HIP, std::string("crt_trace_paths: reset: ") + hipGetErrorString(e));
+    int32_t log2 = 6, blocks = 0;
+    hipError_t e;
+    if (own_grid && variant >= 6 && npaths <= int64_t(grid) * 256) {
+        // a lane for every path: nothing to refill
+        fn = scene->format == CRT_FORMAT_WIDE8 ? crt::path::path_fn<8, true>(variant) : crt::path::path_fn<4, true>(variant);
+        log2 = crt::rays_per_wave_log2(npaths, crt::kSpecWaves);
+        blocks = crt::wave_blocks(npaths, log2);
+        grid = (blocks + 7) / 8 * 8;
+    } else {
+        const int64_t need = (npaths + 255) / 256;
+        if (need < grid) grid = int(need);
+        hipLaunchKernelGGL(crt::reset_queue, dim3(1), dim3(64), 0, st, counters);
+        e = hipGetLastError();
+        if (e != hipSuccess) {
+            (void)crt::queue_release(lease, stream);
+            return crt::set_error(CRT_E_HIP, std::string("crt_trace_paths: reset: ") + hipGetErrorString(e));
+        }
     }
     crt::SceneArgs a = crt::scene_args(*scene);
     int64_t n = npaths;
     float tmax = p.tmax;
     int32_t max_iter = crt::kMaxIterations;
     crt_path_sample* o = out;
-    void* args[] = {&a, &P, &n, &tmax, &max_iter, &counters, &o};
+    void* args[] = {&a, &P, &n, &tmax, &max_iter, &counters, &o, &log2, &blocks};   // (the others take 7)
     e = hipLaunchKernel(fn, dim3(unsigned(grid)), dim3(256), args, 0, st);
     rc = crt::queue_release(lease, stream);
     if (e != hipSuccess) return crt::set_error(CRT_E_HIP, std::string("crt_trace_paths: launch: ") + hipGetErrorString(e));

@@ -36,6 +36,7 @@ struct ShardQueue {
     int32_t shard, visited, cshard;
     bool strided;   // shard k holds k, k + kQueueShards, ... instead of a contiguous range
     bool more;      // wave-uniform: some shard may still hold indices
+    static constexpr unsigned long long lanes = ~0ull;   // those that take indices
 
     __device__ __forceinline__ void init(unsigned long long* c, int64_t total, bool stride_shards = false,
                                          int32_t shards = kQueueShards) {
@@ -91,6 +92,33 @@ struct ShardQueue {
     __device__ __forceinline__ int64_t at(int64_t pos) const {
         return strided ? int64_t(cshard) + int64_t(nsh) * pos : lo(cshard) + pos;
     }
+};
+
+// The same for launches whose indices all fit the device's waves at once: they
+// are dealt out like a grid launch's, fewer than 64 to a wave when there are few
+// (rays_per_wave_log2), and a wave's first claim is its only one.  A sharded
+// queue costs each wave an atomic round trip per shard until it is found dry,
+// and the launch one more to reset it.
+struct DirectQueue {
+    int64_t n, base;
+    unsigned long long lanes;
+    bool more;
+
+    // Workgroups of four waves, `blocks` of which hold work; the grid is padded to a multiple of 8.
+    __device__ __forceinline__ void init(int64_t total, int32_t log2, int32_t blocks) {
+        const int32_t wave = __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x >> 6));
+        const int32_t logical = int32_t(blockIdx.x % 8u) * ((blocks + 7) / 8) + int32_t(blockIdx.x / 8u);
+        n = total;
+        lanes = log2 >= 6 ? ~0ull : (1ull << (1 << log2)) - 1;
+        base = (int64_t(logical) * 4 + wave) << log2;
+        more = logical < blocks && base < total;
+    }
+    __device__ __forceinline__ int64_t claim(int32_t want, int32_t& got) {
+        more = false;
+        got = n - base < want ? int32_t(n - base) : want;
+        return base;
+    }
+    __device__ __forceinline__ int64_t at(int64_t pos) const { return pos; }
 };
 
 }  // namespace crt

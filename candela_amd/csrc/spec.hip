@@ -35,12 +35,9 @@ struct GroupLds {
 template <bool ANY, int W, int D, int I, int Q>
 __device__ __forceinline__ void grid_body(const SceneArgs& s, const crt_ray* __restrict__ rays,
                                           crt_hit* __restrict__ hits, int64_t n, uint32_t flags, int32_t max_iter,
-                                          uint32_t* __restrict__ tri_tests, int32_t blocks,
+                                          uint32_t* __restrict__ tri_tests, int32_t log2, int32_t blocks,
                                           GroupLds<W, D, Q>& lds) {
-    const int32_t per = (blocks + 7) / 8;  // the grid is padded to a multiple of 8
-    const int32_t logical = int32_t(blockIdx.x % 8u) * per + int32_t(blockIdx.x / 8u);
-    if (logical >= blocks) return;
-    const int64_t i = int64_t(logical) * 256 + threadIdx.x;
+    const int64_t i = grid_ray(n, log2, blocks);
     int32_t spill_node[wide::kSpill];
     float spill_t[wide::kSpill];
     wide::Stack<D> st;
@@ -49,22 +46,23 @@ __device__ __forceinline__ void grid_body(const SceneArgs& s, const crt_ray* __r
     st.spill_node = spill_node;
     st.spill_t = spill_t;
     spec::SpecWave<ANY, W, D, I, queue_slots<W, Q>()> w;
-    w.run(s, rays, hits, i < n ? i : -1, flags, max_iter, tri_tests, st, lds.waves[threadIdx.x >> 6]);
+    w.run(s, rays, hits, i, flags, max_iter, tri_tests, st, lds.waves[threadIdx.x >> 6]);
 }
 
 template <bool ANY, int W, int D, int I, int Q, int OCC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1, 8)))
 spec_grid(SceneArgs s, const crt_ray* __restrict__ rays, crt_hit* __restrict__ hits, int64_t n, uint32_t flags,
-          int32_t max_iter, uint32_t* __restrict__ tri_tests, int32_t blocks) {
+          int32_t max_iter, uint32_t* __restrict__ tri_tests, int32_t log2, int32_t blocks) {
     __shared__ GroupLds<W, D, Q> lds;
-    grid_body<ANY, W, D, I, Q>(s, rays, hits, n, flags, max_iter, tri_tests, blocks, lds);
+    grid_body<ANY, W, D, I, Q>(s, rays, hits, n, flags, max_iter, tri_tests, log2, blocks, lds);
 }
 
-template <bool ANY, int W, int D, int I, int Q, int REFILL, int OCC>
+// DIRECT: the rays all fit the launch (queue.h: DirectQueue).
+template <bool ANY, int W, int D, int I, int Q, int REFILL, int OCC, bool DIRECT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1, 8)))
 spec_persistent(SceneArgs s, const crt_ray* __restrict__ rays, crt_hit* __restrict__ hits, int64_t n,
                 uint32_t flags, int32_t max_iter, uint32_t* __restrict__ tri_tests,
-                unsigned long long* __restrict__ counters) {
+                unsigned long long* __restrict__ counters, int32_t log2, int32_t blocks) {
     __shared__ GroupLds<W, D, Q> lds;
     int32_t spill_node[wide::kSpill];
     float spill_t[wide::kSpill];
@@ -74,7 +72,16 @@ spec_persistent(SceneArgs s, const crt_ray* __restrict__ rays, crt_hit* __restri
     st.spill_node = spill_node;
     st.spill_t = spill_t;
     spec::SpecWave<ANY, W, D, I, queue_slots<W, Q>()> w;
-    w.run_refill(s, rays, hits, n, flags, max_iter, tri_tests, st, lds.waves[threadIdx.x >> 6], counters, REFILL);
+    spec::WaveLds<queue_slots<W, Q>()>& wave = lds.waves[threadIdx.x >> 6];
+    if constexpr (DIRECT) {
+        DirectQueue q;
+        q.init(n, log2, blocks);
+        w.run_refill(s, rays, hits, n, flags, max_iter, tri_tests, st, wave, q, REFILL);
+    } else {
+        ShardQueue q;
+        q.init(counters, n);
+        w.run_refill(s, rays, hits, n, flags, max_iter, tri_tests, st, wave, q, REFILL);
+    }
 }
 
 }  // namespace sp
@@ -111,10 +118,10 @@ static const void* spec_grid_fn(int variant) {
 #undef CRT_SPEC_G_FN
 }
 
-template <bool ANY, int W>
+template <bool ANY, int W, bool DIRECT>
 static const void* spec_persistent_fn(int variant) {
 #define CRT_SPEC_P_FN(V, D, I, Q, R, OCC) \
-    case V: return reinterpret_cast<const void*>(&sp::spec_persistent<ANY, W, D, I, Q, R, OCC>);
+    case V: return reinterpret_cast<const void*>(&sp::spec_persistent<ANY, W, D, I, Q, R, OCC, DIRECT>);
     switch (variant) {
         CRT_SPEC_P_PRESETS(CRT_SPEC_P_FN)
         default: return nullptr;
@@ -122,21 +129,27 @@ static const void* spec_persistent_fn(int variant) {
 #undef CRT_SPEC_P_FN
 }
 
-static const void* pick(bool persistent, int format, int query, int variant) {
+static const void* grid_pick(int format, int query, int variant) {
+    const bool any = query == CRT_QUERY_ANY;
+    if (format == CRT_FORMAT_WIDE8) return any ? spec_grid_fn<true, 8>(variant) : spec_grid_fn<false, 8>(variant);
+    return any ? spec_grid_fn<true, 4>(variant) : spec_grid_fn<false, 4>(variant);
+}
+
+template <bool DIRECT>
+static const void* persistent_pick(int format, int query, int variant) {
     const bool any = query == CRT_QUERY_ANY;
     if (format == CRT_FORMAT_WIDE8)
-        return persistent ? (any ? spec_persistent_fn<true, 8>(variant) : spec_persistent_fn<false, 8>(variant))
-                          : (any ? spec_grid_fn<true, 8>(variant) : spec_grid_fn<false, 8>(variant));
-    return persistent ? (any ? spec_persistent_fn<true, 4>(variant) : spec_persistent_fn<false, 4>(variant))
-                      : (any ? spec_grid_fn<true, 4>(variant) : spec_grid_fn<false, 4>(variant));
+        return any ? spec_persistent_fn<true, 8, DIRECT>(variant) : spec_persistent_fn<false, 8, DIRECT>(variant);
+    return any ? spec_persistent_fn<true, 4, DIRECT>(variant) : spec_persistent_fn<false, 4, DIRECT>(variant);
 }
 
 hipError_t launch_spec_grid(const SceneArgs& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                             uint32_t flags, int32_t max_iter, uint32_t* tri_tests, int variant, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    const void* fn = pick(false, s.format, query, variant);
+    const void* fn = grid_pick(s.format, query, variant);
     if (!fn) return hipErrorInvalidValue;
-    int32_t blocks = int32_t((n + 255) / 256);
+    int32_t log2 = rays_per_wave_log2(n, kSpecWaves);
+    int32_t blocks = wave_blocks(n, log2);
     const unsigned padded = unsigned((blocks + 7) / 8 * 8);
     SceneArgs sa = s;
     const crt_ray* r = rays;
@@ -145,7 +158,7 @@ hipError_t launch_spec_grid(const SceneArgs& s, int query, const crt_ray* rays, 
     uint32_t fl = flags;
     int32_t mi = max_iter;
     uint32_t* tt = tri_tests;
-    void* args[] = {&sa, &r, &h, &nn, &fl, &mi, &tt, &blocks};
+    void* args[] = {&sa, &r, &h, &nn, &fl, &mi, &tt, &log2, &blocks};
     const hipError_t e = hipLaunchKernel(fn, dim3(padded), dim3(256), args, 0, stream);
     if (e != hipSuccess) return e;
     return hipGetLastError();
@@ -155,9 +168,11 @@ hipError_t launch_spec_persistent(const SceneArgs& s, int query, const crt_ray* 
                                   uint32_t flags, int32_t max_iter, unsigned long long* counters,
                                   uint32_t* tri_tests, int variant, int grid, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    const void* fn = pick(true, s.format, query, variant);
+    const void* fn = persistent_pick<false>(s.format, query, variant);
     if (!fn) return hipErrorInvalidValue;
-    if (grid <= 0) {
+    int32_t log2 = 6, blocks = 0;
+    const bool own_grid = grid <= 0;
+    if (own_grid) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess) dev = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -165,11 +180,20 @@ hipError_t launch_spec_persistent(const SceneArgs& s, int query, const crt_ray* 
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0) != hipSuccess || per_cu <= 0) per_cu = 4;
         grid = cus * per_cu;
     }
-    const int64_t need = (n + 255) / 256;
-    if (need < grid) grid = int(need);
-    hipLaunchKernelGGL(reset_queue, dim3(1), dim3(64), 0, stream, counters);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipError_t e;
+    if (own_grid && n <= int64_t(grid) * 256) {
+        // a lane for every ray: nothing to refill
+        fn = persistent_pick<true>(s.format, query, variant);
+        log2 = rays_per_wave_log2(n, kSpecWaves);
+        blocks = wave_blocks(n, log2);
+        grid = (blocks + 7) / 8 * 8;
+    } else {
+        const int64_t need = (n + 255) / 256;
+        if (need < grid) grid = int(need);
+        hipLaunchKernelGGL(reset_queue, dim3(1), dim3(64), 0, stream, counters);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     SceneArgs sa = s;
     const crt_ray* r = rays;
     crt_hit* h = hits;
@@ -178,7 +202,7 @@ hipError_t launch_spec_persistent(const SceneArgs& s, int query, const crt_ray* 
     int32_t mi = max_iter;
     uint32_t* tt = tri_tests;
     unsigned long long* c = counters;
-    void* args[] = {&sa, &r, &h, &nn, &fl, &mi, &tt, &c};
+    void* args[] = {&sa, &r, &h, &nn, &fl, &mi, &tt, &c, &log2, &blocks};
     e = hipLaunchKernel(fn, dim3(unsigned(grid)), dim3(256), args, 0, stream);
     if (e != hipSuccess) return e;
     return hipGetLastError();

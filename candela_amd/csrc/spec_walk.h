@@ -439,26 +439,27 @@ struct SpecWave {
         while (__ballot(active)) round(s, rays, hits, flags, max_iter, tri_tests, st, L);
     }
 
-    // Rays [0, n) claimed from the sharded queue between rounds, one per idle
-    // lane, once at least `refill` lanes are idle.
+    // Rays [0, n) claimed from the queue between rounds, one per idle lane of
+    // those that take rays, once at least `refill` of them (or all) are idle.
+    template <typename Queue>
     __device__ __forceinline__ void run_refill(const SceneArgs& s, const crt_ray* __restrict__ rays,
                                                crt_hit* __restrict__ hits, int64_t n, uint32_t flags,
                                                int32_t max_iter, uint32_t* __restrict__ tri_tests,
                                                Stack<LDS_DEPTH> st, WaveLds<Q>& L,
-                                               unsigned long long* __restrict__ counters, int32_t refill) {
+                                               Queue q, int32_t refill) {
         active = false;
         walk_done = false;
         nq = 0;
-        ShardQueue q;
-        q.init(counters, n);
+        const int32_t takers = __popcll(q.lanes);
+        refill = takers < refill ? takers : refill;
         while (true) {
             if (q.more) {
-                const unsigned long long idle = __ballot(!active);
+                const unsigned long long idle = __ballot(!active) & q.lanes;
                 const int32_t cnt = __popcll(idle);
                 if (cnt >= refill) {
                     int32_t got = 0;
                     const int64_t first = q.claim(cnt, got);
-                    if (!active) {
+                    if (!active && (q.lanes >> __lane_id() & 1ull)) {
                         const int32_t rank = lanes_below(idle);
                         if (rank < got) begin_ray(s, rays, hits, q.at(first + rank), flags, tri_tests);
                     }

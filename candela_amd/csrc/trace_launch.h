@@ -120,11 +120,18 @@ hipError_t launch_stack_persistent(const SceneArgs& s, int query, const crt_ray*
 // one ray a wave, 31 with 4 and 40 with 64; 5,976 primary rays 102, 123 and 153;
 // 41,736 bounce rays, with 8, 78 against 90.  More waves than fit only add up:
 // 59,000 rays take 66 us with 16 a wave, 83 with 4 and 166 with one.
-inline int32_t rays_per_wave_log2(int64_t n) {
+inline int32_t rays_per_wave_log2(int64_t n, int64_t waves = 6144) {
     int32_t k = 0;
-    while (k < 6 && (n >> k) > 6144) ++k;
+    while (k < 6 && (n >> k) > waves) ++k;
     return k;
 }
+// The speculative walks want fewer waves: they test the leaves of all their rays
+// together.  Occlusion and bounce rays of an 86 x 85 image 141 us with 64 rays a
+// wave, 122 over 1,024 waves, 114 over 2,048, 108 over 3,072; of 423 x 384
+// pixels 144, 126, 124 and 133.
+constexpr int64_t kSpecWaves = 2048;
+// Workgroups of four waves that n rays then take.
+inline int32_t wave_blocks(int64_t n, int32_t log2) { return int32_t((n + (4 << log2) - 1) >> (log2 + 2)); }
 
 // Ray of a grid launch's lane (workgroups of four waves, dealt to the XCDs so
 // that consecutive ones share an L2; the grid is padded to a multiple of 8), or
