@@ -62,10 +62,11 @@ hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* ver
 }
 
 // LDS stack entries, node steps per round, parked lanes that end the node
-// phase.  12 entries (24 KB a workgroup) leave the 6 waves per SIMD that the
-// registers allow.  Measured on 347,053 bounce rays over 640,000 triangles: 255.6 us
-// with (4, 16) and (4, 8), 261.5 with (8, 8), 274 with (2, 8).
-#define CRT_PAIR_SHAPE 12, 4, 16
+// phase.  10 entries (20 KB a workgroup) leave the 7 waves per SIMD that the
+// registers allow: 1920 x 1080 primary rays over 640,000 triangles take 332 us, with
+// 12 entries (6 waves) 355.  347,053 bounce rays: 256 us with (4, 16) and (4, 8),
+// 261 with (8, 8), 274 with (2, 8).
+#define CRT_PAIR_SHAPE 10, 4, 16
 
 hipError_t launch_pair_grid(const PairScene& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                             uint32_t flags, int32_t max_iter, hipStream_t stream) {

@@ -31,7 +31,7 @@
 // Bound: the chain of a wave's longest ray (511 visits among the bounce rays
 // below, 0.3 us a visit when alone), then VALU issue.  Measured against the
 // walk of the stackless array: 347,053 bounce rays over 640,000 triangles 541 ->
-// 270 us, 1920 x 1080 primary rays of the same scene 676 -> 372 us (with 8 x 8
+// 270 us, 1920 x 1080 primary rays of the same scene 676 -> 350 us (with 8 x 8
 // pixels a wave), 300 rays over 3,074 triangles 58 -> 37 us.  Both loads of a
 // pair have to be in flight at once (pin): with the right box loaded behind
 // the left one's branch, where the compiler moves it, the same walk takes 466,

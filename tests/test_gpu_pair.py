@@ -75,7 +75,7 @@ def along_z(crt, n):
 
 
 @pytest.mark.parametrize("right", [False, True], ids=["left", "right"])
-@pytest.mark.parametrize("depth", [1, 11, 12, 13, 40, 64, 65, 200])
+@pytest.mark.parametrize("depth", [1, 9, 10, 11, 12, 13, 40, 64, 65, 200])
 def test_depths(crt, depth, right):
     """Around the stack's LDS part, its end and the depth from which the array itself is walked."""
     r = context(crt, [chain(crt, depth, right)], [0])
