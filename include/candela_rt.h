@@ -640,7 +640,12 @@ int crt_make_entity(const float model[16], float emissive, float translucency, i
                     int32_t node_count, crt_entity* out);
 /* BufferEntities (Intersector.h:226-239) */
 int crt_buffer_entities(crt_context* ctx);
-/* BufferData (Intersector.h:321-351) */
+/* BufferData (Intersector.h:321-351).  Also lays out what crt_intersect and
+ * crt_intersect_primary walk instead of the buffers themselves, with the same
+ * visits and records: one record per triangle, and the child pairs of a
+ * stackless tree (half as much device memory again as the buffers, more or
+ * less; left out where the nodes are no plain tree or memory is short).  The
+ * memory behind the context's scene view is for reading only. */
 int crt_buffer_data(crt_context* ctx, int clear_cpu_data);
 
 /* Host copies (the public m_BVHNodes / m_BVHVertices / m_BVHTriangles /
