@@ -26,7 +26,9 @@
 // again with `exact` set.  Then, and in an any-hit walk, which ends with
 // pending children unvisited, a right child is kept hit or not while its left
 // sibling's subtree is walked, and counted and checked against the cap when
-// its turn comes.
+// its turn comes.  A ray is walked in one of the two ways from its start to its
+// end, whatever the other lanes of its wave do: what one has counted and kept,
+// the other cannot go on from.
 //
 // Bound: the chain of a wave's longest ray (511 visits among the bounce rays
 // below, 0.3 us a visit when alone), then VALU issue.  Measured against the
@@ -292,14 +294,11 @@ struct PairWave {
     // One round of the wave: node phase, leaf phase, walk ends.
     __device__ __forceinline__ void round(const PairScene& s, const crt_ray* rays, crt_hit* __restrict__ hits,
                                           uint32_t flags, int32_t max_iter, PairStack<D>& st) {
-        const bool in_order = ANY || __any(exact && ref != kIdle);
+        // every lane by its own `exact`: the two count and keep pending children differently
+        const bool some_exact = ANY || __any(exact && ref != kIdle);
         for (int k = 0; k < INNER; ++k) {
-            if (stepping()) {
-                if (in_order)
-                    step_in_order(s, max_iter, st);
-                else
-                    step(s, max_iter, st);
-            }
+            if (!ANY && stepping() && !exact) step(s, max_iter, st);
+            if (some_exact && stepping() && (ANY || exact)) step_in_order(s, max_iter, st);
             if (!__any(stepping()) || __popcll(__ballot(leafing())) >= LEAF_BATCH) break;
         }
         if (leafing()) {

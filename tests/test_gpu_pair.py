@@ -109,6 +109,50 @@ def test_iteration_cap(crt, leaves, per_leaf):
     assert ((hits["status"] & crt.STATUS_ITER_CAP) != 0).any() == (leaves > 512)
 
 
+def patchy(crt, leaves, seed):
+    """A complete tree whose boxes each cover a part of x at random, the middle always: rays visit from a few hundred
+    to all of its nodes.  The triangles cover every ray, each nearer than those before it."""
+    nodes, tris, verts = balanced(crt, leaves, 1)
+    rng = np.random.default_rng(seed)
+    nodes["min"][1:, 0] = rng.uniform(-0.2, 0.0, nodes.size - 1)
+    nodes["max"][1:, 0] = rng.uniform(0.0, 0.2, nodes.size - 1)
+    corners = np.array([(-9, -9, 0), (9, -9, 0), (0, 18, 0)], np.float32)
+    pos = np.repeat(corners[None], leaves, axis=0)
+    pos[:, :, 2] = 7 - np.arange(leaves, dtype=np.float32)[:, None] / leaves
+    verts["position"][:, :3] = pos.reshape(-1, 3)
+    return nodes, tris, verts
+
+
+@pytest.mark.parametrize("entities", [[0], [1, 0, 1]], ids=["one", "several"])
+def test_iteration_cap_in_full_waves(crt, entities):
+    """Rays below and above the cap side by side, 64 to a wave: a ray that starts again to count each visit in its turn
+    leaves its neighbours' records alone."""
+    r = context(crt, [patchy(crt, 2048, 1), chain(crt, 9, True)], entities)
+    rays = random_rays((6144 << 6) // 2 + 777, [-0.04, -0.2, -2], [0.04, 0.2, -1], seed=5)
+    rays["dir"] = (0, 0, 1)
+    rays["dir"][::2, :2] = np.random.default_rng(6).uniform(-1e-3, 1e-3, (len(rays[::2]), 2))
+    hits = same_as_array_walk(crt, r, rays)
+    assert ((hits["status"] & 0xFFFFFF) > 0).all()
+    closest = crt.DeviceArray(crt.HIT_DTYPE, rays.size)
+    r.intersect(crt.QUERY_CLOSEST, crt.DeviceArray.from_host(rays), closest)
+    crt.lib().crt_device_sync()
+    capped = (closest.download()["status"] & crt.STATUS_ITER_CAP) != 0
+    assert 0.2 < capped.mean() < 0.8
+
+
+@pytest.mark.parametrize("log2", range(7))
+def test_rays_per_wave(crt, log2):
+    """Batches on both sides of each change of the rays that a wave takes."""
+    from candela_amd import scenes
+    r = crt.RayIntersector(crt.FORMAT_STACKLESS)
+    r.add_object(0, scenes.icosphere_cloud(count=30, subdivisions=2, seed=log2, box=20.0))
+    r.push_entity(0)
+    r.buffer_entities()
+    r.buffer_data()
+    for n in ((6144 << log2) - 1, 6144 << log2, (6144 << log2) + 1):
+        assert (same_as_array_walk(crt, r, random_rays(n, [-2, -2, -2], [22, 22, 22], seed=n))["t"] > 0).any()
+
+
 def test_one_leaf_object_and_empty_scene(crt):
     nodes, tris, verts = chain(crt, 1, True)
     nodes = nodes[1:2].copy()
