@@ -53,7 +53,8 @@ constexpr int kMaxLights = 16;
 // lane's leaf is tested as soon as it is reached; 805 us with gradients met in
 // LDS and one loop condition per node.  3 waves a tile take 6% more, 4 take 9%.
 // An image of so few tiles that all fit the device at once with kWide waves each
-// takes those: 64 x 64 pixels 204 -> 151 us, 192 x 192 224 -> 171.
+// takes those: 64 x 64 pixels 204 -> 133 us, 192 x 192 224 -> 180 (launch_backward
+// has the adjoint's).
 constexpr int kWaves = 2, kWide = 8;
 constexpr float kPi = 3.14159265359f;      // CookTorranceBRDF.glsl:7
 constexpr float kOffset = 1e-4f;           // surface offset of secondary rays
@@ -540,10 +541,7 @@ backward_kernel(SceneArgs s, const crt_shade_record* __restrict__ rec, int64_t n
             const unsigned long long m = __ballot(seen);
             if (lane == 0) (first ? T.vis_p : T.vis_q)[l] = m;
         }
-        if constexpr (GROUPS == 1)
-            __syncthreads();
-        else
-            group_barrier<WAVES>(&arrived[group], turn + 1);
+        group_barrier<WAVES>(&arrived[group], turn + 1);
         // one wave, another each time, takes the tile's gradients; the others go on
         if (wave != turn % WAVES) continue;
         if (lane == 0) T.next[0] = 0;
@@ -585,22 +583,30 @@ void launch_forward(const SceneArgs& s, const crt_ray* rays, const crt_hit* hits
                        seed, color, rec);
 }
 
+// Waves a tile, and tiles a workgroup, of the adjoint.  A workgroup holds at
+// least two tiles, so that a light's gradient takes one addition per 128 pixels
+// or fewer: with one (64 pixels an addition) the rounding of an image of 128 x
+// 128 pixels was 1.4 times as large.  The most waves with which all tiles are
+// resident at once; kMid by the registers (six waves per SIMD over the
+// stackless layout, five over the stack layout).  64 x 64 pixels take 50 us with
+// 8 waves a tile, 54 with 6, 63 with 4; 192 x 192 pixels 57 with 6, 65 with 4, 100
+// with 2, where 8 no longer fit; over the stack layout 103 with 4, 175 with 2.
 template <int FORMAT>
 void launch_backward(const SceneArgs& s, const crt_shade_record* rec, int64_t npix, const Params& P,
                      const float* color, const float* target, float* g_albedo, float* g_rough, float* g_inten,
                      hipStream_t st) {
-    constexpr int kGroups = kWide / kWaves;
+    constexpr int kMid = FORMAT == CRT_FORMAT_STACKLESS ? 6 : 4, kGroups = 4;
     const int64_t tiles = (npix + 63) / 64;
-    const auto wide = backward_kernel<FORMAT, kWide, 1>;
-    const auto fn = backward_kernel<FORMAT, kWaves, kGroups>;
-    if (tiles <= resident(wide, 64 * kWide)) {
-        hipLaunchKernelGGL(wide, dim3(unsigned(tiles)), dim3(64 * kWide), 0, st, s, rec, npix, P, color, target,
-                           g_albedo, g_rough, g_inten);
-        return;
-    }
-    const int64_t grid = resident(fn, 64 * kWide), need = (tiles + kGroups - 1) / kGroups;
-    hipLaunchKernelGGL(fn, dim3(unsigned(need < grid ? need : grid)), dim3(64 * kWide), 0, st, s, rec, npix, P, color,
-                       target, g_albedo, g_rough, g_inten);
+    const auto launch = [&](auto fn, int waves, int groups, bool all) {
+        const int64_t need = (tiles + groups - 1) / groups, grid = resident(fn, 64 * waves * groups);
+        if (all && need > grid) return false;
+        hipLaunchKernelGGL(fn, dim3(unsigned(need < grid ? need : grid)), dim3(unsigned(64 * waves * groups)), 0, st, s,
+                           rec, npix, P, color, target, g_albedo, g_rough, g_inten);
+        return true;
+    };
+    if (launch(backward_kernel<FORMAT, kWide, 2>, kWide, 2, true)) return;
+    if (launch(backward_kernel<FORMAT, kMid, 2>, kMid, 2, true)) return;
+    launch(backward_kernel<FORMAT, kWaves, kGroups>, kWaves, kGroups, false);
 }
 
 }  // namespace shade

@@ -66,7 +66,7 @@ def test_visibility_equals_traced_shadow_rays(crt, fmt, pixels, lights, entities
 
 
 @pytest.mark.parametrize("fmt", [0, 1], ids=["stackless", "stack"])
-@pytest.mark.parametrize("pixels", [640, 300000])
+@pytest.mark.parametrize("pixels", [640, 40000, 300000])
 def test_gradients_are_the_sum_over_tiles(crt, fmt, pixels):
     """One launch against the sum of launches over parts: several tiles per workgroup at the larger size, triangles
     that share an LDS entry at both."""
