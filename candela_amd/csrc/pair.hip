@@ -39,27 +39,7 @@ __global__ void __launch_bounds__(256) pair_primary(PairScene s, Camera cam, crt
     w.run(s, rays, hits, p.i, flags, max_iter, st);
 }
 
-__global__ void __launch_bounds__(256) gather_records(const crt_triangle* __restrict__ tris,
-                                                      const crt_vertex* __restrict__ verts, int64_t n,
-                                                      float4* __restrict__ out) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int4 t = *reinterpret_cast<const int4*>(tris[i].packed);
-    const f3 a = vertex_pos(verts, t.x), b = vertex_pos(verts, t.y), c = vertex_pos(verts, t.z);
-    out[3 * i] = make_float4(a.x, a.y, a.z, __int_as_float(int32_t(i)));
-    out[3 * i + 1] = make_float4(b.x, b.y, b.z, __int_as_float(t.w));
-    out[3 * i + 2] = make_float4(c.x, c.y, c.z, 0.0f);
-}
-
 }  // namespace pair
-
-hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* verts, int64_t n, crt_tri_record* out,
-                                 hipStream_t stream) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(pair::gather_records, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, tris, verts, n,
-                       reinterpret_cast<float4*>(out));
-    return hipGetLastError();
-}
 
 // LDS stack entries, node steps per round, parked lanes that end the node
 // phase.  10 entries (20 KB a workgroup) leave the 7 waves per SIMD that the

@@ -327,8 +327,8 @@ struct crt_context {
     // where the data allow none; those calls then walk the buffered data.
     void* d_records = nullptr;
     void* d_pairs = nullptr;
-    std::vector<std::pair<int32_t, int32_t>> appended;   // (first node, nodes) of the host copies' objects
-    std::vector<std::pair<int32_t, int32_t>> paired;     // the same of d_pairs
+    std::vector<crt::NodeRange> appended;     // the host copies' objects
+    std::vector<crt::NodeRange> paired;       // those in d_pairs
     bool pairs_fit = false;                   // every buffered entity walks an object of d_pairs
     // Wide layout derived from the buffered data and entities.
     void* d_wide_groups = nullptr;
@@ -362,7 +362,7 @@ struct crt_context {
         pairs_fit = d_pairs != nullptr;
         for (const crt_entity& e : entities)
             pairs_fit = pairs_fit && std::binary_search(paired.begin(), paired.end(),   // in order of the nodes
-                                                        std::make_pair(e.node_offset, e.node_count));
+                                                        crt::NodeRange{e.node_offset, e.node_count});
     }
     void free_wide() {
         if (d_wide_groups) (void)hipFree(d_wide_groups);
@@ -452,7 +452,6 @@ int append_object(crt_context* ctx, int32_t object_id, const void* nodes, int64_
     od.triangle_offset = int64_t(ctx->triangles.size());
     od.vertices_offset = int64_t(ctx->vertices.size());
     od.node_count = node_count;
-    ctx->appended.emplace_back(int32_t(od.node_offset), int32_t(node_count));
     if (ctx->format == CRT_FORMAT_STACKLESS) {
         const auto* n = static_cast<const crt_stackless_node*>(nodes);
         ctx->stackless.insert(ctx->stackless.end(), n, n + node_count);
@@ -470,6 +469,7 @@ int append_object(crt_context* ctx, int32_t object_id, const void* nodes, int64_
         ctx->triangles.push_back(t);
     }
     ctx->index_offset += uint32_t(vert_count);
+    ctx->appended.push_back(crt::NodeRange{int32_t(od.node_offset), int32_t(node_count)});
     ctx->objects[object_id] = od;
     ctx->data_buffered = false;
     return CRT_OK;
@@ -478,38 +478,38 @@ int append_object(crt_context* ctx, int32_t object_id, const void* nodes, int64_
 // The records and pairs of the data just buffered.  They only speed a walk up,
 // so data that allow none (or too little memory) leave them out.
 void derive_unguarded(crt_context* ctx) {
-    const int64_t ntris = int64_t(ctx->triangles.size());
-    const uint32_t nverts = uint32_t(ctx->vertices.size());
+    const int64_t ntris = int64_t(ctx->triangles.size()), nnodes = int64_t(ctx->stackless.size());
     if (ntris == 0) return;
-    for (const crt_triangle& t : ctx->triangles)
-        if (uint32_t(t.packed[0]) >= nverts || uint32_t(t.packed[1]) >= nverts || uint32_t(t.packed[2]) >= nverts)
-            return;
-    void* records = nullptr;
-    bool ok = hipMalloc(&records, size_t(ntris) * sizeof(crt_tri_record)) == hipSuccess;
-    if (ok) {
-        ctx->d_records = records;
-        ok = crt::launch_gather_records(static_cast<const crt_triangle*>(ctx->d_tris),
-                                        static_cast<const crt_vertex*>(ctx->d_verts), ntris,
-                                        static_cast<crt_tri_record*>(records), nullptr) == hipSuccess &&
-             hipStreamSynchronize(nullptr) == hipSuccess;
-    }
-    if (ok && ctx->format == CRT_FORMAT_STACKLESS) {
-        std::vector<crt_stack_node> pairs((ctx->stackless.size() + 1) / 2 + 1);
-        for (const auto& o : ctx->appended)
-            if (crt::build_pairs(ctx->stackless.data(), o.first, o.second, ntris, pairs.data()))
-                ctx->paired.push_back(o);
-        void* d = nullptr;
-        const size_t bytes = pairs.size() * sizeof(crt_stack_node);
-        ok = hipMalloc(&d, bytes) == hipSuccess;
-        if (ok) {
-            ctx->d_pairs = d;
-            ok = hipMemcpy(d, pairs.data(), bytes, hipMemcpyHostToDevice) == hipSuccess;
-        }
-    }
-    if (!ok) {
-        (void)hipGetLastError();
-        ctx->free_derived();
-    }
+    const bool paired = ctx->format == CRT_FORMAT_STACKLESS && nnodes <= INT32_MAX && !ctx->appended.empty();
+    const std::vector<crt::NodeRange>& objects = ctx->appended;
+    const size_t nobjects = paired ? objects.size() : 0;
+    const auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
+    // behind the arrays: a flag for the triangles and each object, the objects, scratch memory
+    std::vector<uint32_t> bad(1 + nobjects, 0u);
+    const size_t flags = align(size_t(ntris) * sizeof(crt_tri_record));
+    const size_t ranges = align(size_t(nnodes + 1) / 2 * sizeof(crt_stack_node));
+    const size_t scratch = ranges + align(nobjects * sizeof(crt::NodeRange));
+    bool ok = hipMalloc(&ctx->d_records, flags + bad.size() * 4) == hipSuccess;
+    if (ok && paired) ok = hipMalloc(&ctx->d_pairs, scratch + crt::pairs_scratch(nnodes, int64_t(nobjects))) == hipSuccess;
+    auto* d_bad = reinterpret_cast<uint32_t*>(static_cast<char*>(ctx->d_records) + flags);
+    char* d_pairs = static_cast<char*>(ctx->d_pairs);
+    ok = ok && hipMemcpy(d_bad, bad.data(), bad.size() * 4, hipMemcpyHostToDevice) == hipSuccess &&
+         crt::launch_gather_records(static_cast<const crt_triangle*>(ctx->d_tris),
+                                    static_cast<const crt_vertex*>(ctx->d_verts), int64_t(ctx->vertices.size()), ntris,
+                                    static_cast<crt_tri_record*>(ctx->d_records), d_bad, nullptr) == hipSuccess;
+    if (paired)
+        ok = ok &&
+             hipMemcpy(d_pairs + ranges, objects.data(), nobjects * sizeof(crt::NodeRange), hipMemcpyHostToDevice) ==
+                 hipSuccess &&
+             crt::launch_build_pairs(static_cast<const crt_stackless_node*>(ctx->d_nodes), nnodes,
+                                     reinterpret_cast<const crt::NodeRange*>(d_pairs + ranges), int64_t(nobjects),
+                                     ntris, reinterpret_cast<crt_stack_node*>(d_pairs), d_pairs + scratch, d_bad + 1,
+                                     nullptr) == hipSuccess;
+    ok = ok && hipMemcpy(bad.data(), d_bad, bad.size() * 4, hipMemcpyDeviceToHost) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    if (!ok || bad[0]) return ctx->free_derived();
+    for (size_t k = 0; k < nobjects; ++k)
+        if (!bad[1 + k]) ctx->paired.push_back(objects[k]);
 }
 
 void derive(crt_context* ctx) {

@@ -34,7 +34,7 @@ struct Camera {
     float tmax;
 };
 
-// A context's stackless scene with the derived arrays of pair_layout.cpp: the
+// A context's stackless scene with the derived arrays of pair_layout.hip: the
 // child pairs of every inner node (an object's first pair is that of its root,
 // at pair_base of its first node) and one record per triangle.
 struct PairScene {
@@ -48,15 +48,25 @@ struct PairScene {
 // Objects are full binary trees one behind the other, so (start + 1) / 2
 // leaves every object room for its (nodes - 1) / 2 pairs.
 __host__ __device__ constexpr int32_t pair_base(int32_t start) { return (start + 1) >> 1; }
-constexpr int32_t kPairStack = 64;   // levels below the root that a pair walk can hold
+constexpr int32_t kPairStack = 64;   // pending right children that a pair walk can hold
 
-// The child pairs of one object's nodes (pair_layout.cpp) into `pairs` from
-// pair_base(start) on; false when the nodes are no pre-order tree of at most
-// kPairStack levels below the root with leaves inside [0, ntris).
-bool build_pairs(const crt_stackless_node* nodes, int64_t start, int64_t count, int64_t ntris, crt_stack_node* pairs);
+// One object's nodes.
+struct NodeRange {
+    int32_t start, count;
+    bool operator<(const NodeRange& o) const { return start != o.start ? start < o.start : count < o.count; }
+};
 
-hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* verts, int64_t n, crt_tri_record* out,
-                                 hipStream_t stream);
+// A record per triangle; *bad = 1 when one names a vertex outside [0, nverts).
+hipError_t launch_gather_records(const crt_triangle* tris, const crt_vertex* verts, int64_t nverts, int64_t n,
+                                 crt_tri_record* out, uint32_t* bad, hipStream_t stream);
+// The child pairs of the objects (in the order of their nodes, none overlapping,
+// below 2^31 nodes) into pairs[(nnodes + 1) / 2]; bad[k] = 1 when object k's
+// nodes are no pre-order tree with leaves inside [0, ntris) whose walk holds at
+// most kPairStack pending children.  scratch: pairs_scratch bytes.
+size_t pairs_scratch(int64_t nnodes, int64_t nobjects);
+hipError_t launch_build_pairs(const crt_stackless_node* nodes, int64_t nnodes, const NodeRange* objects,
+                              int64_t nobjects, int64_t ntris, crt_stack_node* pairs, void* scratch, uint32_t* bad,
+                              hipStream_t stream);
 hipError_t launch_pair_grid(const PairScene& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                             uint32_t flags, int32_t max_iter, hipStream_t stream);
 hipError_t launch_pair_primary(const PairScene& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,

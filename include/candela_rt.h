@@ -643,9 +643,10 @@ int crt_buffer_entities(crt_context* ctx);
 /* BufferData (Intersector.h:321-351).  Also lays out what crt_intersect and
  * crt_intersect_primary walk instead of the buffers themselves, with the same
  * visits and records: one record per triangle, and the child pairs of a
- * stackless tree (half as much device memory again as the buffers, more or
- * less; left out where the nodes are no plain tree or memory is short).  The
- * memory behind the context's scene view is for reading only. */
+ * stackless tree.  They are formed on the device: for 2.56M triangles 1 of 7.5
+ * ms, and 222 MB of device memory beside the buffers' 182 (stack layout: 124
+ * beside 281).  Left out where the nodes are no plain tree or memory is short.
+ * The memory behind the context's scene view is for reading only. */
 int crt_buffer_data(crt_context* ctx, int clear_cpu_data);
 
 /* Host copies (the public m_BVHNodes / m_BVHVertices / m_BVHTriangles /

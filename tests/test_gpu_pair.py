@@ -175,6 +175,48 @@ def test_other_trees_walk_the_array(crt):
         same_as_array_walk(crt, context(crt, [(n, tris, verts), chain(crt, 3, True)], [0, 1]), along_z(crt, 100))
 
 
+def test_many_objects(crt):
+    """Trees of sizes around a workgroup's 256 nodes, one behind the other at any offset, and between them arrays that are
+    no trees (an even number of nodes, inner nodes alone, a leaf beyond the triangles), which no entity names."""
+    trees = [balanced(crt, k, 1) for k in (2, 64, 128, 256)]
+    trees += [chain(crt, d, right) for d in (1, 20, 126, 127, 128, 129, 300) for right in (False, True)]
+    nodes, tris, verts = chain(crt, 130, True)
+    only_inner, beyond = nodes[:200].copy(), nodes.copy()
+    only_inner["min"][:, 3], only_inner["max"][:, 3] = bits([-1]), bits([-1])
+    beyond["min"][-1, 3] = bits([100000 << 4 | 1])[0]
+    others = [(n, tris, verts) for n in (nodes[:-1], only_inner, beyond, nodes[:2])]
+    objects, named = [], []
+    for k, t in enumerate(trees):
+        named.append(len(objects))
+        objects += [t, others[k % len(others)]]
+    rays = along_z(crt, 130)
+    for k in named:
+        assert (same_as_array_walk(crt, context(crt, objects, [k]), rays)["t"] > 0).any()
+    same_as_array_walk(crt, context(crt, objects, named), rays)
+    named.append(1)       # an entity that names such an array: all walk the array
+    same_as_array_walk(crt, context(crt, objects, named), rays)
+
+
+def test_buffering_costs_what_it_copies(crt):
+    """A stackless context, with child pairs, against the stack layout's of the same scene, which copies more."""
+    import time
+
+    from candela_amd import scenes
+    mesh = scenes.icosphere_cloud(count=500, subdivisions=3, seed=2, box=63.0)
+    best = []
+    for fmt in (crt.FORMAT_STACK, crt.FORMAT_STACKLESS):
+        r = crt.RayIntersector(fmt)
+        r.add_object(0, mesh)
+        took = []
+        for _ in range(8):
+            crt.lib().crt_device_sync()
+            t = time.perf_counter()
+            r.buffer_data()
+            took.append(time.perf_counter() - t)
+        best.append(min(took))
+    assert best[1] < 1.6 * best[0], best
+
+
 def test_rebuffered_data_and_cleared_copies(crt):
     """An object that took another's id beside the entities of the first, then the host copies gone."""
     r = context(crt, [chain(crt, 6, True), chain(crt, 9, False)], [1, 0])
