@@ -109,5 +109,32 @@ __device__ __forceinline__ uint32_t pack_status(uint32_t visits, uint32_t flags)
 __device__ __forceinline__ void pin(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 __device__ __forceinline__ void pin(int4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
+// Reads at an address that is the same for the whole wave, of memory that no
+// launch writes while it is read so: scalar loads, into scalar registers.
+struct UniformFloat4 {
+    using Word = const __attribute__((address_space(4))) float;
+    Word* p;
+    __device__ __forceinline__ explicit UniformFloat4(const float4* at) : p((Word*)at) {}
+    __device__ __forceinline__ float4 operator[](int k) const {
+        return make_float4(p[4 * k], p[4 * k + 1], p[4 * k + 2], p[4 * k + 3]);
+    }
+};
+
+struct UniformEntity {
+    using Entity = const __attribute__((address_space(4))) crt_entity;
+    Entity* en;
+    __device__ __forceinline__ UniformEntity(const crt_entity* entities, int32_t e) : en((Entity*)(entities + e)) {}
+    __device__ __forceinline__ float alpha() const { return __int_as_float(en->data[1]); }
+    __device__ __forceinline__ int32_t start() const { return en->node_offset; }
+    __device__ __forceinline__ int32_t count() const { return en->node_count; }
+    // A point (w = 1) or direction (w = 0) in the entity's space.
+    __device__ __forceinline__ f3 to_local(f3 p, float w) const {
+        float m[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) m[k] = en->inverse[k];
+        return xform(m, p, w);
+    }
+};
+
 }  // namespace dm
 }  // namespace crt

@@ -14,7 +14,7 @@
 namespace crt {
 namespace pair {
 
-template <bool ANY, int D, int I, int LB>
+template <bool ANY, bool TOGETHER, int D, int I, int LB>
 __global__ void __launch_bounds__(256) pair_grid(PairScene s, const crt_ray* rays, crt_hit* __restrict__ hits,
                                                  int64_t n, uint32_t flags, int32_t max_iter, int32_t log2,
                                                  int32_t blocks) {
@@ -23,7 +23,10 @@ __global__ void __launch_bounds__(256) pair_grid(PairScene s, const crt_ray* ray
     typename PairStack<D>::Entry spill[spill_entries<D>()];
     PairStack<D> st{lds + threadIdx.x, 256, spill};
     PairWave<ANY, D, I, LB> w;
-    w.run(s, rays, hits, i, flags, max_iter, st);
+    if constexpr (TOGETHER)
+        w.run_together(s, rays, hits, i, flags, max_iter, st);
+    else
+        w.run(s, rays, hits, i, flags, max_iter, st);
 }
 
 template <int D, int I, int LB>
@@ -36,7 +39,7 @@ __global__ void __launch_bounds__(256) pair_primary(PairScene s, Camera cam, crt
     typename PairStack<D>::Entry spill[spill_entries<D>()];
     PairStack<D> st{lds + threadIdx.x, 256, spill};
     PairWave<false, D, I, LB> w;
-    w.run(s, rays, hits, p.i, flags, max_iter, st);
+    w.run_together(s, rays, hits, p.i, flags, max_iter, st);
 }
 
 }  // namespace pair
@@ -48,18 +51,19 @@ __global__ void __launch_bounds__(256) pair_primary(PairScene s, Camera cam, crt
 // 261 with (8, 8), 274 with (2, 8).
 #define CRT_PAIR_SHAPE 10, 4, 16
 
+// Waves of fewer than 64 rays, and images, go from entity to entity together
+// (run_together); full waves, whose rays may meet any of them, each at its own
+// pace.
 hipError_t launch_pair_grid(const PairScene& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                             uint32_t flags, int32_t max_iter, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     const int32_t log2 = rays_per_wave_log2(n);
     const int32_t blocks = int32_t((n + (4 << log2) - 1) >> (log2 + 2));
     const unsigned padded = unsigned((blocks + 7) / 8 * 8);
-    if (query == CRT_QUERY_ANY)
-        hipLaunchKernelGGL((pair::pair_grid<true, CRT_PAIR_SHAPE>), dim3(padded), dim3(256), 0, stream, s, rays, hits,
-                           n, flags, max_iter, log2, blocks);
-    else
-        hipLaunchKernelGGL((pair::pair_grid<false, CRT_PAIR_SHAPE>), dim3(padded), dim3(256), 0, stream, s, rays, hits,
-                           n, flags, max_iter, log2, blocks);
+    const bool any = query == CRT_QUERY_ANY, together = log2 < 6;
+    const auto fn = any ? (together ? pair::pair_grid<true, true, CRT_PAIR_SHAPE> : pair::pair_grid<true, false, CRT_PAIR_SHAPE>)
+                        : (together ? pair::pair_grid<false, true, CRT_PAIR_SHAPE> : pair::pair_grid<false, false, CRT_PAIR_SHAPE>);
+    hipLaunchKernelGGL(fn, dim3(padded), dim3(256), 0, stream, s, rays, hits, n, flags, max_iter, log2, blocks);
     return hipGetLastError();
 }
 

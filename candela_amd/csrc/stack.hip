@@ -86,7 +86,7 @@ stack_persistent_occ(SceneArgs s, const crt_ray* __restrict__ rays, crt_hit* __r
 
 // The walk over a context's triangle records: a ray batch, or an image's
 // primary rays.
-template <bool ANY, int D, int I, int LB, int OCC>
+template <bool ANY, bool TOGETHER, int D, int I, int LB, int OCC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
 stack_records(SceneArgs s, const crt_ray* rays, crt_hit* __restrict__ hits, int64_t n, uint32_t flags, int32_t max_iter,
               int32_t log2, int32_t blocks) {
@@ -95,10 +95,13 @@ stack_records(SceneArgs s, const crt_ray* rays, crt_hit* __restrict__ hits, int6
     int32_t spill[spill_entries<D>()];
     NodeStack<D> st{lds + threadIdx.x, 256, spill};
     StackWave<ANY, D, I, LB, true> w;
-    w.run(s, rays, hits, i, flags, max_iter, nullptr, st);
+    if constexpr (TOGETHER)
+        w.run_together(s, rays, hits, i, flags, max_iter, st);
+    else
+        w.run(s, rays, hits, i, flags, max_iter, nullptr, st);
 }
 
-template <int D, int I, int LB, int OCC>
+template <bool TOGETHER, int D, int I, int LB, int OCC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8)))
 stack_primary(SceneArgs s, Camera cam, crt_ray* rays, crt_hit* __restrict__ hits, ImageTiles image, uint32_t flags,
               int32_t max_iter) {
@@ -109,7 +112,10 @@ stack_primary(SceneArgs s, Camera cam, crt_ray* rays, crt_hit* __restrict__ hits
     int32_t spill[spill_entries<D>()];
     NodeStack<D> st{lds + threadIdx.x, 256, spill};
     StackWave<false, D, I, LB, true> w;
-    w.run(s, rays, hits, p.i, flags, max_iter, nullptr, st);
+    if constexpr (TOGETHER)
+        w.run_together(s, rays, hits, p.i, flags, max_iter, st);
+    else
+        w.run(s, rays, hits, p.i, flags, max_iter, nullptr, st);
 }
 
 template <bool ANY, int D, int I, int LB, int OCC>
@@ -236,25 +242,27 @@ hipError_t launch_stack_persistent(const SceneArgs& s, int query, const crt_ray*
 // 16) 172, 7 waves (with spills) 176, the thread-per-ray walk 240.
 #define CRT_STACK_REC 16, 4, 32, 1
 
+// Several entities are walked together (run_together): at their own pace,
+// instances that most rays pass by take up to 1.8 times the thread-per-ray walk's
+// time.
 hipError_t launch_stack_records(const SceneArgs& s, int query, const crt_ray* rays, crt_hit* hits, int64_t n,
                                 uint32_t flags, int32_t max_iter, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     const int32_t log2 = rays_per_wave_log2(n);
     const int32_t blocks = int32_t((n + (4 << log2) - 1) >> (log2 + 2));
     const unsigned padded = unsigned((blocks + 7) / 8 * 8);
-    if (query == CRT_QUERY_ANY)
-        hipLaunchKernelGGL((sdev::stack_records<true, CRT_STACK_REC>), dim3(padded), dim3(256), 0, stream, s, rays,
-                           hits, n, flags, max_iter, log2, blocks);
-    else
-        hipLaunchKernelGGL((sdev::stack_records<false, CRT_STACK_REC>), dim3(padded), dim3(256), 0, stream, s, rays,
-                           hits, n, flags, max_iter, log2, blocks);
+    const bool any = query == CRT_QUERY_ANY, together = s.entity_count > 1;
+    const auto fn = any ? (together ? sdev::stack_records<true, true, CRT_STACK_REC> : sdev::stack_records<true, false, CRT_STACK_REC>)
+                        : (together ? sdev::stack_records<false, true, CRT_STACK_REC> : sdev::stack_records<false, false, CRT_STACK_REC>);
+    hipLaunchKernelGGL(fn, dim3(padded), dim3(256), 0, stream, s, rays, hits, n, flags, max_iter, log2, blocks);
     return hipGetLastError();
 }
 
 hipError_t launch_stack_primary(const SceneArgs& s, const Camera& cam, crt_ray* rays, crt_hit* hits, int width,
                                 int height, uint32_t flags, int32_t max_iter, hipStream_t stream) {
     const dm::ImageTiles image = dm::image_tiles(width, height);
-    hipLaunchKernelGGL((sdev::stack_primary<CRT_STACK_REC>), dim3(dm::image_grid(image)), dim3(256), 0, stream, s, cam, rays, hits, image, flags, max_iter);
+    const auto fn = s.entity_count > 1 ? sdev::stack_primary<true, CRT_STACK_REC> : sdev::stack_primary<false, CRT_STACK_REC>;
+    hipLaunchKernelGGL(fn, dim3(dm::image_grid(image)), dim3(256), 0, stream, s, cam, rays, hits, image, flags, max_iter);
     return hipGetLastError();
 }
 

@@ -195,6 +195,12 @@ struct StackWave {
         pin(lmax);
         pin(rmin);
         pin(rmax);
+        return enter(lmin, lmax, rmin, rmax, st);
+    }
+
+    // The same once the entry is loaded.
+    __device__ __forceinline__ int32_t enter(float4 lmin, float4 lmax, float4 rmin, float4 rmax,
+                                             NodeStack<LDS_DEPTH>& st) {
         const int32_t lp = __float_as_int(lmin.w), rp = __float_as_int(rmin.w);
         const bool lleaf = lp != -1, rleaf = rp != -1;
         const float lb = bounds_stack(lmin, lmax, ro, inv, tmax), rb = bounds_stack(rmin, rmax, ro, inv, tmax);
@@ -282,24 +288,24 @@ struct StackWave {
         return ANY && (h0 || h1);
     }
 
-    // One round of the wave: node phase, leaf phase, walk ends.
-    __device__ __forceinline__ void round(const SceneArgs& s, const crt_ray* rays,
-                                          crt_hit* __restrict__ hits, uint32_t flags, int32_t max_iter,
-                                          uint32_t* __restrict__ tri_tests, NodeStack<LDS_DEPTH>& st) {
+    // What follows a step.
+    __device__ __forceinline__ void entered(int32_t r) {
+        if (r == kEnd) {
+            walk_done = true;
+        } else if (r == kLeaves) {
+            leafing = true;
+            const bool l0 = leaf_nonempty(leaf0);
+            leaf = l0 ? leaf0 : leaf1;
+            pi = l0 && leaf_nonempty(leaf1) ? 1 : 2;
+            off = 0;
+        }
+    }
+
+    // One round of the wave: node phase, leaf phase.
+    __device__ __forceinline__ void round(const SceneArgs& s, int32_t max_iter, NodeStack<LDS_DEPTH>& st) {
         // --- node phase ----------------------------------------------------------
         for (int k = 0; k < INNER; ++k) {
-            if (active && !walk_done && !leafing) {
-                const int32_t r = step(s, max_iter, st);
-                if (r == kEnd) {
-                    walk_done = true;
-                } else if (r == kLeaves) {
-                    leafing = true;
-                    const bool l0 = leaf_nonempty(leaf0);
-                    leaf = l0 ? leaf0 : leaf1;
-                    pi = l0 && leaf_nonempty(leaf1) ? 1 : 2;
-                    off = 0;
-                }
-            }
+            if (active && !walk_done && !leafing) entered(step(s, max_iter, st));
             const unsigned long long stepping = __ballot(active && !walk_done && !leafing);
             if (stepping == 0 || __popcll(__ballot(leafing)) >= LEAF_BATCH) break;
         }
@@ -330,7 +336,11 @@ struct StackWave {
                 }
             }
         }
-        // --- walk ends: next entity or the ray's result --------------------------
+    }
+
+    // Walk ends: the next entity or the ray's result.
+    __device__ __forceinline__ void walk_ends(const SceneArgs& s, const crt_ray* rays, crt_hit* __restrict__ hits,
+                                              uint32_t flags, uint32_t* __restrict__ tri_tests) {
         // the ends run once kWalkEndBatch lanes wait or no lane can step
         const unsigned long long ends = __ballot(walk_done);
         if (ends && (__popcll(ends) >= kWalkEndBatch || !__ballot(active && !walk_done && !leafing))) {
@@ -355,7 +365,68 @@ struct StackWave {
         leafing = false;
         walk_done = false;
         if (i >= 0) begin_ray(s, rays, hits, i, flags, tri_tests);
-        while (__ballot(active)) round(s, rays, hits, flags, max_iter, tri_tests, st);
+        while (__ballot(active)) {
+            round(s, max_iter, st);
+            walk_ends(s, rays, hits, flags, tri_tests);
+        }
+    }
+
+    // The same, the lanes going from entity to entity together: an entity's record and root entry are read once for the
+    // wave, by scalar loads, and lanes that pass it by wait.  At its own pace every lane fetches its own entities, and
+    // neighbours that met the same nodes no longer do: 1920 x 1080 primary rays over 64 instances of 20,480 triangles take
+    // 1,343 us so, 621 together (a thread per ray 741), 400,000 occlusion rays over 300 instances of 320 triangles 945 and
+    // 597 (872).  But a wave then waits for the longest walk of each entity, not of all together: 1,500,000 rays over 8
+    // overlapping instances of 3,074 triangles take 624 us at their own pace, 922 together (939).
+    __device__ __forceinline__ void run_together(const SceneArgs& s, const crt_ray* rays, crt_hit* __restrict__ hits,
+                                                 int64_t i, uint32_t flags, int32_t max_iter,
+                                                 NodeStack<LDS_DEPTH> st) {
+        const bool valid = i >= 0;
+        active = leafing = walk_done = false;
+        slot = int32_t(i);
+        tmax = ray_tmax = valid ? reinterpret_cast<const float4*>(rays + i)[0].w : 0.0f;
+        hit_ent = tri = mesh = -1;
+        tests = status = visits = 0;
+        for (int32_t e = 0; e < s.entity_count; ++e) {
+            const UniformEntity en(s.entities, e);
+            if ((flags & CRT_FLAG_IGNORE_TRANSPARENT) && en.alpha() < 0.99f) continue;
+            active = valid && !(ANY && tri >= 0);
+            if (!__any(active)) break;
+            ent = e;
+            start = en.start();
+            count = en.count();
+            if (active) {
+                const float4* rp = reinterpret_cast<const float4*>(rays + slot);
+                const float4 a = rp[0], b = rp[1];
+                ro = en.to_local(mk(a.x, a.y, a.z), 1.0f);
+                rd = en.to_local(mk(b.x, b.y, b.z), 0.0f);
+                inv = mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z);
+                cur = start;
+                sp = 0;
+                it = 0;
+                end_bits = 0;
+                if (ANY) tmax = ray_tmax;
+            }
+            // the root entry, which every lane enters, in scalar registers
+            if (start >= 0 && count >= 0 && int64_t(start) < s.total_nodes) {
+                const UniformFloat4 n(reinterpret_cast<const float4*>(s.nodes) + 4 * int64_t(en.start()));
+                if (active) {
+                    it = 1;
+                    entered(enter(n[0], n[1], n[2], n[3], st));
+                    if (walk_done) {
+                        walk_done = active = false;
+                        visits++;
+                    }
+                }
+            }
+            while (__any(active)) {
+                round(s, max_iter, st);
+                if (walk_done) {
+                    walk_done = active = false;
+                    visits += uint32_t(it);
+                }
+            }
+        }
+        if (valid) finish(s, rays, hits, nullptr, flags);
     }
 
     // Rays [0, n) claimed from the sharded queue (queue.h): between rounds,
@@ -389,7 +460,8 @@ struct StackWave {
                 if (!q.more) break;
                 continue;
             }
-            round(s, rays, hits, flags, max_iter, tri_tests, st);
+            round(s, max_iter, st);
+            walk_ends(s, rays, hits, flags, tri_tests);
         }
     }
 };
