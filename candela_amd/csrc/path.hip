@@ -619,7 +619,7 @@ extern "C" int crt_trace_paths(const crt_scene_view* scene, const crt_path_param
     if (own_grid && variant >= 6 && npaths <= int64_t(grid) * 256) {
         // a lane for every path: nothing to refill
         fn = scene->format == CRT_FORMAT_WIDE8 ? crt::path::path_fn<8, true>(variant) : crt::path::path_fn<4, true>(variant);
-        log2 = crt::rays_per_wave_log2(npaths, crt::kSpecWaves);
+        log2 = crt::spec_rays_per_wave_log2(npaths);
         blocks = crt::wave_blocks(npaths, log2);
         grid = (blocks + 7) / 8 * 8;
     } else {

@@ -148,7 +148,7 @@ hipError_t launch_spec_grid(const SceneArgs& s, int query, const crt_ray* rays, 
     if (n <= 0) return hipSuccess;
     const void* fn = grid_pick(s.format, query, variant);
     if (!fn) return hipErrorInvalidValue;
-    int32_t log2 = rays_per_wave_log2(n, kSpecWaves);
+    int32_t log2 = spec_rays_per_wave_log2(n);
     int32_t blocks = wave_blocks(n, log2);
     const unsigned padded = unsigned((blocks + 7) / 8 * 8);
     SceneArgs sa = s;
@@ -184,7 +184,7 @@ hipError_t launch_spec_persistent(const SceneArgs& s, int query, const crt_ray* 
     if (own_grid && n <= int64_t(grid) * 256) {
         // a lane for every ray: nothing to refill
         fn = persistent_pick<true>(s.format, query, variant);
-        log2 = rays_per_wave_log2(n, kSpecWaves);
+        log2 = spec_rays_per_wave_log2(n);
         blocks = wave_blocks(n, log2);
         grid = (blocks + 7) / 8 * 8;
     } else {

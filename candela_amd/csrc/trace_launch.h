@@ -125,8 +125,8 @@ hipError_t launch_stack_persistent(const SceneArgs& s, int query, const crt_ray*
                                    uint32_t* tri_tests, int variant, int grid, hipStream_t stream);
 
 // log2 of the rays a wave takes.  A wave costs what its rays cost together, so
-// a launch of few rays spreads them over all the waves that the device holds at
-// once (6 on each of 1,024 SIMDs): 300 rays over 3,074 triangles take 28 us with
+// a launch of few rays spreads them over about all the waves that the device holds
+// at once (6 or 7 of these walks on each of 1,024 SIMDs): 300 rays over 3,074 triangles take 28 us with
 // one ray a wave, 31 with 4 and 40 with 64; 5,976 primary rays 102, 123 and 153;
 // 41,736 bounce rays, with 8, 78 against 90.  More waves than fit only add up:
 // 59,000 rays take 66 us with 16 a wave, 83 with 4 and 166 with one.
@@ -138,8 +138,19 @@ inline int32_t rays_per_wave_log2(int64_t n, int64_t waves = 6144) {
 // The speculative walks want fewer waves: they test the leaves of all their rays
 // together.  Occlusion and bounce rays of an 86 x 85 image 141 us with 64 rays a
 // wave, 122 over 1,024 waves, 114 over 2,048, 108 over 3,072; of 423 x 384
-// pixels 144, 126, 124 and 133.
+// pixels 144, 126, 124 and 133.  Half waves gain little (40,000 rays over one
+// entity of 77,000 triangles 59 us, 59 with 64 a wave) and cost up to 1.28 times as
+// much where a ray meets several entities (8 of 3,074 triangles: 117 and 92 us), so a
+// wave takes 16 rays or fewer, or 64.  What is left to lose are a few hundred
+// rays over many instances that they pass by, where more waves wait for each
+// other's instruction fetches: 500 rays over 64 of 20 triangles 131 us in one-ray
+// waves, 123 with 64 a wave, in BVH8 218 and 167; overlapping instances gain (8
+// of 3,074 triangles: 42 and 76 us, BVH8 50 and 91).
 constexpr int64_t kSpecWaves = 2048;
+inline int32_t spec_rays_per_wave_log2(int64_t n) {
+    const int32_t k = rays_per_wave_log2(n, kSpecWaves);
+    return k == 5 ? 6 : k;
+}
 // Workgroups of four waves that n rays then take.
 inline int32_t wave_blocks(int64_t n, int32_t log2) { return int32_t((n + (4 << log2) - 1) >> (log2 + 2)); }
 
