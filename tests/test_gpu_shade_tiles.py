@@ -2,6 +2,8 @@
 import numpy as np
 import pytest
 
+from shade_terms import order_bounds
+
 pytestmark = pytest.mark.gpu
 
 
@@ -65,32 +67,60 @@ def test_visibility_equals_traced_shadow_rays(crt, fmt, pixels, lights, entities
                 assert np.array_equal(bit[live].astype(bool), want)
 
 
+def gradients(crt, r, model, rec, color, target, lo, n):
+    from candela_amd import workloads
+    g = [crt.DeviceArray(np.float32, k) for k in (3 * model.ntri, model.ntri, model.nl)]
+    for d in g:
+        d.fill_bytes(0)
+    model.backward(r.scene(), workloads.DeviceSpan(rec, lo, n), workloads.DeviceSpan(color, 3 * lo, 3 * n),
+                   workloads.DeviceSpan(target, 3 * lo, 3 * n), *g)
+    crt.lib().crt_device_sync()
+    return [d.download().astype(np.float64) for d in g]
+
+
 @pytest.mark.parametrize("fmt", [0, 1], ids=["stackless", "stack"])
 @pytest.mark.parametrize("pixels", [640, 40000, 300000])
 def test_gradients_are_the_sum_over_tiles(crt, fmt, pixels):
-    """One launch against the sum of launches over parts: several tiles per workgroup at the larger size, triangles
-    that share an LDS entry at both."""
-    from candela_amd import workloads
+    """One launch against the sum of launches over parts: several tiles per workgroup at the larger sizes, triangles
+    that share an LDS entry at all."""
     r, model, _, _, color, rec = problem(crt, fmt, pixels, 8, 1)
     target = crt.DeviceArray(np.float32, 3 * pixels)
     target.fill_bytes(0)
-
-    def gradients(lo, n):
-        g = [crt.DeviceArray(np.float32, k) for k in (3 * model.ntri, model.ntri, model.nl)]
-        for d in g:
-            d.fill_bytes(0)
-        model.backward(r.scene(), workloads.DeviceSpan(rec, lo, n), workloads.DeviceSpan(color, 3 * lo, 3 * n),
-                       workloads.DeviceSpan(target, 3 * lo, 3 * n), *g)
-        crt.lib().crt_device_sync()
-        return [d.download().astype(np.float64) for d in g]
-
-    whole = gradients(0, pixels)
+    whole = gradients(crt, r, model, rec, color, target, 0, pixels)
     part = max(64, pixels // 30 // 64 * 64)
-    parts = [gradients(lo, min(part, pixels - lo)) for lo in range(0, pixels, part)]
+    parts = [gradients(crt, r, model, rec, color, target, lo, min(part, pixels - lo)) for lo in range(0, pixels, part)]
     assert np.count_nonzero(whole[1]) > 50
+    bounds = order_bounds(model, rec.download(), color.download(), target.download())
     for k, got in enumerate(whole):
         want = sum(p[k] for p in parts)
-        # n terms of one sum in another order: n * 2^-24 of the sum of magnitudes (the color is at least the target
-        # everywhere, so a triangle's terms have one sign but for roughness, whose sum the parts' magnitudes bound)
-        scale = np.maximum(sum(np.abs(p[k]) for p in parts), np.abs(want).max())
-        assert (np.abs(got - want) <= 16 * np.sqrt(pixels) * 2.0 ** -24 * scale).all()
+        assert (np.abs(got - want) <= bounds[k]).all(), (k, np.flatnonzero(np.abs(got - want) > bounds[k]))
+
+
+@pytest.mark.parametrize("fmt", [0, 1], ids=["stackless", "stack"])
+@pytest.mark.parametrize("pixels", [192, 40000, 120000])
+def test_triangles_of_one_lds_entry(crt, fmt, pixels):
+    """Triangles 128 apart, several pixels of each in every wave, so that they keep pushing each other out of the entry
+    they share, against launches over one triangle's pixels at a time."""
+    r, model, _, _, color, rec = problem(crt, fmt, pixels, 4, 1)
+    target = crt.DeviceArray(np.float32, 3 * pixels)
+    target.fill_bytes(0)
+    host = rec.download()
+    rng = np.random.default_rng(pixels)
+    tris = 5 + 128 * np.arange(6)
+    live = host["tri0"] >= 0
+    pick = rng.choice(tris, pixels).astype(np.int32)
+    host["tri0"] = np.where(live, pick, -1)
+    host["tri1"] = np.where(live & (host["tri1"] >= 0), rng.choice(tris + 1, pixels), -1)
+    rec.upload(host)
+    whole = gradients(crt, r, model, rec, color, target, 0, pixels)
+    bounds = order_bounds(model, host, color.download(), target.download())
+    want = [np.zeros_like(w) for w in whole]
+    for t in tris:
+        one = host.copy()
+        one["tri0"] = np.where(live & (pick == t), t, -1)
+        rec.upload(one)
+        for w, g in zip(want, gradients(crt, r, model, rec, color, target, 0, pixels)):
+            w += g
+    assert (whole[1][tris] != 0).all()
+    for k, got in enumerate(whole):
+        assert (np.abs(got - want[k]) <= bounds[k]).all(), (k, np.flatnonzero(np.abs(got - want[k]) > bounds[k]))
