@@ -1,7 +1,7 @@
 // One ray per lane: the reference's walks and scene loop as plain device
-// functions (used by the one-ray-per-lane kernels of trace.hip and inline by
-// the shading kernels of shade.hip).  Each function restates one GLSL
-// function of Source/Core/Shaders/Intersectors/Include/:
+// functions, used by the one-ray-per-lane kernels of trace.hip and the stack
+// layout's tiles of batched.hip.  Each function restates one GLSL function of
+// Source/Core/Shaders/Intersectors/Include/:
 //   walk_stackless<ANY>  TraverseBVHStackless.glsl:175-278 / :463-556
 //   walk_stack<ANY>      TraverseBVHStack.glsl:168-324 / :509-657
 //   wide::walk_wide_thread  the same closest / any-hit contract over the wide

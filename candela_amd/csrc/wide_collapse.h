@@ -1,10 +1,11 @@
 // Per-node logic of the device BVH4 / BVH8 collapse (wide_gpu.hip): one
-// wide node's slots from its BVH2 stack entry, and its children's numbers.
+// wide node's slots from its BVH2 stack entry, its children's numbers, and where
+// the level passes keep them.
 // Kept free of HIP headers so the same functions also build on the host
 // (the collapse tests compile them with clang++ under the undefined-behaviour
 // sanitizer, with every local initialized to a pattern, and compare the
 // layout with crt_wide_build's); the including file provides __device__,
-// __forceinline__, atomicOr, __float_as_int, min, max, fminf and fmaxf.
+// __host__, __forceinline__, atomicOr, __float_as_int, min, max, fminf and fmaxf.
 #pragma once
 
 #include <cstdint>
@@ -174,31 +175,32 @@ __device__ __forceinline__ void assign_slot(int64_t w, int s, int64_t idx, crt_w
     groups[w * (W / 4) + s / 4].child[s % 4] = int32_t(idx);
 }
 
-// Child indices of wide node w, one node at a time (the level passes of
-// wide_gpu.hip number a workgroup's slots at once): its inner children are
-// next_base + off + 0, 1, ... in slot order, and entries off, off + 1, ... of
-// the next level's list.  False when an index reaches cap (the links do not
-// form a tree).
+// Where the level passes of wide_gpu.hip keep a level's children and sums.  A
+// pass takes kParents nodes of a level per workgroup, whose children are at most
+// kBlock.
+constexpr int kBlock = 256;
 template <int W>
-__device__ __forceinline__ bool assign_one(int64_t w, const int32_t* __restrict__ kids, int64_t off,
-                                           int64_t next_base, int64_t cap, crt_wide_group* __restrict__ groups,
-                                           int32_t* __restrict__ next_entries, int32_t* __restrict__ next_wides,
-                                           unsigned* __restrict__ err) {
-    int64_t r = 0;
-    for (int s = 0; s < W; ++s) {
-        const int32_t e = kids[s];
-        if (e < 0) continue;
-        const int64_t idx = next_base + off + r;
-        if (idx >= cap) {   // nothing past the outputs is written
-            atomicOr(err, kErrCap);
-            return false;
-        }
-        assign_slot<W>(w, s, idx, groups);
-        next_entries[off + r] = e;
-        next_wides[off + r] = int32_t(idx);
-        ++r;
-    }
-    return true;
+constexpr int kParents = kBlock / W;
+
+// Item of a level in the array of child slots, which holds `cap` items: even
+// levels from its front, odd ones from its back (two levels in a row hold at
+// most cap nodes together).
+__device__ __forceinline__ int64_t kids_item(int32_t level, int64_t item, int64_t cap) {
+    return level & 1 ? cap - 1 - item : item;
+}
+
+// The one of three arrays of sums that a level's nodes add their children to:
+// a pass reads its level's, adds to the next one's and clears the third.
+__device__ __forceinline__ int32_t sums_array(int32_t level) { return level % 3; }
+
+// The sum of an item's workgroup, and the sums (or workgroups) of `items`.
+template <int W>
+__host__ __device__ constexpr int64_t sum_of(int64_t item) {
+    return item / kParents<W>;
+}
+template <int W>
+__host__ __device__ constexpr int64_t sums_for(int64_t items) {
+    return (items + kParents<W> - 1) / kParents<W>;
 }
 
 // A root entry whose two children are leaves with two adjacent triangles in

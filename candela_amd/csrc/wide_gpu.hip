@@ -34,8 +34,6 @@
 namespace crt {
 namespace wg {
 
-constexpr int kBlock = 256;
-
 // ---- level passes --------------------------------------------------------
 //
 // The host launches a fixed number of passes and reads nothing back, so the
@@ -72,13 +70,7 @@ static_assert(kErrLink == CRT_WIDE_GPU_BAD_LINK && kErrCap == CRT_WIDE_GPU_NOT_T
 // 2 us with these, 4.6 us with 4,096.
 constexpr int kGridMax = 1024;
 
-template <int W>
-constexpr int kParents = kBlock / W;
-
-// Level state and lists in the workspace.  The kids of even levels fill their
-// array from the front and those of odd levels from the back: two levels in a
-// row hold at most `cap` nodes together.  sums rotates over three arrays: the
-// one a pass reads, the one it adds to and the one it clears for the next.
+// Level state and lists in the workspace (kids and sums: wide_collapse.h).
 struct Lists {
     int64_t* lvl;
     int32_t* first;
@@ -90,9 +82,9 @@ struct Lists {
 
     template <int W>
     __device__ __forceinline__ int32_t* kids_of(int32_t level, int64_t item) const {
-        return kids + (level & 1 ? cap - 1 - item : item) * W;
+        return kids + kids_item(level, item, cap) * W;
     }
-    __device__ __forceinline__ uint32_t* sums_of(int32_t level) const { return sums + (level % 3) * sum_stride; }
+    __device__ __forceinline__ uint32_t* sums_of(int32_t level) const { return sums + sums_array(level) * sum_stride; }
 };
 
 // Sums of a and b over the workgroup (kBlock threads); every thread gets them.
@@ -151,15 +143,15 @@ __device__ __forceinline__ void expand_chunk(const crt_stack_node* __restrict__ 
         lds.list[rank] = entry;
     }
     __syncthreads();
-    const int64_t seg0 = before / kParents<W>;
+    const int64_t seg0 = sum_of<W>(before);
     if (tid < int(count)) {
         const int64_t item = before + tid;
         const uint32_t m = expand_one<W>(nodes, node_count, ntris, lds.list[tid], next_base + item, groups,
                                          L.kids_of<W>(p + 1, item), L.err);
-        if (m) atomicAdd(&lds.children[item / kParents<W> - seg0], m);
+        if (m) atomicAdd(&lds.children[sum_of<W>(item) - seg0], m);
     }
     __syncthreads();
-    if (tid <= W && count > 0u && seg0 + tid <= (before + count - 1) / kParents<W>) {
+    if (tid <= W && count > 0u && seg0 + tid <= sum_of<W>(before + count - 1)) {
         uint32_t* out = L.sums_of(p + 1) + seg0 + tid;
         if (alone)
             *out = lds.children[tid];
@@ -171,7 +163,7 @@ __device__ __forceinline__ void expand_chunk(const crt_stack_node* __restrict__ 
 // Clears the sums that level p + 2 will need, when level p + 1 has `count` nodes.
 template <int W>
 __device__ __forceinline__ void clear_sums(const Lists& L, int32_t p, int64_t count, int64_t first, int64_t stride) {
-    const int64_t need = (count * W + kParents<W> - 1) / kParents<W>;
+    const int64_t need = sums_for<W>(count * W);
     uint32_t* out = L.sums_of(p + 2);
     for (int64_t k = first; k < need && k < L.sum_stride; k += stride) out[k] = 0u;
 }
@@ -235,7 +227,7 @@ __global__ void __launch_bounds__(kBlock) level_async(const crt_stack_node* __re
         if (threadIdx.x == 0) L.first[k + 1] = p;
         return;
     }
-    const int64_t chunks = (np + kParents<W> - 1) / kParents<W>;
+    const int64_t chunks = sums_for<W>(np);
     const uint32_t* sums = L.sums_of(p);
     if (blockIdx.x >= chunks) return;
     uint64_t before = 0, all = 0;
@@ -283,7 +275,7 @@ __global__ void __launch_bounds__(kBlock) finish_async(Lists L, int32_t levels, 
     const int32_t p = L.first[levels - 1];   // the first empty level, or the last one expanded
     const int64_t np = L.lvl[2 * p + 1];
     uint64_t all = 0, unused = 0;            // children of the last level, which nothing numbered
-    for (int64_t j = threadIdx.x; j < (np + kParents<W> - 1) / kParents<W>; j += kBlock) all += L.sums_of(p)[j];
+    for (int64_t j = threadIdx.x; j < sums_for<W>(np); j += kBlock) all += L.sums_of(p)[j];
     block_sum2(all, unused, sh);
     const int64_t count = L.lvl[2 * p];
     const bool over = count + int64_t(all) > L.cap;
@@ -342,8 +334,7 @@ inline Layout layout(int64_t cap, int32_t width, int32_t levels) {
         off = align256(off + bytes);
         return at;
     };
-    const int64_t parents = kBlock / width;
-    L.sum_stride = (cap + parents - 1) / parents + 1;
+    L.sum_stride = (width == 8 ? sums_for<8>(cap) : sums_for<4>(cap)) + 1;
     L.kids = take(n * size_t(width) * 4);
     L.sums = take(size_t(L.sum_stride) * 3 * 4);
     L.err = take(4);
@@ -366,7 +357,7 @@ void collapse_async(const crt_stack_node* nodes, int64_t node_count, const crt_t
                       reinterpret_cast<int32_t*>(ws + L.kids),  reinterpret_cast<uint32_t*>(ws + L.sums),
                       L.sum_stride,                              cap,
                       reinterpret_cast<unsigned*>(ws + L.err)};
-    const int32_t grid = int32_t(std::min<int64_t>(kGridMax, (cap + kParents<W> - 1) / kParents<W>));
+    const int32_t grid = int32_t(std::min<int64_t>(kGridMax, sums_for<W>(cap)));
     hipLaunchKernelGGL(root_async<W>, dim3(1), dim3(64), 0, st, nodes, node_count, cap, lists, groups);
     hipLaunchKernelGGL(records, dim3(unsigned((cap + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, tris, verts, nverts,
                        cap, recs, lists.err);

@@ -1,9 +1,9 @@
 // Host build of the device BVH4 / BVH8 collapse (candela_amd/csrc/wide_gpu.hip).
 //
-// Runs the per-node functions of wide_collapse.h -- the ones the expand,
-// assign and root kernels call -- level by level on one thread, in the order
-// the device numbers nodes (breadth-first, items of a level in order), so the
-// layout equals the device's.  tests/test_wide_collapse_host.py builds it with
+// Runs the per-node functions of wide_collapse.h level by level on one thread,
+// with the numbering, the two-ended child lists and the rotating sums of the
+// device's level passes (the same index functions; every index checked against
+// its array), so the layout equals the device's.  tests/test_wide_collapse_host.py builds it with
 // clang++ three ways -- under -fsanitize=undefined with every local set to a
 // pattern (-ftrivial-auto-var-init=pattern), with every local zeroed, and
 // plainly optimized -- and compares the layouts with crt_wide_build's: a value
@@ -17,11 +17,13 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <vector>
 
 // What the HIP headers provide to the device build, for one host thread.
 #define __device__
+#define __host__
 #define __forceinline__ inline
 static inline unsigned atomicOr(unsigned* p, unsigned v) {
     const unsigned old = *p;
@@ -40,11 +42,24 @@ using std::min;
 
 using namespace crt::wg;
 
+// Exits when an index leaves its array.
+template <typename T>
+struct Checked : std::vector<T> {
+    using std::vector<T>::vector;
+    T& operator[](int64_t i) {
+        if (i < 0 || i >= int64_t(this->size())) {
+            std::fprintf(stderr, "index %lld of %zu\n", static_cast<long long>(i), this->size());
+            std::exit(3);
+        }
+        return std::vector<T>::operator[](size_t(i));
+    }
+};
+
 template <int W>
 static int run(const std::vector<crt_stack_node>& nodes, int64_t ntris) {
     const int64_t node_count = int64_t(nodes.size());
     const int64_t cap = ntris;   // the device's output capacity: one wide node per triangle
-    std::vector<crt_wide_group> groups(size_t(cap) * (W / 4));
+    Checked<crt_wide_group> groups(size_t(cap) * (W / 4));
     unsigned err = 0;
     int64_t total = 1;
     Kid k;
@@ -53,30 +68,60 @@ static int run(const std::vector<crt_stack_node>& nodes, int64_t ntris) {
         if (!ok) err = kErrLeaf;
         write_one_slot_root<W>(groups.data(), k, ok);
     } else {
-        std::vector<int32_t> entries{0}, wides{0};
-        while (!entries.empty()) {
-            const size_t nf = entries.size();
-            std::vector<int32_t> kids(nf * W);
-            std::vector<uint32_t> counts(nf);
-            for (size_t i = 0; i < nf; ++i)
-                counts[i] = expand_one<W>(nodes.data(), node_count, ntris, entries[i], wides[i], groups.data(),
-                                          kids.data() + i * W, &err);
-            uint64_t all = 0;
-            for (uint32_t c : counts) all += c;
-            if (int64_t(total + int64_t(all)) > cap) {   // assign_async's cap check
+        // the workspace holds anything
+        const int64_t stride = sums_for<W>(cap) + 1;
+        Checked<int32_t> kids(size_t(cap) * W, 0x5A5A5A5A);
+        Checked<uint32_t> sums(size_t(stride) * 3, 0xEEEEEEEEu);
+        const auto kid = [&](int32_t level, int64_t item) { return &kids[kids_item(level, item, cap) * W]; };
+        const auto sum = [&](int32_t level, int64_t at) -> uint32_t& {
+            if (at >= stride) std::exit(4);
+            return sums[sums_array(level) * stride + at];
+        };
+        sum(0, 0) = expand_one<W>(nodes.data(), node_count, ntris, 0, 0, groups.data(), kid(0, 0), &err);
+        sum(1, 0) = 0u;
+        int64_t np = 1;   // nodes of level p, the last numbered total - 1
+        for (int32_t p = 0; np > 0; ++p) {
+            const bool alone = np <= kParents<W>;
+            int64_t all = 0;
+            for (int64_t c = 0; c < sums_for<W>(np); ++c) all += sum(p, c);
+            if (total + all > cap) {   // the pass's cap check
                 err |= kErrCap;
                 break;
             }
-            std::vector<int32_t> next_entries(all), next_wides(all);
-            int64_t off = 0;
-            for (size_t i = 0; i < nf; ++i) {
-                (void)assign_one<W>(wides[i], kids.data() + i * W, off, total, cap, groups.data(),
-                                    next_entries.data(), next_wides.data(), &err);
-                off += counts[i];
+            for (int64_t at = 0; at < sums_for<W>(all * W) && at < stride; ++at) sum(p + 2, at) = 0u;
+            int64_t before = 0;
+            for (int64_t chunk = 0; chunk < sums_for<W>(np) && all > 0; ++chunk) {   // expand_chunk
+                int32_t list[kBlock];
+                uint32_t children[W + 1] = {};
+                int64_t count = 0;
+                for (int tid = 0; tid < kBlock; ++tid) {
+                    const int64_t parent = chunk * kParents<W> + tid / W;
+                    const int32_t entry = parent < np ? kid(p, parent)[tid % W] : -1;
+                    if (entry < 0) continue;
+                    (void)groups[(total - np + parent) * (W / 4)];
+                    assign_slot<W>(total - np + parent, tid % W, total + before + count, groups.data());
+                    list[count++] = entry;
+                }
+                const int64_t first = sum_of<W>(before);
+                for (int64_t i = 0; i < count; ++i) {
+                    const int64_t item = before + i;
+                    (void)groups[(total + item + 1) * (W / 4) - 1];
+                    const uint32_t m = expand_one<W>(nodes.data(), node_count, ntris, list[i], total + item,
+                                                     groups.data(), kid(p + 1, item), &err);
+                    if (sum_of<W>(item) - first > W) std::exit(5);
+                    children[sum_of<W>(item) - first] += m;
+                }
+                for (int64_t at = 0; at <= W && count > 0 && first + at <= sum_of<W>(before + count - 1); ++at) {
+                    if (alone)
+                        sum(p + 1, first + at) = children[at];
+                    else
+                        sum(p + 1, first + at) += children[at];
+                }
+                before += count;
             }
-            total += int64_t(all);
-            entries.swap(next_entries);
-            wides.swap(next_wides);
+            if (before != all) std::exit(6);   // the sums count the children
+            total += all;
+            np = all;
         }
     }
     if (err) {   // finish_async: any status bit leaves the root empty

@@ -1,4 +1,4 @@
-"""The device builder at the edges of its tiles: sort tiles of 2,048 codes and their super-tiles, chunks of 256
+"""The device builder at the edges of its tiles: sort tiles of 2,048 codes and their super-tiles, chunks of 512
 leaves, groups of 64 and super-groups of 4,096, all against the host twin byte for byte."""
 import numpy as np
 import pytest
@@ -17,7 +17,8 @@ def _soup(n, seed, cells):
 
 
 @pytest.mark.parametrize("cells", [2, 40, 100000])
-@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 66, 255, 256, 257, 258, 511, 513, 2047, 2048, 2049, 4095, 4096, 4097,
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 66, 255, 256, 257, 258, 511, 512, 513, 514, 1023, 1024, 1025,
+                               2047, 2048, 2049, 4095, 4096, 4097,
                                4352, 8191, 32767, 32769, 65537, 262145, 1100001])
 def test_build_edges(n, cells):
     import candela_amd as crt

@@ -2,7 +2,8 @@
 
 tests/cpp/wide_collapse_host.cpp runs the per-node functions the collapse
 kernels call (candela_amd/csrc/wide_collapse.h: root_one_slot, make_kid,
-expand_one, assign_one) level by level in the device's order.  It is built
+expand_one, assign_slot) level by level in the device's order, with the device's
+index functions for child lists and sums and a check on every index.  It is built
 three ways -- under the undefined-behaviour sanitizer with every local set to
 a pattern, with every local zeroed, and plainly optimized -- and each build's
 layout must equal crt_wide_build's, renumbered breadth-first, on SAH trees
