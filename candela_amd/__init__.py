@@ -652,6 +652,8 @@ class RayIntersector:
         return out
 
     def scene(self) -> SceneView:
+        """crt_context_scene: the device buffers, for reading only (intersect walks arrays that buffer_data derived
+        from them)."""
         s = SceneView()
         check(lib().crt_context_scene(self.handle, C.byref(s)))
         return s

@@ -30,8 +30,8 @@
 //   Entry i holds internal node i's two children; a child covering two
 //   triangles is written as a 2-triangle leaf.
 //
-// Measured on 2.56M triangles (2,000 spheres): 308 us, of them bounds and codes
-// 40, sort 110, tree with boxes and entries 104 + 5 + 45; with 4-bit digits,
+// Measured on 2.56M triangles (2,000 spheres): 301 us, of them bounds and codes
+// 38, sort 109, tree with boxes and entries 104 + 5 + 45; with 4-bit digits,
 // three launches a pass and separate tree, box and entry passes it was 743 us.
 // 11,520 triangles: 82 us instead of 145, nearly all launches and latency.
 #include <hip/hip_runtime.h>
@@ -430,7 +430,8 @@ __device__ __forceinline__ void put_entry(crt_stack_node* __restrict__ out, int3
 // table of boxes over 2^k leaves, which is built level by level in two LDS
 // buffers, a level's queries answered while it is there: 24 KB in all, so the
 // CU keeps its 32 waves.  Nodes whose range leaves the chunk are marked in a
-// bit mask for span_nodes (no list: its one counter took 300 us), which also reads the leaf boxes and 64-leaf boxes written here.
+// bit mask for span_nodes (no list: its one counter took 300 us), which also
+// reads the leaf boxes and 64-leaf boxes written here.
 //
 // Bound: the gathers of the sorted triangles' indices and vertices and the
 // 64-byte entries (about 190 bytes a triangle).  2.56M triangles: 104 us, 4.7

@@ -46,9 +46,9 @@ __global__ void __launch_bounds__(256) pair_primary(PairScene s, Camera cam, crt
 
 // LDS stack entries, node steps per round, parked lanes that end the node
 // phase.  10 entries (20 KB a workgroup) leave the 7 waves per SIMD that the
-// registers allow: 1920 x 1080 primary rays over 640,000 triangles take 332 us, with
-// 12 entries (6 waves) 355.  347,053 bounce rays: 256 us with (4, 16) and (4, 8),
-// 261 with (8, 8), 274 with (2, 8).
+// registers allow: with 12 (6 waves) 1920 x 1080 primary rays over 640,000 triangles
+// take 7% longer.  Bounce rays take as long with (4, 8), 2% longer with (8, 8), 7%
+// with (2, 8).
 #define CRT_PAIR_SHAPE 10, 4, 16
 
 // Waves of fewer than 64 rays, and images, go from entity to entity together

@@ -32,12 +32,12 @@
 //
 // Bound: the chain of a wave's longest ray (511 visits among the bounce rays
 // below, 0.3 us a visit when alone), then VALU issue.  Measured against the
-// walk of the stackless array: 347,053 bounce rays over 640,000 triangles 541 ->
-// 270 us, 1920 x 1080 primary rays of the same scene 676 -> 350 us (with 8 x 8
-// pixels a wave), 300 rays over 3,074 triangles 58 -> 37 us.  Both loads of a
-// pair have to be in flight at once (pin): with the right box loaded behind
-// the left one's branch, where the compiler moves it, the same walk takes 466,
-// 582 and 55 us.
+// walk of the stackless array: 347,053 bounce rays over 640,000 triangles 422 ->
+// 214 us (of another view 541 -> 265), 1920 x 1080 primary rays of the same scene
+// 671 -> 343 us (with 8 x 8 pixels a wave), 300 rays over 3,074 triangles 52 -> 25
+// us (one ray a wave).  Both loads of a pair have to be in flight at once (pin):
+// with the right box loaded behind the left one's branch, where the compiler moves
+// it, the walk takes 1.5 to 1.8 times as long.
 #pragma once
 
 #include <hip/hip_runtime.h>

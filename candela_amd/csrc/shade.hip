@@ -20,10 +20,10 @@
 //
 // Backward, loss = sum (C - T)^2: geometry (p, q, normals) comes from the
 // forward records; visibility is re-traced, not stored.  Gradients of
-// albedo[t0], roughness[t0], albedo[t1] and every intensity are accumulated
-// with wave-aggregated atomics: lanes that share a triangle add their
-// contributions in-wave first, so the two ground-plane triangles that cover
-// half the image cost one atomic per wave, not one per pixel.
+// albedo[t0], roughness[t0], albedo[t1] and every intensity are summed over the
+// lanes of a wave that share them, then in the workgroup's LDS, and reach memory
+// by atomics: the two ground-plane triangles that cover half the image cost one
+// per workgroup, not one per pixel.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

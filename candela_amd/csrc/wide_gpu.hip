@@ -54,11 +54,12 @@ namespace wg {
 // the root and at the end of the tree share a launch.
 //
 // Bound: the chain of an expansion's dependent loads (its entry, then twice
-// the opened child's and its children's), 5 to 12 us a level, and on the wide
+// the opened child's and its children's), 5 to 10 us a level, and on the wide
 // levels the gathered entries.  With two launches a level (expand, then assign
 // numbers) and the children in scratch memory, the levels of 2.56M triangles
-// took 703 us and those of 11,520 took 223; now 360 and 105 (width 4, 32
-// passes launched, of which 9 and 25 past the end at 2 us each).
+// took 703 us and those of 11,520 took 223; now 367 and 110 (width 4, 31 passes:
+// the first, with the narrow levels at the root, 30 and 22, the widest 52 and 10,
+// 4 and 25 past the end at 2 us each).
 
 // Bit of *err: the tree has more levels than were launched.
 constexpr unsigned kErrDepth = 8u;

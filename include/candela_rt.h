@@ -656,7 +656,8 @@ int crt_context_host_buffers(const crt_context* ctx, const void** nodes, int64_t
                              const crt_triangle** tris, int64_t* tri_count,
                              const crt_vertex** verts, int64_t* vert_count,
                              const crt_entity** entities, int64_t* entity_count);
-/* Device scene of the context (valid after buffer_data + buffer_entities). */
+/* Device scene of the context (valid after buffer_data + buffer_entities), for
+ * reading only: see crt_buffer_data. */
 int crt_context_scene(const crt_context* ctx, crt_scene_view* out);
 /* Builds the wide layout (crt_wide_build) from the context's host copies of
  * the buffered data and entities and uploads it (needs buffer_data without

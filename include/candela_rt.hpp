@@ -120,6 +120,8 @@ public:
     std::vector<Vertex> Vertices() const { return host<Vertex>(2); }
     std::vector<BVHEntity> Entities() const { return host<BVHEntity>(3); }
 
+    // The device buffers, for reading only: Intersect walks arrays that BufferData
+    // derived from them.
     crt_scene_view Scene() const {
         crt_scene_view s;
         check(crt_context_scene(ctx_, &s), "Scene");
